@@ -422,36 +422,6 @@ __device__ __forceinline__ void seg_write(int j, int S, const int* __restrict__ 
     }
 }
 
-// Run edges of sorted keys (the knn's cell ranges): tstart[k] / tend[k] =
-// first / one past the last position of key k.  Four keys per thread with
-// one 16-byte load (tkey is 256-byte aligned); the neighbours across a
-// thread's four come from single loads of the same or the adjacent line.
-__global__ __launch_bounds__(256) void k_run_edges(int64_t I, const uint32_t* __restrict__ tkey,
-                                                   int* __restrict__ tstart,
-                                                   int* __restrict__ tend) {
-    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t p0 = 4 * q;
-    if (p0 >= I) return;
-    uint32_t k[6];      // k[1..4]: this thread's keys, k[0] / k[5]: the neighbours
-    if (p0 + 4 <= I) {
-        const uint4 v = reinterpret_cast<const uint4*>(tkey)[q];
-        k[1] = v.x; k[2] = v.y; k[3] = v.z; k[4] = v.w;
-    } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) k[1 + j] = p0 + j < I ? tkey[p0 + j] : 0xFFFFFFFFu;
-    }
-    k[0] = p0 > 0 ? tkey[p0 - 1] : 0xFFFFFFFFu;
-    k[5] = p0 + 4 < I ? tkey[p0 + 4] : 0xFFFFFFFFu;
-#pragma unroll
-    for (int j = 1; j <= 4; ++j) {
-        const int64_t p = p0 + j - 1;
-        if (p >= I) break;
-        const uint32_t t = k[j];
-        if (p == 0 || k[j - 1] != t) tstart[t] = (int)p;
-        if (p == I - 1 || k[j + 1] != t) tend[t] = (int)(p + 1);
-    }
-}
-
 // Tile scan over TS_BLOCK tiles per workgroup: k_seg_offsets has added up
 // each block's tile count total, chunk-item total and largest count.
 // k_tile_offsets: each block adds the totals of the blocks before it, scans
@@ -644,12 +614,6 @@ __global__ __launch_bounds__(1024) void k_lists_and_items(int nsb, int S, const 
 }
 
 }  // namespace
-
-void launch_run_edges(hipStream_t s, int64_t n, const uint32_t* sorted_keys, int* start, int* end) {
-    if (n > 0)
-        hipLaunchKernelGGL(k_run_edges, dim3(blocks_for((n + 3) / 4)), dim3(256), 0, s, n,
-                           sorted_keys, start, end);
-}
 
 void launch_depth_order(hipStream_t s, int N, uint32_t* dkey, uint32_t* dval, uint32_t* dkey2,
                         uint32_t* dval2, int* radix_temp, const uint2* rect, uint2* rect_sorted,

@@ -114,9 +114,9 @@ struct Ctx {
     bool isect_dirty = false;   // counters written and not yet cleared by a tile scan
     // evaluation: per-workgroup fp64 partials and the three sums
     Buf eval_part, eval_out;
-    // nearest-neighbour scales: cell keys / point ids (ping-pong), sort
-    // scratch, cell ranges
-    Buf knn_k, knn_v, knn_k2, knn_v2, knn_tmp, knn_s, knn_e;
+    // nearest-neighbour scales: Morton keys / point ids (ping-pong), sort
+    // scratch, sorted points, boxes of the tree, frame of the keys
+    Buf knn_k, knn_v, knn_k2, knn_v2, knn_tmp, knn_pts, knn_box, knn_frame;
     Meta* meta_h = nullptr;
     float* loss_h = nullptr;
     float* loss_hd = nullptr;   // loss_h as a device pointer: the loss kernel writes loss_h[1]
@@ -200,7 +200,7 @@ void free_all(Ctx* c) {
                    &c->c_idx, &c->c_pT, &c->c_aC, &c->final_T, &c->final_idx, &c->out_img,
                    &c->v_rendered, &c->loss_part, &c->meta_d, &c->loss_d,
                    &c->count_d, &c->work_d, &c->isect_d, &c->eval_part, &c->eval_out, &c->knn_k, &c->knn_v, &c->knn_k2, &c->knn_v2,
-                   &c->knn_tmp, &c->knn_s, &c->knn_e, &c->d_split, &c->d_dup, &c->d_sp, &c->d_dp, &c->d_keep, &c->d_kp,
+                   &c->knn_tmp, &c->knn_pts, &c->knn_box, &c->knn_frame, &c->d_split, &c->d_dup, &c->d_sp, &c->d_dp, &c->d_keep, &c->d_kp,
                    &c->d_tot, &c->d_scratch, &c->d_rnd, &c->d_src};
     for (Buf* b : bufs)
         if (b->p) { (void)hipFree(b->p); b->p = nullptr; b->bytes = 0; }
@@ -353,24 +353,16 @@ CamParams cam_params(const MsplatRenderArgs* a) {
     return p;
 }
 
-// forward_pipeline (.mm:462-750): project -> depth order -> tile lists -> raster (+merge).
-// The image goes to dst_img, or to the context's own buffer when NULL.
-// Waits for the totals word of the current frame (bit 63 set) in coherent
-// host memory.  With no gaussians nothing writes it: the stream is drained
-// instead, so that the caller may rely on the earlier work having completed
-// either way.  A failed or stopped stream ends the wait with its error: the
+// Waits for a word (bit 63 set) that a queued kernel writes to coherent host
+// memory.  A failed or stopped stream ends the wait with its error: the
 // stream is queried once the wait has lasted 20 ms, then every 20 ms (a
 // stream query queues a packet that holds the GPU for about 5 us between
 // two kernels, so a frame's ordinary wait of a millisecond or two makes none).
-hipError_t wait_totals(Ctx* c, int N, uint64_t* word) {
-    if (N <= 0) {
-        *word = 0;
-        return hipStreamSynchronize(c->stream);
-    }
+hipError_t wait_word(Ctx* c, const uint64_t* host, uint64_t* word) {
     using clock = std::chrono::steady_clock;
     auto next_query = clock::now() + std::chrono::milliseconds(20);
     for (unsigned k = 1;; ++k) {
-        const uint64_t w = __atomic_load_n(&c->isect_h[0], __ATOMIC_ACQUIRE);
+        const uint64_t w = __atomic_load_n(host, __ATOMIC_ACQUIRE);
         if (w >> 63) {
             *word = w;
             return hipSuccess;
@@ -379,7 +371,7 @@ hipError_t wait_totals(Ctx* c, int N, uint64_t* word) {
             next_query = clock::now() + std::chrono::milliseconds(20);
             const hipError_t e = hipStreamQuery(c->stream);
             if (e == hipSuccess) {   // drained: the word must be there now
-                const uint64_t v = __atomic_load_n(&c->isect_h[0], __ATOMIC_ACQUIRE);
+                const uint64_t v = __atomic_load_n(host, __ATOMIC_ACQUIRE);
                 if (v >> 63) {
                     *word = v;
                     return hipSuccess;
@@ -392,6 +384,17 @@ hipError_t wait_totals(Ctx* c, int N, uint64_t* word) {
     }
 }
 
+// Waits for the totals word of the current frame.  With no gaussians nothing
+// writes it: the stream is drained instead, so that the caller may rely on
+// the earlier work having completed either way.
+hipError_t wait_totals(Ctx* c, int N, uint64_t* word) {
+    if (N > 0) return wait_word(c, &c->isect_h[0], word);
+    *word = 0;
+    return hipStreamSynchronize(c->stream);
+}
+
+// forward_pipeline (.mm:462-750): project -> depth order -> tile lists -> raster (+merge).
+// The image goes to dst_img, or to the context's own buffer when NULL.
 int forward(Ctx* c, const MsplatRenderArgs* a, bool training, float* dst_img = nullptr,
             int32_t* radii_dst = nullptr) {
     const CamParams p = cam_params(a);
@@ -947,69 +950,29 @@ int msplat_hip_knn_mean_dist(const float* xyz, int64_t n, float* mean_dist) {
     if (!xyz || !mean_dist) return fail(MSPLAT_ERR_ARG, "null knn argument");
     if (n < 4) return fail(MSPLAT_ERR_ARG, "%lld points: at least 4 are needed", (long long)n);
     if (n > 0x7FFFFFFF) return fail(MSPLAT_ERR_ARG, "too many points");
-    // bounding box on the host (an initialisation-time call)
-    std::vector<float> host((size_t)n * 3);
-    HIP_TRY(hipMemcpyAsync(host.data(), xyz, host.size() * 4, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    float lo[3], hi[3];
-    for (int k = 0; k < 3; ++k) { lo[k] = INFINITY; hi[k] = -INFINITY; }
-    for (int64_t i = 0; i < n; ++i)
-        for (int k = 0; k < 3; ++k) {
-            const float v = host[3 * i + k];
-            if (!std::isfinite(v)) return fail(MSPLAT_ERR_ARG, "point %lld is not finite", (long long)i);
-            lo[k] = std::min(lo[k], v);
-            hi[k] = std::max(hi[k], v);
-        }
-    // cell edge: about one point per cell, at most 4 n cells and 1024 per axis
-    double ext[3], emax = 0.0, amax = 0.0;
-    for (int k = 0; k < 3; ++k) {
-        ext[k] = (double)hi[k] - (double)lo[k];
-        emax = std::max(emax, ext[k]);
-        amax = std::max(amax, std::max(std::fabs((double)lo[k]), std::fabs((double)hi[k])));
-    }
-    KnnGrid g;
-    double h = emax > 0.0 ? emax / std::cbrt((double)n) : 1.0;
-    auto dims_for = [&](double hh, int* d) {
-        double cells = 1.0;
-        for (int k = 0; k < 3; ++k) {
-            d[k] = (int)std::min(1024.0, std::max(1.0, std::ceil(ext[k] / hh)));
-            cells *= d[k];
-        }
-        return cells;
-    };
-    for (int it = 0; it < 40 && dims_for(h, g.dim) < 0.5 * (double)n; ++it) {
-        if (std::max(g.dim[0], std::max(g.dim[1], g.dim[2])) >= 1024) break;
-        h *= 0.8;
-    }
-    while (dims_for(h, g.dim) > 4.0 * (double)n) h *= 1.25;
-    if (emax > 0.0) h = std::max(h, emax / 1024.0);
-    dims_for(h, g.dim);
-    for (int k = 0; k < 3; ++k) g.lo[k] = lo[k];
-    g.h = (float)h;
-    g.inv_h = (float)(1.0 / h);
-    g.margin = (float)(1e-3 * h + 1e-6 * amax);
-    const int64_t cells = (int64_t)g.dim[0] * g.dim[1] * g.dim[2];
-    int bits = 1;
-    while (((int64_t)1 << bits) < cells) ++bits;
     const size_t N = (size_t)n;
+    KnnTree tr;
+    const int64_t nodes = knn_tree_layout(n, tr);
     ENSURE(c->knn_k, N * 4);
     ENSURE(c->knn_v, N * 4);
     ENSURE(c->knn_k2, N * 4);
     ENSURE(c->knn_v2, N * 4);
     ENSURE(c->knn_tmp, (size_t)radix_temp_ints(n) * 4);
-    ENSURE(c->knn_s, (size_t)cells * 4);
-    ENSURE(c->knn_e, (size_t)cells * 4);
-    HIP_TRY(hipMemsetAsync(c->knn_s.p, 0, (size_t)cells * 4, c->stream));
-    HIP_TRY(hipMemsetAsync(c->knn_e.p, 0, (size_t)cells * 4, c->stream));
-    launch_knn_cells(c->stream, n, xyz, g, P<uint32_t>(c->knn_k), P<uint32_t>(c->knn_v));
-    const bool flip = launch_radix_sort(c->stream, P<uint32_t>(c->knn_k), P<uint32_t>(c->knn_v),
-                                        P<uint32_t>(c->knn_k2), P<uint32_t>(c->knn_v2), n, bits,
-                                        P<int>(c->knn_tmp));
-    const uint32_t* sk = flip ? P<uint32_t>(c->knn_k2) : P<uint32_t>(c->knn_k);
-    const uint32_t* order = flip ? P<uint32_t>(c->knn_v2) : P<uint32_t>(c->knn_v);
-    launch_run_edges(c->stream, n, sk, P<int>(c->knn_s), P<int>(c->knn_e));
-    launch_knn_search(c->stream, n, xyz, g, order, P<int>(c->knn_s), P<int>(c->knn_e), mean_dist);
+    ENSURE(c->knn_pts, N * sizeof(float4));
+    ENSURE(c->knn_box, (size_t)nodes * 2 * sizeof(float4));
+    ENSURE(c->knn_frame, knn_frame_bytes());
+    tr.pts = P<float4>(c->knn_pts);
+    tr.box = P<float4>(c->knn_box);
+    __atomic_store_n(&c->isect_h[1], (uint64_t)0, __ATOMIC_RELEASE);
+    launch_knn(c->stream, xyz, tr, c->knn_frame.p, P<uint32_t>(c->knn_k), P<uint32_t>(c->knn_v),
+               P<uint32_t>(c->knn_k2), P<uint32_t>(c->knn_v2), P<int>(c->knn_tmp), c->isect_hd + 1,
+               mean_dist);
     HIP_TRY(hipGetLastError());
+    // the search writes nothing when a point is not finite
+    uint64_t word = 0;
+    HIP_TRY(wait_word(c, &c->isect_h[1], &word));
+    const uint32_t bad = (uint32_t)word;
+    if (bad) return fail(MSPLAT_ERR_ARG, "point %lld is not finite", (long long)bad - 1);
     return MSPLAT_OK;
 }
 

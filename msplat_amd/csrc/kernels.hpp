@@ -333,21 +333,27 @@ void launch_to_rgba8(hipStream_t s, const float* img, int64_t n, uint32_t* rgba)
 void launch_image_metrics(hipStream_t s, const float* img, const float* gt, int H, int W,
                           const EvalWindow& win, double* part, double* out3);
 
-// Nearest-neighbour scales of a point cloud (uniform grid).
-struct KnnGrid {
-    float lo[3];
-    float h, inv_h;     // cell edge and its reciprocal
-    float margin;       // bound on the cell-assignment rounding, in distance
-    int dim[3];
+// Nearest-neighbour scales of a point cloud: the points in Morton order and
+// a tree of bounding boxes over that order, level after level (level 0: the
+// leaves; the last level has one node).
+constexpr int KNN_LEVELS = 12;
+struct KnnTree {
+    int64_t n;
+    int levels;
+    int64_t cnt[KNN_LEVELS];   // nodes of each level
+    int64_t off[KNN_LEVELS];   // first node of each level
+    float4* pts;               // n: x, y, z, index bits
+    float4* box;               // two per node: low and high corner
 };
-void launch_knn_cells(hipStream_t s, int64_t n, const float* xyz, const KnnGrid& g,
-                      uint32_t* key, uint32_t* val);
-void launch_knn_search(hipStream_t s, int64_t n, const float* xyz, const KnnGrid& g,
-                       const uint32_t* order, const int* cstart, const int* cend,
-                       float* mean_dist);
-// Run edges of sorted keys (sorted_keys 16-byte aligned): start[k] / end[k] =
-// first / one past the last position of key k; keys absent keep their value.
-void launch_run_edges(hipStream_t s, int64_t n, const uint32_t* sorted_keys, int* start, int* end);
+// Fills n, levels, cnt and off; returns the number of nodes.
+int64_t knn_tree_layout(int64_t n, KnnTree& tr);
+size_t knn_frame_bytes();
+// mean_dist[i] for every point i, unless a coordinate is not finite: word
+// (coherent host memory) gets bit 63 and, in its low 32 bits, the first such
+// point's index plus one, or 0.  key .. val2: n each.
+void launch_knn(hipStream_t s, const float* xyz, const KnnTree& tr, void* frame, uint32_t* key,
+                uint32_t* val, uint32_t* key2, uint32_t* val2, int* radix_temp,
+                unsigned long long* word, float* mean_dist);
 
 // Target images: area resize and Brown-Conrady undistortion (image.hip).
 struct UndistortParams {

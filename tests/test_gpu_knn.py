@@ -94,3 +94,31 @@ def test_dataset_initial_gaussians(mods, tmp_path):
     again = ds.init_gaussians(sh_degree=3)
     for a, b in zip(g, again):
         assert_bits_equal(a, b, "deterministic")
+
+
+def _uneven(n, seed):
+    """Dense patches, a spread volume and far outliers, with the first point repeated."""
+    rng = np.random.default_rng(seed)
+    x = rng.normal(0, 1.5, (n, 3))
+    a, b = int(0.6 * n), int(0.95 * n)
+    x[:a] = rng.uniform(-2, 2, (8, 3))[rng.integers(0, 8, a)] + rng.normal(0, 0.02, (a, 3))
+    x[b:] = rng.normal(0, 300.0, (n - b, 3))
+    x[n // 2] = x[0]
+    return x
+
+
+# around the leaves of 16, the inner nodes of 8 leaves, the 1024 points of a
+# build workgroup and the first level that the top kernel builds (8 x 1024)
+@pytest.mark.parametrize("n", [5, 15, 16, 17, 33, 127, 128, 129, 1023, 1024, 1025, 8191, 8193])
+def test_knn_tree_edges(mods, n):
+    torch, device, _abi = mods
+    for name, cloud in (("uneven", _uneven(n, n)), ("equal", np.full((n, 3), 0.25)),
+                        ("huge", 3e37 * np.random.default_rng(n).uniform(-10, 10, (n, 3)))):
+        xyz = np.ascontiguousarray(cloud, np.float32)
+        print(f"knn {name} n={n}", flush=True)
+        d_xyz = torch.from_numpy(xyz).cuda()
+        out = torch.empty(n, dtype=torch.float32, device="cuda")
+        torch.cuda.synchronize()
+        _abi.check(device.init().msplat_hip_knn_mean_dist(device.ptr(d_xyz), n, device.ptr(out)))
+        device.sync()
+        assert_bits_equal(out.cpu().numpy(), orc.knn_mean_dist(xyz), f"knn {name} {n}")
