@@ -186,7 +186,7 @@ __global__ __launch_bounds__(256) void k_seg_count(int S, const int* __restrict_
         // counters (k_tile_offsets adds, the item build reads) and chunked-tile
         // count start at zero; the previous frame read them before this launch
         for (int i = tid; i < 3 * ntb; i += 256) tot[i] = 0;
-        if (tid < 128) cls[tid] = 0;
+        if (tid < 192) cls[tid] = 0;
         if (tid == 0) meta->n_chunked_tiles = 0;
     }
     const int per = (S + 255) / 256;
@@ -453,6 +453,12 @@ __device__ __forceinline__ int size_class(int n, int K) {
     return w > 0 ? 31 - __clz(w) : 0;
 }
 
+// Size class of a backward record of a tile of n entries in K chunks, G a record.
+__device__ __forceinline__ int group_class(int n, int K, int G) {
+    const int w = K == 1 ? n : min(n, G * CHUNK);
+    return w > 0 ? 31 - __clz(w) : 0;
+}
+
 __global__ __launch_bounds__(TS_T) void k_tile_offsets(int T, int nb,
                                                        const int* __restrict__ tcount,
                                                        const int* __restrict__ tot,
@@ -461,9 +467,9 @@ __global__ __launch_bounds__(TS_T) void k_tile_offsets(int T, int nb,
                                                        TileLists tl, Meta* __restrict__ meta) {
     __shared__ int sh[TS_T / 64];
     __shared__ int s_n[TS_T], s_k[TS_T];
-    __shared__ int s_cls[64];       // this block's items / tiles per size class
-    const int b = blockIdx.x, tid = threadIdx.x;
-    if (tid < 64) s_cls[tid] = 0;
+    __shared__ int s_cls[96];       // this block's items / tiles / groups per size class
+    const int b = blockIdx.x, tid = threadIdx.x, G = bwd_group(T);
+    if (tid < 96) s_cls[tid] = 0;
     int pn = 0, pk = 0;
     for (int i = tid; i < b; i += TS_T) {
         pn += tot[3 * i];
@@ -508,12 +514,10 @@ __global__ __launch_bounds__(TS_T) void k_tile_offsets(int T, int nb,
         const int c = size_class(n[k], K[k]);
         atomicAdd(&s_cls[c], K[k]);
         atomicAdd(&s_cls[32 + c], 1);
+        atomicAdd(&s_cls[64 + group_class(n[k], K[k], G)], (K[k] + G - 1) / G);
     }
     __syncthreads();
-    if (tid < 32) {
-        if (s_cls[tid]) atomicAdd(&it.cls[tid], s_cls[tid]);
-        if (s_cls[32 + tid]) atomicAdd(&it.cls[64 + tid], s_cls[32 + tid]);
-    }
+    if (tid < 96 && s_cls[tid]) atomicAdd(&it.cls[64 * (tid >> 5) + (tid & 31)], s_cls[tid]);
     // the projection's intersection and reference counters, copied to the
     // host earlier on the stream, cleared for the next frame
     if (b == 0 && tid < 2 * ISECT_SLOTS) isect[(size_t)(tid >> 1) * ISECT_STRIDE + (tid & 1)] = 0ull;
@@ -554,41 +558,56 @@ __device__ __forceinline__ int class_slot(bool ok, int c, const int* base, int* 
 // search, and its chunk i - tile_item0[t].  Each item, and each tile (thread
 // i < T), also takes its slot in the launch orders, heaviest class first.
 // Items vb * blockDim.x .. of the workgroup's share (any block size).
-__device__ __forceinline__ void build_items(int vb, int T, const Meta* __restrict__ meta,
+__device__ __forceinline__ void build_items(int vb, int T, Meta* __restrict__ meta,
                                             const int* __restrict__ tile_bins, Items it) {
-    __shared__ int s_base[2][32];
-    const int i = vb * (int)blockDim.x + (int)threadIdx.x;
-    if (threadIdx.x < 64) {
+    __shared__ int s_base[3][32];
+    const int i = vb * (int)blockDim.x + (int)threadIdx.x, G = bwd_group(T);
+    if (threadIdx.x < 96) {
         // first slot of each class: the elements of all higher classes
         const int k = threadIdx.x >> 5, c = threadIdx.x & 31;
         int sum = 0;
         for (int d = 31; d > c; --d) sum += it.cls[64 * k + d];
         s_base[k][c] = sum;
+        if (vb == 0 && threadIdx.x == 64) meta->n_groups = sum + it.cls[128];
     }
     __syncthreads();
     const int n_items = meta->n_items;
     const bool item_ok = i < n_items;
-    int c = 0;
+    int c = 0, cg = 0;
+    bool lead = false;
+    int4 rec = make_int4(0, 0, 0, 0), grec = rec;
     if (item_ok) {
         int lo = 0, hi = T - 1;
         while (lo < hi) {
             const int mid = (lo + hi + 1) >> 1;
             if (it.tile_item0[mid] <= i) lo = mid; else hi = mid - 1;
         }
-        it.tile[i] = lo;
-        it.k[i] = i - it.tile_item0[lo];
-        c = size_class(tile_bins[2 * lo + 1] - tile_bins[2 * lo], it.tile_K[lo]);
+        const int k = i - it.tile_item0[lo], K = it.tile_K[lo];
+        const int s = tile_bins[2 * lo], e = tile_bins[2 * lo + 1];
+        const int cs = s + k * CHUNK;
+        rec = make_int4(i, lo | (K > 1 ? ITEM_MULTI : 0) | (k >= FWD_P ? ITEM_LATE : 0), cs,
+                        K > 1 ? min(cs + CHUNK, e) : e);
+        c = size_class(e - s, K);
+        lead = k % G == 0;
+        grec = make_int4(i, rec.y, cs, K > 1 ? min(cs + G * CHUNK, e) : e);
+        cg = group_class(e - s, K, G);
     }
     if (__syncthreads_or(item_ok)) {
         const int slot = class_slot(item_ok, c, s_base[0], it.cls + 32);
-        if (item_ok) it.order[slot] = i;
+        if (item_ok) it.rec[slot] = rec;
+        const int gslot = class_slot(lead, cg, s_base[2], it.cls + 160);
+        if (lead) it.bwd_rec[gslot] = grec;
     }
     const bool tile_ok = i < T;
     int ct = 0;
-    if (tile_ok) ct = size_class(tile_bins[2 * i + 1] - tile_bins[2 * i], it.tile_K[i]);
+    int4 trec = make_int4(0, 0, 0, 0);
+    if (tile_ok) {
+        trec = make_int4(i, it.tile_K[i], tile_bins[2 * i], tile_bins[2 * i + 1]);
+        ct = size_class(trec.w - trec.z, trec.y);
+    }
     if (__syncthreads_or(tile_ok)) {
         const int slot = class_slot(tile_ok, ct, s_base[1], it.cls + 96);
-        if (tile_ok) it.tile_order[slot] = i;
+        if (tile_ok) it.tile_rec[slot] = trec;
     }
 }
 
@@ -604,7 +623,7 @@ __global__ __launch_bounds__(1024) void k_lists_and_items(int nsb, int S, const 
                                                           const int* __restrict__ hist,
                                                           const int* __restrict__ tile_bins, int tbx,
                                                           int tby, int sbx, uint32_t* __restrict__ ids,
-                                                          int T, const Meta* __restrict__ meta,
+                                                          int T, Meta* __restrict__ meta,
                                                           Items it) {
     if ((int)blockIdx.x >= nsb) {
         build_items((int)blockIdx.x - nsb, T, meta, tile_bins, it);
@@ -676,7 +695,7 @@ void launch_tile_lists(hipStream_t s, const CamParams& p, int64_t I, int64_t R,
     const int nib = (int)((std::max<int64_t>(items_bound(T, I), T) + 1023) / 1024);
     hipLaunchKernelGGL(k_lists_and_items, dim3((unsigned)(nsb + nib)), dim3(1024), 0, s, nsb, S,
                        (const int*)rb.sstart, (const int4*)rb.seg, rk, rv, (const int*)rb.hist,
-                       (const int*)tile_bins, p.tbx, p.tby, sbx, ids, T, (const Meta*)meta, it);
+                       (const int*)tile_bins, p.tbx, p.tby, sbx, ids, T, meta, it);
 }
 
 }  // namespace msp

@@ -92,15 +92,15 @@ struct Ctx {
     Buf rec, radii, tiles_hit, rect, gacc;
     Buf dkey, dval, dkey2, dval2, rect_sorted, hits, dtemp, stemp;
     // per tile
-    Buf tcount, tscan, tile_bins, tile_K, tile_item0, l_chunked, tile_done;
+    Buf tcount, tscan, tile_bins, tile_K, tile_item0, l_chunked, tile_done, live_end;
     // per super-tile, per super-tile reference, per pair block
     Buf st_r0, st_r1, sstart;
     Buf rkey, rval, rkey2, rval2, rtemp;
     Buf seg, phist;
     // per intersection: the tile-sorted gaussian ids
-    Buf tval, qmask;
+    Buf tval, bmask;
     // per item
-    Buf it_tile, it_k, it_order, tile_order, it_cls, c_T, c_C, c_idx, c_pT, c_aC;
+    Buf it_rec, tile_rec, bwd_rec, it_cls, c_T, c_C, c_idx, c_pT, c_aC;
     // per pixel
     Buf final_T, final_idx, out_img, v_rendered, loss_part;
     // scalars
@@ -133,7 +133,7 @@ struct Ctx {
     float last_loss = __builtin_nanf("");
     float loss_scale = 1.f;
     bool loss_pending = false;
-    int64_t max_items = 0;
+    int64_t max_items = 0, max_groups = 0;
     int last_N = 0, last_T = 0, last_W = 0, last_H = 0;
     bool have_bwd = false;
 };
@@ -192,11 +192,11 @@ T* P(Buf& b) { return reinterpret_cast<T*>(b.p); }
 void free_all(Ctx* c) {
     Buf* bufs[] = {&c->rec, &c->radii, &c->tiles_hit, &c->rect, &c->rect_sorted,
                    &c->gacc, &c->dkey, &c->dval, &c->dkey2, &c->dval2, &c->hits,
-                   &c->dtemp, &c->stemp, &c->tcount, &c->tscan, &c->tile_done, &c->tile_bins, &c->tile_K,
+                   &c->dtemp, &c->stemp, &c->tcount, &c->tscan, &c->tile_done, &c->live_end, &c->tile_bins, &c->tile_K,
                    &c->tile_item0, &c->l_chunked, &c->st_r0, &c->st_r1, &c->sstart,
                    &c->rkey, &c->rval, &c->rkey2, &c->rval2, &c->rtemp, &c->seg, &c->phist,
-                   &c->tval, &c->qmask,
-                   &c->it_tile, &c->it_k, &c->it_order, &c->tile_order, &c->it_cls, &c->c_T, &c->c_C,
+                   &c->tval, &c->bmask,
+                   &c->it_rec, &c->tile_rec, &c->bwd_rec, &c->it_cls, &c->c_T, &c->c_C,
                    &c->c_idx, &c->c_pT, &c->c_aC, &c->final_T, &c->final_idx, &c->out_img,
                    &c->v_rendered, &c->loss_part, &c->meta_d, &c->loss_d,
                    &c->count_d, &c->work_d, &c->isect_d, &c->eval_part, &c->eval_out, &c->knn_k, &c->knn_v, &c->knn_k2, &c->knn_v2,
@@ -226,12 +226,11 @@ GaussOut gauss_out(Ctx* c) {
 
 Items items(Ctx* c) {
     Items it;
-    it.tile = P<int>(c->it_tile);
-    it.k = P<int>(c->it_k);
+    it.rec = P<int4>(c->it_rec);
+    it.tile_rec = P<int4>(c->tile_rec);
+    it.bwd_rec = P<int4>(c->bwd_rec);
     it.tile_K = P<int>(c->tile_K);
     it.tile_item0 = P<int>(c->tile_item0);
-    it.order = P<int>(c->it_order);
-    it.tile_order = P<int>(c->tile_order);
     it.cls = P<int>(c->it_cls);
     return it;
 }
@@ -240,7 +239,7 @@ Entries packed(Ctx* c) {
     Entries pk;
     pk.ids = c->sorted_ids;
     pk.rec = P<float4>(c->rec);
-    pk.qmask = P<uint8_t>(c->qmask);
+    pk.bmask = P<uint16_t>(c->bmask);
     return pk;
 }
 
@@ -431,6 +430,7 @@ int forward(Ctx* c, const MsplatRenderArgs* a, bool training, float* dst_img = n
     ENSURE(c->tile_item0, (size_t)T * 4);
     ENSURE(c->l_chunked, (size_t)T * 4);
     ENSURE(c->tile_done, (size_t)T * 4);
+    ENSURE(c->live_end, (size_t)T * 4);
     ENSURE(c->final_T, Px * 4);
     ENSURE(c->final_idx, Px * 4);
     ENSURE(c->out_img, Px * 12);
@@ -479,7 +479,7 @@ int forward(Ctx* c, const MsplatRenderArgs* a, bool training, float* dst_img = n
     const size_t R = (size_t)std::max<int64_t>(R64, 1);
     const size_t NS = (size_t)segments_bound(R64, nst);
     ENSURE(c->tval, I * 4);
-    ENSURE(c->qmask, I);
+    ENSURE(c->bmask, I * 2);
     ENSURE(c->rkey, R * 4);
     ENSURE(c->rval, R * 4);
     ENSURE(c->rkey2, R * 4);
@@ -488,11 +488,10 @@ int forward(Ctx* c, const MsplatRenderArgs* a, bool training, float* dst_img = n
     ENSURE(c->seg, NS * 16);
     ENSURE(c->phist, NS * SUPER * SUPER * 4);
     const int64_t max_items = items_bound(T, I64);
-    ENSURE(c->it_tile, (size_t)max_items * 4);
-    ENSURE(c->it_k, (size_t)max_items * 4);
-    ENSURE(c->it_order, (size_t)max_items * 4);
-    ENSURE(c->tile_order, (size_t)T * 4);
-    ENSURE(c->it_cls, 4 * 32 * 4);
+    ENSURE(c->it_rec, (size_t)max_items * 16);
+    ENSURE(c->tile_rec, (size_t)T * 16);
+    ENSURE(c->bwd_rec, (size_t)groups_bound(T, I64) * 16);
+    ENSURE(c->it_cls, 6 * 32 * 4);
     const size_t S = (size_t)max_items * TILE_PIX;
     ENSURE(c->c_T, S * 4);
     ENSURE(c->c_C, S * 12);
@@ -502,6 +501,7 @@ int forward(Ctx* c, const MsplatRenderArgs* a, bool training, float* dst_img = n
         ENSURE(c->c_aC, S * 12);
     }
     c->max_items = max_items;
+    c->max_groups = groups_bound(T, I64);
     stage_mark(c, S_TILES);
     TileLists tl{P<int>(c->l_chunked), nullptr, nullptr};
     Items it = items(c);
@@ -530,14 +530,13 @@ int forward(Ctx* c, const MsplatRenderArgs* a, bool training, float* dst_img = n
     if (training) {
         // every chunk's state is kept: the backward's suffix sums run over
         // all chunks of a tile
-        launch_raster_fwd(c->stream, p, max_items, P<Meta>(c->meta_d), it, P<int>(c->tile_bins),
-                          pk, P<float>(c->final_T), P<int>(c->final_idx), img, cb,
+        launch_raster_fwd(c->stream, p, max_items, P<Meta>(c->meta_d), it, pk, P<float>(c->final_T), P<int>(c->final_idx), img, cb,
                           work_counters(c, S_RFWD), P<int>(c->l_chunked), P<int>(c->tile_done));
         launch_raster_merge(c->stream, p, P<Meta>(c->meta_d), P<int>(c->l_chunked), it,
                             P<float>(c->final_T), P<int>(c->final_idx), img, cb, true,
-                            P<int>(c->tile_done));
+                            P<int>(c->tile_done), P<int>(c->live_end));
     } else {
-        launch_render_tiles(c->stream, p, it, P<int>(c->tile_bins), pk, P<float>(c->final_T),
+        launch_render_tiles(c->stream, p, it, pk, P<float>(c->final_T),
                             P<int>(c->final_idx), img, work_counters(c, S_RFWD));
     }
     // the previous call's stage times (it has completed: the event above
@@ -741,10 +740,9 @@ int msplat_hip_train_step(const MsplatTrainArgs* a, int32_t* radii_out, float* l
     // the raster backward's workgroup 0 folds the partials into loss_h[1]
     const LossFold lf{P<float>(c->loss_part), nparts, a->ssim_weight, c->loss_hd + 1};
     stage_mark(c, S_RBWD);
-    launch_raster_bwd(c->stream, p, c->max_items, P<Meta>(c->meta_d), items(c),
-                      P<int>(c->tile_bins), packed(c),
+    launch_raster_bwd(c->stream, p, c->max_groups, P<Meta>(c->meta_d), items(c), packed(c),
                       P<float>(c->final_T), P<int>(c->final_idx), chunks(c),
-                      P<float>(c->v_rendered), P<float>(c->gacc), work_counters(c, S_RBWD), lf);
+                      P<int>(c->live_end), P<float>(c->v_rendered), P<float>(c->gacc), work_counters(c, S_RBWD), lf);
     AdamHP hp;
     for (int g = 0; g < 6; ++g) { hp.step[g] = a->adam_step_sizes[g]; hp.inv_bc2[g] = 1.0f / a->adam_bc2_sqrts[g]; }
     hp.b1 = a->adam_beta1;
@@ -1139,8 +1137,8 @@ int msplat_hip_raster_work(int64_t counts[6]) {
     p.tby = (p.H + BLOCK - 1) / BLOCK;
     unsigned long long* d = P<unsigned long long>(c->count_d);
     if (c->last_N > 0 && c->meta_d.p)
-        launch_raster_work(c->stream, p, c->max_items, P<Meta>(c->meta_d), items(c),
-                           P<int>(c->tile_bins), packed(c), P<int>(c->final_idx), chunks(c), d);
+        launch_raster_work(c->stream, p, c->max_items, P<Meta>(c->meta_d), items(c), packed(c), P<int>(c->final_idx), chunks(c),
+                           P<int>(c->live_end), d);
     unsigned long long h[6];
     HIP_TRY(hipMemcpyAsync(h, d, sizeof(h), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));

@@ -43,22 +43,31 @@ struct GaussOut {
 struct Entries {
     const uint32_t* ids;
     const float4* rec;
-    // One byte per entry: the 4-bit quadrant mask that the training
-    // forward computes for every entry it stages, read back by the backward
-    // (which walks only entries up to the last contributor, all of them
-    // staged by the forward) instead of computing it again.
-    uint8_t* qmask;
+    // The 16-bit block mask of each entry, which the training forward computes
+    // for every entry it stages, read back by the backward (which walks only
+    // entries up to the last contributor, all of them staged by the forward)
+    // instead of computing it again.
+    uint16_t* bmask;
 };
 
-// Work items of the rasteriser: item i covers chunk item_k[i] of tile item_tile[i].
+// Work items of the rasteriser, one per (tile, chunk).  The kernels take one
+// record each, in launch order (heaviest size class first), so that a
+// workgroup knows its range after a single load:
+//   rec[slot]      = (item, tile | flags, first entry, end entry)
+//   tile_rec[slot] = (tile, chunks, first entry, end entry)
+//   bwd_rec[slot] = (first item, tile | flags, first entry, end entry) of the
+//     backward: a whole tile, or up to BWD_GROUP consecutive chunks of one
+// item numbers count the chunks tile by tile (tile_item0).
+constexpr int ITEM_MULTI = 1 << 30;              // the tile has more than one chunk
+constexpr int ITEM_LATE = (int)0x80000000u;      // chunk FWD_P or later of its tile
+constexpr int ITEM_TILE = ITEM_MULTI - 1;
 struct Items {
-    int* tile;
-    int* k;
+    int4* rec;
+    int4* tile_rec;
+    int4* bwd_rec;
     int* tile_K;         // chunks per tile
     int* tile_item0;     // first item of each tile
-    int* order;          // items, heaviest size class first (the raster launch order)
-    int* tile_order;     // tiles, heaviest size class first (the render launch order)
-    int* cls;            // 4 x 32 counters of the size classes (items, tiles; counts, fills)
+    int* cls;            // 6 x 32 counters of the size classes (items, tiles, groups; counts, fills)
 };
 
 // Host-visible summary written by the tile scan.
@@ -69,7 +78,7 @@ struct Meta {
     int32_t n_chunked_tiles;   // tiles with more than one chunk
     int32_t n_large;           // unused (0)
     int32_t n_huge;            // unused (0)
-    int32_t pad;
+    int32_t n_groups;          // records of the backward
 };
 
 // Tile lists written by the tile scan (order within a list is arbitrary).
@@ -204,6 +213,17 @@ constexpr int WORK_SLOT_U64 = 16;
 // Upper bound of the number of (tile, chunk) work items for I intersections.
 inline int64_t items_bound(int64_t T, int64_t I) { return T + I / 512 + I / 2048 + 1; }
 
+// Chunks of one tile that a backward record covers: most of a deep tile's
+// chunks lie behind every pixel's cutoff and have no work, and a wave of their
+// own each, which finds that out after two dependent loads, cost more than the
+// chunks that have some (1M gaussians in a blob at 2594x1680: 89k items, 355k
+// waves, about 0.2 of 0.62 ms).  Images of few tiles (where every tile is cut
+// into chunks) need the chunks' parallelism instead.
+inline __host__ __device__ int bwd_group(int64_t T) { return T < 400 ? 1 : 8; }
+inline int64_t groups_bound(int64_t T, int64_t I) {
+    return bwd_group(T) == 1 ? items_bound(T, I) : T + I / (8 * 512) + 1;
+}
+
 // Rasterisation (raster.hip); grids are sized by items_bound / T and the
 // kernels read the exact counts from meta.  A non-null `work` (the counter
 // sets above) makes the forward add its composited (pixel, entry) pairs to
@@ -217,17 +237,18 @@ inline int64_t items_bound(int64_t T, int64_t I) { return T + I / 512 + I / 2048
 // change no output, are not computed; chunked is the tile scan's list.
 constexpr int FWD_P = 16;
 void launch_raster_fwd(hipStream_t s, const CamParams& p, int64_t max_items, const Meta* meta,
-                       Items it, const int* tile_bins, Entries pk, float* final_T, int* final_idx,
+                       Items it, Entries pk, float* final_T, int* final_idx,
                        float* out_img, ChunkBufs cb, unsigned long long* work, const int* chunked,
                        int* done);
 // Render-only forward, one workgroup per tile (chunked tiles rasterised chunk
 // by chunk up to the merge cutoff); writes the final image, T and index.
-void launch_render_tiles(hipStream_t s, const CamParams& p, Items it, const int* tile_bins,
-                         Entries pk, float* final_T, int* final_idx, float* out_img,
+void launch_render_tiles(hipStream_t s, const CamParams& p, Items it, Entries pk, float* final_T, int* final_idx, float* out_img,
                          unsigned long long* work);
+// Folds the chunked tiles' chunks; live_end[t] (T ints) becomes the item of
+// such a tile from which on no pixel has backward work.
 void launch_raster_merge(hipStream_t s, const CamParams& p, const Meta* meta, const int* chunked,
                          Items it, float* final_T, int* final_idx, float* out_img, ChunkBufs cb,
-                         bool with_suffix, const int* done);
+                         bool with_suffix, const int* done, int* live_end);
 // Fold of the SSIM tiles' loss partials into the loss sum, done by one
 // workgroup of a later kernel (the raster backward's first): in float64, in a
 // fixed order (thread t adds parts t, t + blockDim.x, ... in order, then a
@@ -267,14 +288,14 @@ __device__ inline void loss_fold(const LossFold& lf, double* s) {
 }
 // Workgroup 0 of the launch folds the loss when lf.part is set (loss_fold);
 // the items take workgroups 1 ...
-void launch_raster_bwd(hipStream_t s, const CamParams& p, int64_t max_items, const Meta* meta,
-                       Items it, const int* tile_bins, Entries pk, const float* final_T,
-                       const int* final_idx, ChunkBufs cb, const float* v_out, float* gacc,
-                       unsigned long long* work, const LossFold& lf);
+void launch_raster_bwd(hipStream_t s, const CamParams& p, int64_t max_groups, const Meta* meta,
+                       Items it, Entries pk, const float* final_T,
+                       const int* final_idx, ChunkBufs cb, const int* live_end, const float* v_out,
+                       float* gacc, unsigned long long* work, const LossFold& lf);
 // Adds the six pair counts of the most recent forward/backward into out[6].
 void launch_raster_work(hipStream_t s, const CamParams& p, int64_t max_items, const Meta* meta,
-                        Items it, const int* tile_bins, Entries pk, const int* final_idx,
-                        ChunkBufs cb, unsigned long long* out);
+                        Items it, Entries pk, const int* final_idx,
+                        ChunkBufs cb, const int* live_end, unsigned long long* out);
 
 // The loss: SSIM + L1 forward and backward per 32x32 tile; writes the loss
 // gradient image and one partial (sum SSIM, sum L1, pixels) per tile, and

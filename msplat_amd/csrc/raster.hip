@@ -1,10 +1,11 @@
 // raster.hip — alpha compositing forward, chunk merge and backward.
 //
 // Work decomposition: one 256-thread workgroup (four wave64) per (tile,
-// chunk) item; each wave owns one 8x8 quadrant of the 16x16 tile, one lane per
-// pixel.  Sorted entries (gaussian ids; each entry's projection record is
-// gathered by id) are staged through LDS 256 at a time and read by all lanes
-// as broadcasts.  A tile that is rasterised in one piece writes the
+// chunk) item; each wave owns one 8x8 quadrant of the 16x16 tile and each of
+// its 16-lane rows one 4x4 block of that quadrant, one lane per pixel.
+// Sorted entries (gaussian ids; each entry's projection record is gathered by
+// id) are staged through LDS 256 at a time; every row walks the list of the
+// staged entries that reach its block.  A tile that is rasterised in one piece writes the
 // final image directly; a chunked tile writes per-pixel chunk state that the
 // merge kernel folds front to back.
 //
@@ -16,14 +17,16 @@
 //   backward     rasterize_backward_kernel (.metal:898-1099) and
 //                rasterize_backward_chunked_kernel (.metal:2844-3031)
 // with these MI355X differences: each loaded entry carries a conservative
-// mask of the 8x8 wave quadrants it can reach and a wave walks only the
-// entries of its own quadrant; a workgroup-wide vote stops the forward once
+// mask of the tile's sixteen 4x4 blocks it can reach and a row of lanes walks
+// only the entries of its own block; a workgroup-wide vote stops the forward once
 // every pixel of the item has terminated; the backward reduces each
 // gaussian's per-pixel terms across the 64 lanes of a wave (eight of them
 // transposed through LDS, the ninth by DPP) and nine lanes issue one float
 // atomic each.
 #include "common.hpp"
 #include "kernels.hpp"
+
+#include <utility>
 
 namespace msp {
 
@@ -35,15 +38,25 @@ struct Px {
     bool inside;
 };
 
-__device__ __forceinline__ Px pixel_of(int t, int tbx, int W, int H) {
-    const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
-    const int lx = (w & 1) * 8 + (l & 7), ly = (w >> 1) * 8 + (l >> 3);
+// Pixel of thread tid of the tile's 256.
+__device__ __forceinline__ Px pixel_at(int t, int tbx, int W, int H, int tid) {
+    const int w = tid >> 6, r = (tid >> 4) & 3, i = tid & 15;
+    const int lx = (w & 1) * 8 + (r & 1) * 4 + (i & 3), ly = (w >> 1) * 8 + (r >> 1) * 4 + (i >> 2);
     Px p;
     p.j = (t % tbx) * BLOCK + lx;
     p.i = (t / tbx) * BLOCK + ly;
     p.lp = ly * BLOCK + lx;
     p.inside = p.i < H && p.j < W;
     return p;
+}
+__device__ __forceinline__ Px pixel_of(int t, int tbx, int W, int H) {
+    return pixel_at(t, tbx, W, H, threadIdx.x);
+}
+
+// Lanes below this one in a lane mask.
+__device__ __forceinline__ int lanes_below(uint64_t m) {
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                          __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
 // Pair counters: WORK_SLOTS copies of the counter set, one 128-byte line
@@ -53,59 +66,50 @@ __device__ __forceinline__ unsigned long long* work_slot(unsigned long long* wor
     return work + (size_t)(blockIdx.x % WORK_SLOTS) * WORK_SLOT_U64;
 }
 
-__device__ __forceinline__ void item_range(const Items& it, const int* tile_bins, int item,
-                                           int& t, int& K, int& cs, int& ce) {
-    t = it.tile[item];
-    const int k = it.k[item];
-    K = it.tile_K[t];
-    const int s = tile_bins[2 * t], e = tile_bins[2 * t + 1];
-    if (K == 1) {
-        cs = s;
-        ce = e;
-    } else {
-        cs = s + k * CHUNK;
-        ce = min(cs + CHUNK, e);
-    }
-}
-
-// Minimum over the segment X = const, Y in [y0, y1] of
-// q(X, Y) = 0.5 (a X^2 + c Y^2) + b X Y  (c > 0, ic = 1 / c).
-__device__ __forceinline__ float qmin_edge(float a, float b, float c, float ic, float X, float y0,
-                                           float y1) {
-    const float Y = fminf(fmaxf(-b * X * ic, y0), y1);
-    return 0.5f * (a * X * X + c * Y * Y) + b * X * Y;
-}
-
-// Conservative quadrant mask of one entry: bit w is set when the entry can
-// reach alpha >= 1/255 at a pixel of wave w's 8x8 quadrant of the tile at
-// (tx0, ty0).  The reach is sigma < min(5.55, ln(255 o)); the test takes the
-// exact minimum of the convex quadratic sigma over the quadrant's pixel
-// rectangle (zero when the centre lies inside, else the least of the four
-// edge minima) and compares it with the threshold plus a margin far above
-// fp32 rounding.  Entries outside a quadrant are exactly the ones the
-// per-pixel tests would skip there, so culling them changes no result.
-__device__ __forceinline__ int quad_mask(float x, float y, float a, float b, float c, float o,
-                                         int tx0, int ty0) {
-    if (!(o >= 0.0039f)) return o == o ? 0 : 0xF;      // alpha <= o < 1/255 everywhere
-    const float det = a * c - b * b;
-    if (!(det > 0.f) || !(a > 0.f) || !(c > 0.f) || !(a < 1e30f) || !(c < 1e30f) ||
-        !(fabsf(b) < 1e30f) || !(fabsf(x) < 1e30f) || !(fabsf(y) < 1e30f))
-        return 0xF;
-    const float thr = fminf(5.55f, __logf(255.f * o) + 0.05f) * 1.002f + 1e-3f;
-    const float ia = 1.f / a, ic = 1.f / c;
+// Conservative block mask of one entry: bit 4 w + r is set when the entry can
+// reach alpha >= 1/255 at a pixel of the 4x4 block of row r of wave w, in the
+// tile at (tx0, ty0).  The reach is the ellipse sigma < min(5.55, ln(255 o)),
+// with a margin far above fp32 rounding on that threshold and 1/32 pixel
+// around the blocks.  For the tile's four strips of 4 pixel rows, the part of
+// the ellipse inside a strip spans an interval of x whose ends are the
+// ellipse's extremes with their offset dy clamped to the strip (the ellipse
+// is convex); the blocks of the strip that meet the interval are set.  Entries
+// outside a block are exactly the ones the per-pixel tests would skip there,
+// so culling them changes no result.  About 140 vector instructions (the four
+// exact quadrant minima that a coarser mask of 8x8 quadrants took were 250).
+__device__ __forceinline__ int block_mask(float x, float y, float a, float b, float c, float o,
+                                          int tx0, int ty0) {
+    if (!(o >= 0.0039f)) return o == o ? 0 : 0xFFFF;   // alpha <= o < 1/255 everywhere
+    // a c - b^2 with the rounding error of b^2 put back: needle-shaped conics
+    // leave few bits of the plain difference
+    const float bb = b * b;
+    const float det = fmaf(a, c, -bb) - fmaf(b, b, -bb);
+    if (!(det > 1e-30f) || !(det < 1e30f) || !(a > 0.f) || !(c > 0.f) || !(a < 1e30f) ||
+        !(c < 1e30f) || !(fabsf(x) < 1e30f) || !(fabsf(y) < 1e30f))
+        return 0xFFFF;
+    constexpr float M = 0.03125f;
+    const float thr2 = 2.f * (fminf(5.55f, __logf(255.f * o) + 0.05f) * 1.002f + 1e-3f);
+    const float ia = __builtin_amdgcn_rcpf(a), id = __builtin_amdgcn_rcpf(det);
+    // offsets d = centre - pixel: at offset dy the ellipse spans dx = (-b dy
+    // -+ sqrt(a thr2 - det dy^2)) / a; its largest dx lies at dy = -k
+    const float k = b * __builtin_amdgcn_rcpf(c) * __builtin_amdgcn_sqrtf(c * thr2 * id);
+    const float at = a * thr2, ymax = __builtin_amdgcn_sqrtf(at * id);
+    const float cx = x - (float)tx0, cy = y - (float)ty0;
     int m = 0;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        const float qx0 = (float)(tx0 + (q & 1) * 8), qy0 = (float)(ty0 + (q >> 1) * 8);
-        // offsets d = centre - pixel over the quadrant's pixels
-        const float dx0 = x - (qx0 + 7.f), dx1 = x - qx0;
-        const float dy0 = y - (qy0 + 7.f), dy1 = y - qy0;
-        const bool inside = dx0 <= 0.f && dx1 >= 0.f && dy0 <= 0.f && dy1 >= 0.f;
-        const float e = fminf(fminf(qmin_edge(a, b, c, ic, dx0, dy0, dy1),
-                                    qmin_edge(a, b, c, ic, dx1, dy0, dy1)),
-                              fminf(qmin_edge(c, b, a, ia, dy0, dx0, dx1),
-                                    qmin_edge(c, b, a, ia, dy1, dx0, dx1)));
-        if (inside || e < thr) m |= 1 << q;
+        const float d0 = cy - (4 * q + 3 + M), d1 = cy - (4 * q - M);
+        const float yl = __builtin_amdgcn_fmed3f(-k, d0, d1), yr = __builtin_amdgcn_fmed3f(k, d0, d1);
+        const float el = fmaf(-det * yl, yl, at), er = fmaf(-det * yr, yr, at);
+        // pixel interval [cx - largest dx, cx - smallest dx] in tile coordinates
+        const float l = cx - fmaf(-b, yl, __builtin_amdgcn_sqrtf(fmaxf(el, 0.f))) * ia - M;
+        const float r = cx - fmaf(-b, yr, -__builtin_amdgcn_sqrtf(fmaxf(er, 0.f))) * ia + M;
+        const int j0 = (int)fminf(fmaxf(ceilf((l - 3.f) * 0.25f), 0.f), 4.f);
+        const int j1 = (int)fminf(fmaxf(floorf(r * 0.25f), -1.f), 3.f);
+        int s = (0xF << j0) & (0xF >> (3 - j1)) & 0xF;
+        if (d0 > ymax || d1 < -ymax) s = 0;           // the strip misses the ellipse
+        const int sh = 8 * (q >> 1) + 2 * (q & 1);
+        m |= (s & 3) << sh | (s >> 2) << (sh + 4);
     }
     return m;
 }
@@ -130,121 +134,167 @@ __device__ __forceinline__ float4 lds_f4(const float4* base, int qb) {
         __builtin_assume_aligned(reinterpret_cast<const char*>(base) + qb, 16));
 }
 
-// LDS row of one reduced value: the 64 lane partials.  The 8-lane groups of
-// odd rows read their two 16-byte halves in the opposite order, so that the
-// two groups served in the same LDS cycle (rows 2p and 2p + 1) read
-// disjoint banks.
-constexpr int RED_ROW = 64;
+// Byte offset of the dummy record behind the staged ones: opacity 0, no pixel
+// takes it.
+constexpr int DUMMY = 256;
 
-// Sum over the 64 lanes of a wave of eight values per lane, through the
-// wave's own LDS area red[8][RED_ROW], in three parts: red8_write puts each
-// lane's eight values in rows 0..7; red8_issue loads, for lane l, the eight
-// partials 8 (l & 7) .. 8 (l & 7) + 7 of row l >> 3; red8_finish adds them
-// and combines the eight lanes of each group by DPP (xor 1, xor 2, mirror
-// within 8), so that lane 8k ends with the total of value k.  The raster
-// backward reads a step's partials back one evaluated step after it wrote
-// them, so that the LDS round trip overlaps that step's arithmetic.  Only
-// this wave touches red, and a wave's LDS accesses are performed in order:
-// a read issued before the next write sees the earlier partials, with no
-// barrier; wave barriers keep the compiler from moving the accesses across
-// each other.  All lanes must be active.
-__device__ __forceinline__ void red8_write(const float* v, int lane, float* red) {
+// The value of lane N of each row of 16, in all lanes of the row.
+template <int N>
+__device__ __forceinline__ int row_bcast(int v) {
+    return __builtin_amdgcn_mov_dpp(v, 0x150 + N, 0xF, 0xF, true);
+}
+
+// Entry lists of a wave's four rows: the batch's entries whose mask (s_mask,
+// one per staged entry, bit 4 w + r) names the row's block, in order, as one
+// byte each in s_list[256 r ...].  Returns this lane's
+// row's count; longest is the largest of the four (both wave-uniform per row).
+// Costs about 9 instructions per row and 64 entries.
+__device__ __forceinline__ int build_lists(int w, const uint16_t* s_mask, uint8_t* s_list,
+                                           int& longest) {
+    const int lane = threadIdx.x & 63;
+    int n[4] = {0, 0, 0, 0};
 #pragma unroll
-    for (int k = 0; k < 8; ++k) red[k * RED_ROW + lane] = v[k];
-}
-__device__ __forceinline__ void red8_issue(int lane, const float* red, float4& a, float4& b) {
-    const int g = lane >> 3, h = (g & 1) << 2;
-    const float* rb = red + g * RED_ROW + (lane & 7) * 8;
-    a = *reinterpret_cast<const float4*>(rb + h);
-    b = *reinterpret_cast<const float4*>(rb + (h ^ 4));
-}
-__device__ __forceinline__ float red8_finish(float4 a, float4 b) {
-    float u = ((a.x + a.y) + (a.z + a.w)) + ((b.x + b.y) + (b.z + b.w));
-    u += dpp<0xB1>(u);     // quad_perm [1,0,3,2]
-    u += dpp<0x4E>(u);     // quad_perm [2,3,0,1]
-    u += dpp<0x141>(u);    // row_half_mirror: lane ^ 7 within each 8 lanes
-    // completed here, with every lane active, so that the move and the add
-    // stay one DPP add (sunk into a caller's lane-masked block they are two)
-    asm volatile("" : "+v"(u));
-    return u;
+    for (int ch = 0; ch < 256; ch += 64) {
+        const int q = ch + lane;
+        const unsigned m = (unsigned)s_mask[q] >> (4 * w);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const uint64_t in = wave_ballot((m >> r) & 1u);
+            const int at = n[r] + lanes_below(in);
+            if (lane_of(in)) s_list[256 * r + at] = (uint8_t)q;
+            n[r] += __popcll(in);
+        }
+    }
+    __builtin_amdgcn_wave_barrier();
+    longest = max(max(n[0], n[1]), max(n[2], n[3]));
+    const int row = lane >> 4;
+    return row == 0 ? n[0] : row == 1 ? n[1] : row == 2 ? n[2] : n[3];
 }
 
+// LDS of a forward workgroup: 256 staged entries and the dummy.
+struct FwdLds {
+    float4 geo[257];         // x, y, conic a, b
+    float4 col[257];         // conic c, opacity, clamped r, g
+    float4 aux[257];         // clamped b; 16-byte stride shares the address
+    uint16_t mask[256];      // block masks
+    uint8_t list[4][4 * 256];   // per wave: its rows' entry lists
+};
+
+// One entry of the forward at this lane's pixel: qb is the byte offset of the
+// entry's record, different from row to row.  A lane whose pixel has stopped
+// (or lies outside the image) has thr = 2 and takes nothing.  Lanes without a
+// hit run the same steps with alpha = 0, which leaves T and the colours as
+// they are (the staged colours are finite); the rare step in which a pixel
+// stops is put right in a branch.
+template <bool COUNT>
+__device__ __forceinline__ void fwd_step(int qb, float fx, float fy, const FwdLds& s, float& thr,
+                                         float& T, float& C0, float& C1, float& C2, int& lqb,
+                                         unsigned& ncl) {
+    const float4 g = lds_f4(s.geo, qb);
+    const float4 c = lds_f4(s.col, qb);
+    const float cb = lds_f4(s.aux, qb).x;
+    const float dx = g.x - fx, dy = g.y - fy;
+    const float sigma = fmaf(0.5f, fmaf(g.z, dx * dx, c.x * dy * dy), g.w * dx * dy);
+    const float alpha = fminf(0.999f, c.y * exp_neg_raster(sigma_clamp(sigma)));
+    // hit: the pixel is live and alpha >= 1/255 (sigma out of range: alpha < 1/255)
+    const bool hit = alpha >= thr;
+    float a = hit ? alpha : 0.f;
+    float nT = T * (1.f - a);
+    lqb = hit ? qb : lqb;
+    if (COUNT) ncl += hit ? 1u : 0u;
+    // T > 1e-4 at every pixel, so only a hit can get here
+    const uint64_t sm = mask_le(nT, 1e-4f);
+    if (__builtin_expect(sm != 0, 0)) {      // once per pixel: this entry is not composited
+        if (lane_of(sm)) {
+            a = 0.f;
+            nT = T;
+            thr = 2.f;
+            lqb = qb - (int)sizeof(float4);  // the entry before this one
+            if (COUNT) --ncl;
+        }
+    }
+    const float vis = a * T;
+    C0 = fmaf(c.z, vis, C0);
+    C1 = fmaf(c.w, vis, C1);
+    C2 = fmaf(cb, vis, C2);
+    T = nT;
+}
+
+// Four consecutive list entries (positions B .. B + 3 of the row's 16).
+template <bool COUNT, int B>
+__device__ __forceinline__ void fwd_four(int off, float fx, float fy, const FwdLds& s, float& thr,
+                                         float& T, float& C0, float& C1, float& C2, int& lqb,
+                                         unsigned& ncl) {
+    fwd_step<COUNT>(row_bcast<B>(off), fx, fy, s, thr, T, C0, C1, C2, lqb, ncl);
+    fwd_step<COUNT>(row_bcast<B + 1>(off), fx, fy, s, thr, T, C0, C1, C2, lqb, ncl);
+    fwd_step<COUNT>(row_bcast<B + 2>(off), fx, fy, s, thr, T, C0, C1, C2, lqb, ncl);
+    fwd_step<COUNT>(row_bcast<B + 3>(off), fx, fy, s, thr, T, C0, C1, C2, lqb, ncl);
+}
+
+// Colour of a staged entry's channel: clamped from below as the reference
+// does, and finite, so that alpha = 0 composites nothing.
+__device__ __forceinline__ float staged_colour(float raw) {
+    return fminf(fmaxf(raw + 0.5f, 0.f), 3.402823466e38f);
+}
+
+// Bound: vector and scalar issue.  Rows with lists of their own take 2.23M wave
+// steps where waves with one list for an 8 x 8 quadrant took 3.08M (1.5M
+// gaussians at 1297x840), and a step has no scalar mask work: forward 165 ->
+// 137 us there, 499 -> 402 us for a 1M blob at 2594x1680, 30 -> 20 us for 10k
+// at 256x256, and in renders 118 -> 97 us (500k at 1297x840) and 1151 -> 1039
+// us (6M at 4946x3286).
 // Forward of the entries [cs, ce) at this lane's pixel, from the state
 // (T, C, last) passed in: entries are staged 256 at a time through LDS and
-// each wave walks the entries of its quadrant in order.  live: the lanes
-// whose pixel still composites (wave-uniform mask).  Every thread of the
-// workgroup calls this with the same range (it holds workgroup barriers).
-// MASKS (the training forward): each staged entry's quadrant mask is also
+// each row walks the entries of its block in order.  live: this lane's pixel
+// still composites.  Every thread of the workgroup calls this with the same
+// range (it holds workgroup barriers).
+// MASKS (the training forward): each staged entry's block mask is also
 // stored for the backward.
 template <bool COUNT, bool MASKS = false>
-__device__ __forceinline__ void fwd_range(int cs, int ce, uint64_t live, float fx, float fy,
-                                          int tx0, int ty0, const Entries& pk, float4* s_geo,
-                                          float4* s_col, float4* s_aux, float& T, float& C0,
-                                          float& C1, float& C2, int& last, unsigned& ncl,
-                                          unsigned& nwit) {
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+__device__ __forceinline__ void fwd_range(int cs, int ce, bool live, float fx, float fy,
+                                          int tx0, int ty0, const Entries& pk, FwdLds& s, float& T,
+                                          float& C0, float& C1, float& C2, int& last,
+                                          unsigned& ncl, unsigned& nwit) {
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    float thr = live ? 1.f / 255.f : 2.f;
+    if (tid == 0) s.geo[DUMMY] = s.col[DUMMY] = s.aux[DUMMY] = make_float4(0.f, 0.f, 0.f, 0.f);
     for (int b = cs; b < ce; b += 256) {
-        if (__syncthreads_and(live == 0)) break;
+        if (__syncthreads_and(thr > 1.f)) break;
         const int idx = b + tid;
         int mask = 0;
-        float bl_raw = 0.f;
         if (idx < ce) {
             const float4* r = pk.rec + 4 * (size_t)pk.ids[idx];
             const float4 g = r[0];
             const float4 c = r[1];
-            bl_raw = r[2].x;
-            mask = quad_mask(g.x, g.y, g.z, g.w, c.x, c.y, tx0, ty0);
-            if (MASKS) pk.qmask[idx] = (uint8_t)mask;
-            s_geo[tid] = g;
-            s_col[tid] = make_float4(c.x, c.y, fmaxf(c.z + 0.5f, 0.f), fmaxf(c.w + 0.5f, 0.f));
+            const float bl = r[2].x;
+            mask = block_mask(g.x, g.y, g.z, g.w, c.x, c.y, tx0, ty0);
+            if (MASKS) pk.bmask[idx] = (uint16_t)mask;
+            s.geo[tid] = g;
+            s.col[tid] = make_float4(c.x, c.y, staged_colour(c.z), staged_colour(c.w));
+            s.aux[tid] = make_float4(staged_colour(bl), 0.f, 0.f, 0.f);
         }
-        s_aux[tid] = make_float4(fmaxf(bl_raw + 0.5f, 0.f), __int_as_float(mask), 0.f, 0.f);
+        s.mask[tid] = (uint16_t)mask;
         __syncthreads();
-        const int nb = min(256, ce - b);
+        if (wave_ballot(thr < 1.f) == 0) continue;
+        int longest;
+        const int n = build_lists(w, s.mask, s.list[w], longest);
+        const uint8_t* list = s.list[w] + 256 * (lane >> 4);
         // this batch's last contributor as the entry's LDS byte offset (a
         // vector register copy per step), turned into the index at the end
         int lqb = INT_MIN;
-        for (int ch = 0; ch < nb; ch += 64) {
-            const int q = ch + lane;
-            uint64_t m = wave_ballot(q < nb && ((__float_as_int(s_aux[q].y) >> w) & 1));
-            if (COUNT) nwit += __popcll(m);
-            // the chunk's byte offset in a VGPR: each entry's offset is then
-            // one vector shift-add from the bit index, shared by its LDS reads
-            int chb = ch * (int)sizeof(float4);
-            asm volatile("" : "+v"(chb));
-            while (m) {
-                const int qb = chb + pop_low_bit(m) * (int)sizeof(float4);
-                const float4 g = lds_f4(s_geo, qb);
-                const float4 c = lds_f4(s_col, qb);
-                const float cb = lds_f4(s_aux, qb).x;
-                const float dx = g.x - fx, dy = g.y - fy;
-                const float sigma = fmaf(0.5f, fmaf(g.z, dx * dx, c.x * dy * dy), g.w * dx * dy);
-                const float alpha = fminf(0.999f, c.y * exp_neg_raster(sigma_clamp(sigma)));
-                // hit: live && !(alpha < 1/255) (sigma out of range: alpha < 1/255)
-                const uint64_t hm = live & mask_uge(alpha, 1.f / 255.f);
-                const float nT = T * (1.f - alpha);
-                const uint64_t sm = hm & mask_le(nT, 1e-4f);     // stops here
-                const uint64_t cm = hm & ~sm;                    // composites
-                // the colour reads complete behind the exp above, not inside
-                // the update block
-                asm volatile("" ::"v"(c.z), "v"(c.w), "v"(cb));
-                // only the compositing lanes execute the update (an exec-masked
-                // block: no per-lane selects)
-                if (lane_of(cm)) {
-                    const float vis = alpha * T;
-                    C0 = fmaf(c.z, vis, C0);
-                    C1 = fmaf(c.w, vis, C1);
-                    C2 = fmaf(cb, vis, C2);
-                    T = nT;
-                    lqb = qb;
-                    if (COUNT) ++ncl;
-                }
-                if (sm) {      // at most once per pixel: the entry before this one
-                    if (lane_of(sm)) lqb = qb - (int)sizeof(float4);
-                    live &= ~sm;
-                }
-            }
-            if (live == 0) break;
+        for (int p = 0; p < longest; p += 16) {
+            const int q = p + (lane & 15);
+            const int off = (q < n ? (int)list[q] : DUMMY) * (int)sizeof(float4);
+            if (COUNT) nwit += min(longest - p, 16);
+            fwd_four<COUNT, 0>(off, fx, fy, s, thr, T, C0, C1, C2, lqb, ncl);
+            if (p + 4 >= longest) break;
+            fwd_four<COUNT, 4>(off, fx, fy, s, thr, T, C0, C1, C2, lqb, ncl);
+            if (p + 8 >= longest) break;
+            fwd_four<COUNT, 8>(off, fx, fy, s, thr, T, C0, C1, C2, lqb, ncl);
+            if (p + 12 >= longest) break;
+            fwd_four<COUNT, 12>(off, fx, fy, s, thr, T, C0, C1, C2, lqb, ncl);
+            if (wave_ballot(thr < 1.f) == 0) break;
         }
         if (lqb != INT_MIN) last = b + (lqb >> 4);   // sizeof(float4) = 16; -16 gives b - 1
     }
@@ -264,14 +314,11 @@ __device__ __forceinline__ void add_work(unsigned long long* work, unsigned ncl,
 // One work item of the training forward: its chunk's state (chunked tile)
 // or the tile's final pixels (tile in one piece).
 template <bool COUNT>
-__device__ __forceinline__ void fwd_item(int item, int W, int H, int tbx, float bg0, float bg1,
-                                         float bg2, const Items& it, const int* tile_bins,
-                                         const Entries& pk, float* final_T, int* final_idx,
+__device__ __forceinline__ void fwd_item(int4 rec, int W, int H, int tbx, float bg0, float bg1,
+                                         float bg2, const Entries& pk, float* final_T, int* final_idx,
                                          float* out_img, const ChunkBufs& cb,
-                                         unsigned long long* work, float4* s_geo, float4* s_col,
-                                         float4* s_aux) {
-    int t, K, cs, ce;
-    item_range(it, tile_bins, item, t, K, cs, ce);
+                                         unsigned long long* work, FwdLds& s) {
+    const int item = rec.x, t = rec.y & ITEM_TILE, cs = rec.z, ce = rec.w;
     const Px px = pixel_of(t, tbx, W, H);
     float fx = (float)px.j, fy = (float)px.i;
     // opaque to the compiler, so that the loop keeps the converted
@@ -283,11 +330,10 @@ __device__ __forceinline__ void fwd_item(int item, int W, int H, int tbx, float 
     int last = cs - 1;
     unsigned ncl = 0;       // pairs composited by this lane
     unsigned nwit = 0;      // entries this wave evaluated (wave-uniform)
-    fwd_range<COUNT, true>(cs, ce, wave_ballot(px.inside), fx, fy, tx0, ty0, pk, s_geo, s_col, s_aux, T,
-                           C0, C1, C2, last, ncl, nwit);
+    fwd_range<COUNT, true>(cs, ce, px.inside, fx, fy, tx0, ty0, pk, s, T, C0, C1, C2, last, ncl, nwit);
     add_work<COUNT>(work, ncl, nwit);
     if (!px.inside) return;
-    if (K == 1) {
+    if (!(rec.y & ITEM_MULTI)) {
         const size_t pix = (size_t)px.i * W + px.j;
         final_T[pix] = T;
         final_idx[pix] = last;
@@ -304,46 +350,56 @@ __device__ __forceinline__ void fwd_item(int item, int W, int H, int tbx, float 
     }
 }
 
-// Chunks 0 .. kmax - 1 of every tile, one item per workgroup.
+// Chunks 0 .. FWD_P - 1 of every tile, one item per workgroup.
 template <bool COUNT>
 __global__ __launch_bounds__(256) void k_raster_fwd(int W, int H, int tbx, float bg0, float bg1,
                                                     float bg2, const Meta* __restrict__ meta,
-                                                    Items it,
-                                                    const int* __restrict__ tile_bins, Entries pk,
+                                                    Items it, Entries pk,
                                                     float* __restrict__ final_T,
                                                     int* __restrict__ final_idx,
                                                     float* __restrict__ out_img, ChunkBufs cb,
-                                                    unsigned long long* __restrict__ work,
-                                                    int kmax) {
-    __shared__ float4 s_geo[256];    // x, y, conic a, b
-    __shared__ float4 s_col[256];    // conic c, opacity, clamped r, g
-    __shared__ float4 s_aux[256];    // clamped b, mask (bits); 16-byte stride shares the address
+                                                    unsigned long long* __restrict__ work) {
+    __shared__ FwdLds s;
     // items in launch order (heaviest size class first)
     if ((int)blockIdx.x >= meta->n_items) return;
-    const int item = it.order[blockIdx.x];
-    if (it.k[item] >= kmax) return;
-    fwd_item<COUNT>(item, W, H, tbx, bg0, bg1, bg2, it, tile_bins, pk, final_T, final_idx, out_img, cb,
-             work, s_geo, s_col, s_aux);
+    const int4 rec = it.rec[blockIdx.x];
+    if (rec.y & ITEM_LATE) return;
+    fwd_item<COUNT>(rec, W, H, tbx, bg0, bg1, bg2, pk, final_T, final_idx, out_img, cb,
+             work, s);
 }
 
-// Chunks kmin and later of the tiles not marked done, the workgroups striding
-// over the items (few items qualify, so a small grid visits them all).
+// Chunks FWD_P and later of the tiles not marked done: few items qualify, so a
+// small grid visits them all, each thread looking at one item of its
+// workgroup's next 256 and the workgroup rasterising those found.
 template <bool COUNT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_raster_fwd_tail(int W, int H, int tbx,
                                                          const Meta* __restrict__ meta, Items it,
-                                                         const int* __restrict__ tile_bins,
                                                          Entries pk, ChunkBufs cb,
                                                          unsigned long long* __restrict__ work,
-                                                         int kmin, const int* __restrict__ done) {
-    __shared__ float4 s_geo[256];
-    __shared__ float4 s_col[256];
-    __shared__ float4 s_aux[256];
+                                                         const int* __restrict__ done) {
+    __shared__ FwdLds s;
+    __shared__ int s_slot[256];
+    __shared__ int s_n;
     const int n = meta->n_items;
-    for (int item = blockIdx.x; item < n; item += gridDim.x) {
-        if (it.k[item] < kmin || done[it.tile[item]]) continue;
-        // chunked tiles only (k >= kmin > 0): no final pixels are written
-        fwd_item<COUNT>(item, W, H, tbx, 0.f, 0.f, 0.f, it, tile_bins, pk, nullptr, nullptr, nullptr, cb,
-                 work, s_geo, s_col, s_aux);
+    for (int i0 = blockIdx.x; i0 < n; i0 += 256 * gridDim.x) {
+        // items i0, i0 + gridDim.x, ...: neighbouring ones, which belong to
+        // one tile, go to different workgroups
+        const int64_t i = i0 + (int64_t)threadIdx.x * gridDim.x;
+        bool mine = false;
+        if (i < n) {
+            const int y = it.rec[i].y;
+            mine = (y & ITEM_LATE) && !done[y & ITEM_TILE];
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) s_n = 0;
+        __syncthreads();
+        if (mine) s_slot[atomicAdd(&s_n, 1)] = (int)i;
+        __syncthreads();
+        const int m = s_n;
+        for (int j = 0; j < m; ++j)
+            // chunked tiles only: no final pixels are written
+            fwd_item<COUNT>(it.rec[s_slot[j]], W, H, tbx, 0.f, 0.f, 0.f, pk, nullptr, nullptr, nullptr, cb,
+                            work, s);
     }
 }
 
@@ -362,17 +418,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
 template <bool COUNT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_render_tiles(int W, int H, int tbx, float bg0,
                                                       float bg1, float bg2, Items it,
-                                                      const int* __restrict__ tile_bins,
                                                       Entries pk, float* __restrict__ final_T,
                                                       int* __restrict__ final_idx,
                                                       float* __restrict__ out_img,
                                                       unsigned long long* __restrict__ work) {
-    __shared__ float4 s_geo[256];
-    __shared__ float4 s_col[256];
-    __shared__ float4 s_aux[256];
-    const int t = it.tile_order[blockIdx.x];   // heaviest size class first
-    const int K = it.tile_K[t];
-    const int s = tile_bins[2 * t], e = tile_bins[2 * t + 1];
+    __shared__ FwdLds lds;
+    const int4 rec = it.tile_rec[blockIdx.x];   // heaviest size class first
+    const int t = rec.x, K = rec.y, s = rec.z, e = rec.w;
     const Px px = pixel_of(t, tbx, W, H);
     float fx = (float)px.j, fy = (float)px.i;
     asm volatile("" : "+v"(fx), "+v"(fy));
@@ -382,8 +434,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
     int li;
     if (K == 1) {
         li = s - 1;
-        fwd_range<COUNT>(s, e, wave_ballot(px.inside), fx, fy, tx0, ty0, pk, s_geo, s_col, s_aux, Tr, R0,
-                  R1, R2, li, ncl, nwit);
+        fwd_range<COUNT>(s, e, px.inside, fx, fy, tx0, ty0, pk, lds, Tr, R0, R1, R2, li, ncl, nwit);
     } else {
         li = -1;
         bool done = !px.inside;
@@ -392,8 +443,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
             const int cs = s + k * CHUNK, ce = min(cs + CHUNK, e);
             float T = 1.f, C0 = 0.f, C1 = 0.f, C2 = 0.f;
             int last = cs - 1;
-            fwd_range<COUNT>(cs, ce, wave_ballot(!done), fx, fy, tx0, ty0, pk, s_geo, s_col, s_aux, T,
-                      C0, C1, C2, last, ncl, nwit);
+            fwd_range<COUNT>(cs, ce, !done, fx, fy, tx0, ty0, pk, lds, T, C0, C1, C2, last, ncl, nwit);
             if (!done) {
                 R0 = fmaf(C0, Tr, R0);
                 R1 = fmaf(C1, Tr, R1);
@@ -466,8 +516,11 @@ __global__ __launch_bounds__(256) void k_raster_merge(int W, int H, int tbx, flo
                                                       int* __restrict__ final_idx,
                                                       float* __restrict__ out_img, ChunkBufs cb,
                                                       int with_suffix, const int* __restrict__ done,
-                                                      int P) {
+                                                      int P, int* __restrict__ live_end) {
+    __shared__ int s_cut;
     if ((int)blockIdx.x >= meta->n_chunked_tiles) return;
+    if (threadIdx.x == 0) s_cut = 0;
+    __syncthreads();
     const int t = chunked[blockIdx.x];
     const int K = it.tile_K[t], i0 = it.tile_item0[t];
     // chunks with state: all K, or the first P of a tile whose later chunks
@@ -475,15 +528,15 @@ __global__ __launch_bounds__(256) void k_raster_merge(int W, int H, int tbx, flo
     const int Kc = (done && done[t]) ? min(K, P) : K;
     const int lp = threadIdx.x, lx = lp & 15, ly = lp >> 4;
     const int j = (t % tbx) * BLOCK + lx, i = (t / tbx) * BLOCK + ly;
-    if (i >= H || j >= W) return;
+    const bool inside = i < H && j < W;
     float Tr = 1.f, R0 = 0.f, R1 = 0.f, R2 = 0.f;
-    int li = -1, cutoff = K;
+    int li = -1, cutoff = inside ? K : 0;
     // Chunks are folded front to back, stopping at an empty chunk or once
     // T <= 1e-4.  The state of MG chunks is loaded ahead of folding them
     // (every k < K is a valid chunk), so a tile with hundreds of chunks
     // costs one memory round trip per MG chunks instead of two per chunk.
     constexpr int MG = 8;
-    bool stop = false;
+    bool stop = !inside;
     for (int k0 = 0; k0 < Kc && !stop; k0 += MG) {
         int cf[MG];
         float cT[MG], c0[MG], c1[MG], c2[MG];
@@ -516,7 +569,17 @@ __global__ __launch_bounds__(256) void k_raster_merge(int W, int H, int tbx, flo
             }
         }
     }
-    for (int k = cutoff; k < K; ++k) cb.cidx[(size_t)(i0 + k) * TILE_PIX + lp] = -1;
+    // The chunks past a pixel's cutoff have no backward work there.  The items
+    // from the largest cutoff of the tile's pixels on have none at all: the
+    // backward stops at that item (live_end) and reads nothing of them, and
+    // their indexes need no marking.
+    const int wave_cut = wave_max_i(cutoff);
+    if ((threadIdx.x & 63) == 0) atomicMax(&s_cut, wave_cut);
+    __syncthreads();
+    const int cut = s_cut;
+    if (threadIdx.x == 0) live_end[t] = i0 + cut;
+    if (!inside) return;
+    for (int k = cutoff; k < cut; ++k) cb.cidx[(size_t)(i0 + k) * TILE_PIX + lp] = -1;
     const size_t pix = (size_t)i * W + j;
     final_T[pix] = Tr;
     final_idx[pix] = li;
@@ -565,77 +628,263 @@ __global__ __launch_bounds__(256) void k_raster_merge(int W, int H, int tbx, flo
     }
 }
 
+// Inclusive product / sum scans over the 16 lanes of each row, of four values
+// at once: the four chains fill the two wait states that a DPP read needs
+// after the write of its source (the first pair of s_nop covers the caller's
+// last write).  A lane without a source keeps its value.  All lanes must be
+// active.
+#define MSP_ROW_SCAN4(op, v)                                                              \
+    asm volatile(                                                                        \
+        "s_nop 1\n\t" MSP_ROW_SCAN4_STEP(op, "1") MSP_ROW_SCAN4_STEP(op, "2")            \
+            MSP_ROW_SCAN4_STEP(op, "4") MSP_ROW_SCAN4_STEP(op, "8") "s_nop 1"            \
+        : "+v"((v)[0]), "+v"((v)[1]), "+v"((v)[2]), "+v"((v)[3]))
+#define MSP_ROW_SCAN4_STEP(op, n)                                              \
+    op " %0, %0, %0 row_shr:" n " row_mask:0xf bank_mask:0xf\n\t"              \
+    op " %1, %1, %1 row_shr:" n " row_mask:0xf bank_mask:0xf\n\t"              \
+    op " %2, %2, %2 row_shr:" n " row_mask:0xf bank_mask:0xf\n\t"              \
+    op " %3, %3, %3 row_shr:" n " row_mask:0xf bank_mask:0xf\n\t"
+
+// The value of lane N of each row of 16, in all lanes of the row.
+template <int N>
+__device__ __forceinline__ float row_bcast(float v) {
+    return __int_as_float(row_bcast<N>(__float_as_int(v)));
+}
+// acc + a's value in lane N of the row x b, rounded once.  The compiler does
+// not fold the broadcast into a multiply-add by itself.  a must have been
+// written at least two instructions before (settled()).
+template <int N>
+__device__ __forceinline__ void row_fmac(float& acc, float a, float b) {
+    asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+        : "+v"(acc) : "v"(a), "v"(b), "n"(N));
+}
+// A point after which a, b and c may be read through DPP, and before which
+// the compiler forms no broadcast of them or of d (a loop's broadcasts are
+// not hoisted into registers of their own).
+__device__ __forceinline__ void settled(float& a, float& b, float& c, int& d) {
+    asm volatile("s_nop 1" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
+}
+// The value of the lane before within the row; lane 0 gets first.
+__device__ __forceinline__ float row_before(float v, float first) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(first), __float_as_int(v), 0x111,
+                                                      0xF, 0xF, false));
+}
+__device__ __forceinline__ int row_max(int v) {
+    v = max(v, __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true));    // quad_perm [1,0,3,2]
+    v = max(v, __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, true));    // quad_perm [2,3,0,1]
+    v = max(v, __builtin_amdgcn_mov_dpp(v, 0x124, 0xF, 0xF, true));   // row_ror:4
+    return max(v, __builtin_amdgcn_mov_dpp(v, 0x128, 0xF, 0xF, true));  // row_ror:8
+}
+
+// f(0), f(1), ... f(N - 1) with the index as a compile-time constant.
+template <typename F, int... P>
+__device__ __forceinline__ void for_each_of(F& f, std::integer_sequence<int, P...>) {
+    (f(std::integral_constant<int, P>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void for_each_to(F f) {
+    for_each_of(f, std::make_integer_sequence<int, N>{});
+}
+
+// Window of a backward wave: up to WIN entries that reach its quadrant, and
+// the dummy behind them; their gradient sums; the rows' lists of window slots.
+// 8.1 KB; the 107 vector registers allow four waves a SIMD (five, at 96
+// registers with spills, measured 2% slower; 128 entries the same).
+constexpr int WIN = 96;
+struct BwdLds {
+    float4 geo[WIN + 1];      // x, y, conic a, b
+    float4 col[WIN + 1];      // conic c, opacity, clamped r, g
+    float2 aux[WIN + 1];      // clamped b, -entry index (bits)
+    int gid[WIN];             // gaussian
+    float4 sa[WIN], sb[WIN];  // the sums 0..3 and 4..7 of gacc's nine
+    float sc[WIN];            // and the last
+    uint8_t list[4][WIN];
+};
+
+// The state of a row's 16 pixels, pixel p of the row's block in register p
+// (the same in all lanes of the row): transmittance behind and E (below).
+struct RowState {
+    float T[16], E[16];
+};
+
+// This lane's entry and its sums over the pixels of the row's block.
+struct EntrySums {
+    float s0, s1, s2, s11, s12, s22;   // v_sigma, v_sigma (dx, dy, dx^2, dx dy, dy^2)
+    float c0, c1, c2;                  // fac v_out
+};
+
+// Column X of the row's block (pixels X, X + 4, X + 8, X + 12), all 16 entries
+// of the group at once: lane l of a row holds the row's l-th entry, deepest
+// first.  vo0..2 and bf are per pixel, in the pixel's lane: the pixel takes the
+// entries up to index bf (tested as the sign of bf - index, formed by an add:
+// a subtraction that takes its subtrahend through DPP, v_subrev, was measured
+// to broadcast the other operand).
+template <bool COUNT, int X>
+__device__ __forceinline__ void bwd_column(float4 g, float4 c, float blue, int nidx, float fx0,
+                                           const float* dy, const float* cy2, float vo0, float vo1,
+                                           float vo2, int bf, RowState& st, EntrySums& es,
+                                           unsigned& ngrad) {
+    const float dx = g.x - (fx0 + (float)X);
+    const float dx2 = dx * dx, bx = g.w * dx;
+    float ag[4], ra[4], P[4], Tn[4], fac[4], RV[4], S[4];
+    auto pixel = [&](auto yc) {
+        constexpr int y = decltype(yc)::value, p = 4 * y + X;
+        const float sigma = fmaf(0.5f, fmaf(g.z, dx2, cy2[y]), bx * dy[y]);
+        const float alpha = c.y * exp_neg_raster(sigma_clamp(sigma));
+        // a gradient flows where the entry is not behind the pixel's last
+        // contributor and 1/255 <= alpha < 0.999 (one unsigned compare of the
+        // bits; NaN is above); elsewhere alpha = 0 leaves the state as it is
+        // (1 / (1 - 0) = 1) and makes every term zero
+        const unsigned behind = (unsigned)(row_bcast<p>(bf) + nidx) & 0x80000000u;
+        const bool ok = ((__float_as_uint(alpha) - 0x3B808081u) | behind) < 0x3F7FBE77u - 0x3B808081u;
+        ag[y] = ok ? alpha : 0.f;
+        if (COUNT) ngrad += (unsigned)__popcll(wave_ballot(ok));
+        // hardware reciprocal (1 ulp, exact at 1): the backward is compared
+        // with a tolerance
+        P[y] = ra[y] = __builtin_amdgcn_rcpf(1.f - ag[y]);
+    };
+    for_each_to<4>(pixel);
+    MSP_ROW_SCAN4("v_mul_f32_dpp", P);
+    auto terms = [&](auto yc) {
+        constexpr int y = decltype(yc)::value, p = 4 * y + X;
+        Tn[y] = st.T[p] * P[y];
+        fac[y] = ag[y] * Tn[y];
+        RV[y] = row_bcast<p>(vo0) * c.z;
+        row_fmac<p>(RV[y], vo1, c.w);
+        row_fmac<p>(RV[y], vo2, blue);
+        S[y] = fac[y] * RV[y];
+        row_fmac<p>(es.c0, vo0, fac[y]);
+        row_fmac<p>(es.c1, vo1, fac[y]);
+        row_fmac<p>(es.c2, vo2, fac[y]);
+        st.T[p] = row_bcast<15>(Tn[y]);
+    };
+    for_each_to<4>(terms);
+    MSP_ROW_SCAN4("v_add_f32_dpp", S);
+    float s = 0.f, t = 0.f;     // the column's sums of v and v dy
+    auto sums = [&](auto yc) {
+        constexpr int y = decltype(yc)::value, p = 4 * y + X;
+        const float Ei = st.E[p] + S[y];
+        const float E = row_before(Ei, st.E[p]);    // behind this entry
+        st.E[p] = row_bcast<15>(Ei);
+        // v_alpha = sum_k (r_k Tn - (B_k + T_final bg_k) ra) v_out_k
+        const float v_alpha = fmaf(Tn[y], RV[y], -ra[y] * E);
+        const float v = -ag[y] * v_alpha;
+        const float vy = v * dy[y];
+        s = y == 0 ? v : s + v;
+        t = y == 0 ? vy : t + vy;
+        es.s22 = fmaf(vy, dy[y], es.s22);
+    };
+    for_each_to<4>(sums);
+    es.s0 += s;
+    es.s1 = fmaf(s, dx, es.s1);
+    es.s11 = fmaf(s, dx2, es.s11);
+    es.s12 = fmaf(t, dx, es.s12);
+    es.s2 += t;
+    // one column at a time: interleaved columns would need more registers
+    // than the four pixels of one, which already fill the DPP wait states,
+    // and so would sums put off until they are used
+    asm volatile("" : "+v"(es.s0), "+v"(es.s1), "+v"(es.s2), "+v"(es.s11), "+v"(es.s12), "+v"(es.s22),
+                 "+v"(es.c0), "+v"(es.c1), "+v"(es.c2));
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// The backward turns the forward's roles round: a row of 16 lanes takes 16
+// entries of its block's list at once, one per lane and deepest first, and
+// goes through the block's 16 pixels one after the other.  What a pixel
+// carries from entry to entry (the transmittance behind the entry and the
+// colour accumulated behind it) becomes a product and a sum scan over the
+// row's lanes (four DPP steps each), and an entry's gradient sums over the
+// pixels stay in its lane's registers: no reduction over lanes.
+// One wave is a workgroup of its own, for one quadrant of a record: no
+// barriers, and a heavy quadrant holds up nothing but itself.  It gathers a
+// window of up to WIN entries that reach its quadrant, walks them, and adds
+// the window's sums to gacc with consecutive lanes on consecutive floats.
+// The window's sums are kept in LDS; an LDS float atomic takes 193 cycles of
+// the CU for a wave whatever its addresses (a plain store 7.5), so each row
+// adds its sums in turn with ordinary loads and stores (entries of one row are
+// distinct, those of different rows are not).
+// Bound: the vector units (153M instructions in 1.5M gaussians' step at
+// 1297x840, four cycles each, are its 286 us).  Per (entry, pixel) pair of
+// lanes: about 57 vector instructions, no scalar ones and no LDS access, where
+// lane = pixel took 65, 11 and 11; a block of 4 x 4 pixels leaves fewer pairs
+// without a gradient than an 8 x 8 quadrant (2.10M wave steps against 2.75M).
+// Measured against lane = pixel with 8 x 8 quadrants: 10k gaussians at 256x256
+// 33 -> 17 us, 120k at 324x210 59 -> 38 us, 1M in a blob at 2594x1680 581 ->
+// 552 us, 1.5M at 1297x840 283 -> 286 us.  The colour terms on the matrix cores
+// (v_mfma_f32_4x4x1) instead of by DPP: the same time, from register spills.
 // COUNT: count the wave's evaluated entries and gradient pairs into work
 // (a launch without counters runs the variant that does not count).
 template <bool COUNT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_raster_bwd(int W, int H, int tbx, float bg0, float bg1,
-                                                    float bg2, const Meta* __restrict__ meta,
-                                                    Items it,
-                                                    const int* __restrict__ tile_bins, Entries pk,
-                                                    const float* __restrict__ final_T,
-                                                    const int* __restrict__ final_idx,
-                                                    ChunkBufs cb, const float* __restrict__ v_out,
-                                                    float* __restrict__ gacc,
-                                                    unsigned long long* __restrict__ work,
-                                                    LossFold lf) {
-    __shared__ float4 s_geo[256];    // x, y, conic a, b
-    __shared__ float4 s_col[256];    // conic c, opacity, clamped r, g
-    __shared__ float4 s_aux[256];    // clamped b, opacity - 1, accumulator byte offset, mask
-    // per-wave gradient reductions; its first word holds the workgroup's
-    // largest final index before the entry loop uses the area
-    __shared__ float4 s_red4[4 * 8 * RED_ROW / 4];
-    int& s_max = *reinterpret_cast<int*>(s_red4);
-    // Workgroup 0 folds the loss partials of the SSIM tiles (in the reduction
-    // area) and takes no item: dispatched first, it runs beside the heaviest
-    // items instead of at the end of the launch.
-    static_assert(sizeof(s_red4) >= 3 * 256 * sizeof(double), "loss fold area");
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_raster_bwd(
+    int W, int H, int tbx, float bg0, float bg1, float bg2, const Meta* __restrict__ meta, Items it,
+    Entries pk, const float* __restrict__ final_T, const int* __restrict__ final_idx, ChunkBufs cb,
+    const int* __restrict__ live_end, const float* __restrict__ v_out,
+    float* __restrict__ gacc, unsigned long long* __restrict__ work, LossFold lf) {
+    __shared__ BwdLds s;
+    // Workgroup 0 folds the loss partials of the SSIM tiles and takes no
+    // item: dispatched first, it runs beside the heaviest items instead of
+    // at the end of the launch.
+    static_assert(sizeof(s.sa) >= 3 * 64 * sizeof(double), "loss fold area");
     if (blockIdx.x == 0) {
-        if (lf.part) loss_fold(lf, reinterpret_cast<double*>(s_red4));
+        if (lf.part) loss_fold(lf, reinterpret_cast<double*>(s.sa));
         return;
     }
-    // items in launch order (heaviest size class first)
-    const int bi = (int)blockIdx.x - 1;
-    if (bi >= meta->n_items) return;
-    const int item = it.order[bi];
-    int t, K, cs, ce;
-    item_range(it, tile_bins, item, t, K, cs, ce);
-    const Px px = pixel_of(t, tbx, W, H);
-    const float fx = (float)px.j, fy = (float)px.i;
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    // items in launch order (heaviest size class first); the four quadrants of
+    // an item are eight workgroups apart, so they run on one XCD at about the
+    // same time and gather the entries' records through one L2
+    const int wg = (int)blockIdx.x - 1;
+    const int bi = (wg >> 5) * 8 + (wg & 7), w = (wg >> 3) & 3;
+    if (bi >= meta->n_groups) return;
+    const int4 rec = it.bwd_rec[bi];
+    const bool multi = (rec.y & ITEM_MULTI) != 0;
+    const int t = rec.y & ITEM_TILE;
+    const int item_end = multi ? live_end[t] : rec.x + 1;   // (of a chunked tile) items with work
+    if (rec.x >= item_end) return;
+    const int lane = threadIdx.x, i = lane & 15, row = lane >> 4;
+    const Px px = pixel_at(t, tbx, W, H, 64 * w + lane);
 
+    const size_t pix = (size_t)px.i * W + px.j;
+    if (lane == 0) {
+        s.geo[WIN] = s.col[WIN] = make_float4(0.f, 0.f, 0.f, 0.f);
+        s.aux[WIN] = make_float2(0.f, 0.f);
+    }
+    for (int k = lane; k < WIN; k += 64) {
+        s.sa[k] = s.sb[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+        s.sc[k] = 0.f;
+    }
+    // the pixel whose lane this is lies in column i & 3, row i >> 2 of its
+    // block, whose first pixel is (fx0, fy0)
+    const float fx0 = (float)(px.j - (i & 3)), fy0 = (float)(px.i - (i >> 2));
+    unsigned ngrad = 0;     // pairs of this wave that carry a gradient (wave-uniform)
+    unsigned nwit = 0;      // entries this wave evaluated (wave-uniform)
+
+    // the record's chunks one after the other (a tile in one piece is one);
+    // each starts from its own state
+    int item = rec.x;
+    for (int cs = rec.z, ce; cs < rec.w && item < item_end; cs = ce, ++item) {
+    ce = multi ? min(cs + CHUNK, rec.w) : rec.w;
     float T = 1.f, Tfin = 1.f, B0 = 0.f, B1 = 0.f, B2 = 0.f, vo0 = 0.f, vo1 = 0.f, vo2 = 0.f;
     // bf = cs - 1 for pixels outside the image: no entry passes e_idx <= bf
     int bf = cs - 1;
-    unsigned ngrad = 0;     // pairs of this wave that carry a gradient (wave-uniform)
-    // After the reductions lane 8k holds the k-th of the eight LDS sums and
-    // lane 63 the ninth; each adds it at byte kofs of the gaussian's nine
-    // accumulators, all nine in one atomic instruction.
-    const bool own = (lane & 7) == 0 || lane == 63;
-    const uint32_t kofs = lane == 63 ? 32u : (uint32_t)(lane >> 3) * 4u;
-    float* red = reinterpret_cast<float*>(s_red4) + w * 8 * RED_ROW;
-    // The gradient sums of an evaluated step are completed during the next
-    // one: pend says a step's eight partials are in red, pofs is that
-    // gaussian's accumulator byte offset and puo its per-lane opacity term.
-    bool pend = false;
-    uint32_t pofs = 0u;
-    float puo = 0.f;
-    unsigned nwit = 0;      // entries this wave evaluated (wave-uniform)
+    const size_t chunk_pix = (size_t)item * TILE_PIX + px.lp;
+    if (px.inside) bf = multi ? cb.cidx[chunk_pix] : final_idx[pix];
+    // the last contributor of each row's pixels (wave-uniform)
+    const int rbf = row_max(bf);
+    const int row_bf[4] = {__builtin_amdgcn_readlane(rbf, 0), __builtin_amdgcn_readlane(rbf, 16),
+                           __builtin_amdgcn_readlane(rbf, 32), __builtin_amdgcn_readlane(rbf, 48)};
+    int top = min(ce - 1, max(max(row_bf[0], row_bf[1]), max(row_bf[2], row_bf[3])));
+    if (top < cs) continue;
     if (px.inside) {
-        const size_t pix = (size_t)px.i * W + px.j;
         Tfin = final_T[pix];
         vo0 = v_out[3 * pix + 0];
         vo1 = v_out[3 * pix + 1];
         vo2 = v_out[3 * pix + 2];
-        if (K == 1) {
+        if (!multi) {
             T = Tfin;
-            bf = final_idx[pix];
         } else {
-            const size_t o = (size_t)item * TILE_PIX + px.lp;
-            T = cb.pT[o] * cb.cT[o];
-            B0 = cb.aC[3 * o + 0];
-            B1 = cb.aC[3 * o + 1];
-            B2 = cb.aC[3 * o + 2];
-            bf = cb.cidx[o];
+            T = cb.pT[chunk_pix] * cb.cT[chunk_pix];
+            B0 = cb.aC[3 * chunk_pix + 0];
+            B1 = cb.aC[3 * chunk_pix + 1];
+            B2 = cb.aC[3 * chunk_pix + 2];
         }
     }
     // The colour terms of v_alpha enter only as sum_k v_out_k (...)_k:
@@ -643,134 +892,115 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
     // v_out_k T_final bg_k are carried instead of the three channels.
     // E = D + TB, the two carried together: D changes, TB does not
     const float TB = fmaf(Tfin * bg2, vo2, fmaf(Tfin * bg1, vo1, (Tfin * bg0) * vo0));
-    float E = fmaf(B2, vo2, fmaf(B1, vo1, B0 * vo0)) + TB;
-    // wave-uniform (readfirstlane): the entry loop indexes then live in scalar registers
-    const int wave_bf = __builtin_amdgcn_readfirstlane(wave_max_i(bf));
-    if (tid == 0) s_max = cs - 1;
-    __syncthreads();
-    if (lane == 0) atomicMax(&s_max, wave_bf);
-    __syncthreads();
-    const int hi = min(ce - 1, s_max);
+    const float E = fmaf(B2, vo2, fmaf(B1, vo1, B0 * vo0)) + TB;
+    RowState st;
+    auto spread = [&](auto pc) {
+        constexpr int p = decltype(pc)::value;
+        st.T[p] = row_bcast<p>(T);
+        st.E[p] = row_bcast<p>(E);
+    };
+    for_each_to<16>(spread);
 
-    for (int top = hi; top >= cs; top -= 256) {
-        __syncthreads();
-        const int idx = top - tid;
-        // the entry's quadrant mask from the forward; an entry that reaches
-        // no quadrant is not gathered
-        const int mask = idx >= cs ? (int)pk.qmask[idx] : 0;
-        if (mask) {
-            const int gid = (int)pk.ids[idx];
-            const float4* r = pk.rec + 4 * (size_t)gid;
-            const float4 g = r[0];
-            float4 c = r[1];
-            const float braw = r[2].x;
-            s_geo[tid] = g;
-            s_col[tid] = make_float4(c.x, c.y, fmaxf(c.z + 0.5f, 0.f), fmaxf(c.w + 0.5f, 0.f));
-            // z: byte offset of the gaussian's accumulators (N * 36 < 2^31)
-            s_aux[tid] = make_float4(fmaxf(braw + 0.5f, 0.f), c.y - 1.f, __int_as_float(gid * 36),
-                                     __int_as_float(mask));
-        } else {
-            s_aux[tid].w = __int_as_float(0);
+    // the next 64 entries' block masks and ids, loaded ahead of their use
+    int idx = top - lane;
+    unsigned mask = idx >= cs ? pk.bmask[idx] : 0u;
+    int gid = idx >= cs ? (int)pk.ids[idx] : 0;
+    while (top >= cs) {
+        // fill the window, 64 entries at a time while they fit
+        int nw = 0, n[4] = {0, 0, 0, 0};
+        while (top >= cs) {
+            // rows this entry is wanted by: its block is reached, and it is
+            // not behind the last contributor of the row's pixels
+            unsigned m = (mask >> (4 * w)) & 15u;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (idx > row_bf[r]) m &= ~(1u << r);
+            const uint64_t in = wave_ballot(m != 0u);
+            const int cnt = __popcll(in);
+            if (nw + cnt > WIN) break;
+            const int slot = nw + lanes_below(in);
+            if (m) {
+                const float4* r = pk.rec + 4 * (size_t)gid;
+                const float4 g = r[0];
+                const float4 c = r[1];
+                const float braw = r[2].x;
+                s.geo[slot] = g;
+                s.col[slot] = make_float4(c.x, c.y, fmaxf(c.z + 0.5f, 0.f), fmaxf(c.w + 0.5f, 0.f));
+                s.aux[slot] = make_float2(fmaxf(braw + 0.5f, 0.f), __int_as_float(-idx));
+                s.gid[slot] = gid;
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const uint64_t b = wave_ballot((m >> r) & 1u);
+                const int at = n[r] + lanes_below(b);
+                if (lane_of(b)) s.list[r][at] = (uint8_t)slot;
+                n[r] += __popcll(b);
+            }
+            nw += cnt;
+            top -= 64;
+            idx = top - lane;
+            mask = idx >= cs ? pk.bmask[idx] : 0u;
+            gid = idx >= cs ? (int)pk.ids[idx] : 0;
         }
-        __syncthreads();
-        const int nb = min(256, top - cs + 1);
-        const int q0 = max(0, top - wave_bf);
-        const int qlo = top - bf;      // this pixel takes entries qq >= qlo (e_idx <= bf)
-        // in bytes of the LDS arrays, so that the step's index test compares
-        // two VGPRs; clamped to [0, 256] first, which keeps the test's outcome
-        // for every qq in [0, 256) (bf = -1 of a cut-off chunk makes qlo a
-        // global entry index, too large to scale)
-        const int qlob = min(max(qlo, 0), 256) * (int)sizeof(float4);
-        for (int ch = (q0 / 64) * 64; ch < nb; ch += 64) {
-            const int q = ch + lane;
-            uint64_t m = wave_ballot(q >= q0 && q < nb &&
-                                     ((__float_as_int(s_aux[q].w) >> w) & 1));
-            if (COUNT) nwit += __popcll(m);
-            // the chunk's byte offset in a VGPR: each entry's offset is then
-            // one vector shift-add from the bit index, shared by its LDS reads
-            int chb = ch * (int)sizeof(float4);
-            asm volatile("" : "+v"(chb));
-            while (m) {
-                const int qb = chb + pop_low_bit(m) * (int)sizeof(float4);
-                const float4 g = lds_f4(s_geo, qb);
-                const float4 c = lds_f4(s_col, qb);
-                const float4 x = lds_f4(s_aux, qb);
-                const float dx = g.x - fx, dy = g.y - fy;
-                const float sigma = fmaf(0.5f, fmaf(g.z, dx * dx, c.x * dy * dy), g.w * dx * dy);
-                const float alpha = fminf(0.999f, c.y * exp_neg_raster(sigma_clamp(sigma)));
-                // valid: qq >= qlo && !(alpha < 1/255) (sigma out of range: alpha < 1/255)
-                const uint64_t vmask = mask_ge_i(qb, qlob) & mask_uge(alpha, 1.f / 255.f);
-                if (vmask == 0) continue;
-                // the previous evaluated step's partials (written a step ago):
-                // read now (unused when there is none), summed below, after
-                // this step's arithmetic
-                float4 pa, pb;
-                __builtin_amdgcn_wave_barrier();
-                red8_issue(lane, red, pa, pb);
-                // Branch-free per lane: lanes without a gradient run the same
-                // steps with alpha = 0, which leaves their state as it is
-                // (1 / (1 - 0) = 1 exactly, so Tn = T; fac = 0, so E is
-                // unchanged) and makes every term they contribute zero.
-                const uint64_t gmask = vmask & mask_lt(alpha, 0.999f);
-                const float ag = lane_of(gmask) ? alpha : 0.f;
-                if (COUNT) ngrad += (unsigned)__popcll(gmask);
-                const float r0 = c.z, r1 = c.w, r2 = x.x;   // max(raw + 0.5, 0)
-                // hardware reciprocal (1 ulp, exact at 1): the backward is
-                // compared with a tolerance
-                const float ra = __builtin_amdgcn_rcpf(1.f - ag);
-                const float Tn = T * ra;
-                const float fac = ag * Tn;
-                // v_alpha = sum_k (r_k Tn - (B_k + T_final bg_k) ra) v_out_k
-                const float RV = fmaf(r2, vo2, fmaf(r1, vo1, r0 * vo0));
-                const float v_alpha = fmaf(Tn, RV, -ra * E);
-                E = fmaf(fac, RV, E);
-                T = Tn;
-                // v_sigma: zero (signed) on the lanes without a gradient
-                const float vsg = -ag * v_alpha;
-                // v_xy = v_sigma (a dx + b dy, b dx + c dy) and v_conic =
-                // v_sigma / 2 (dx^2, dx dy, dy^2) are linear in the moments
-                // below with the gaussian's own conic, the same in every
-                // tile: the moments are summed, the projection backward
-                // applies the conic once per gaussian.
-                const float w0 = vsg * dx, w1 = vsg * dy;
-                float v[8];
-                v[0] = w0;
-                v[1] = w1;
-                v[2] = w0 * dx;
-                v[3] = w0 * dy;
-                v[4] = w1 * dy;
-                v[5] = fac * vo0;
-                v[6] = fac * vo1;
-                v[7] = fac * vo2;
-                // The previous step's sums follow this step's arithmetic
-                // (the empty asm keeps them there, so that the loads' latency
-                // is spent on it); the opacity (logit) term -v_sigma (1 - o)
-                // goes to lane 63 of them (lanes 60..62 are no owners).  v_rgb
-                // of a channel whose raw colour + 0.5 < 0 is dropped by its
-                // consumers (the mask is per gaussian, not per pixel).
-                asm volatile("" : "+v"(pa.x), "+v"(pa.y), "+v"(pa.z), "+v"(pa.w), "+v"(pb.x),
-                             "+v"(pb.y), "+v"(pb.z), "+v"(pb.w) : "v"(v[7]), "v"(v[4]));
-                if (pend) {
-                    const float s = wave_sum_into_lane63(puo, red8_finish(pa, pb));
-                    float* ap = reinterpret_cast<float*>(reinterpret_cast<char*>(gacc) + (pofs + kofs));
-                    if (own) atomicAdd(ap, s);
+        __builtin_amdgcn_wave_barrier();
+        const int longest = max(max(n[0], n[1]), max(n[2], n[3]));
+        const int mine = row == 0 ? n[0] : row == 1 ? n[1] : row == 2 ? n[2] : n[3];
+        for (int p0 = 0; p0 < longest; p0 += 16) {
+            const int slot = p0 + i < mine ? (int)s.list[row][p0 + i] : WIN;
+            const float4 g = s.geo[slot];
+            const float4 c = s.col[slot];
+            const float blue = s.aux[slot].x;
+            const int nidx = __float_as_int(s.aux[slot].y);
+            if (COUNT) nwit += min(longest - p0, 16);
+            float dy[4], cy2[4];
+#pragma unroll
+            for (int y = 0; y < 4; ++y) {
+                dy[y] = g.y - (fy0 + (float)y);
+                cy2[y] = c.x * dy[y] * dy[y];
+            }
+            EntrySums es{};
+            settled(vo0, vo1, vo2, bf);
+            bwd_column<COUNT, 3>(g, c, blue, nidx, fx0, dy, cy2, vo0, vo1, vo2, bf, st, es, ngrad);
+            bwd_column<COUNT, 2>(g, c, blue, nidx, fx0, dy, cy2, vo0, vo1, vo2, bf, st, es, ngrad);
+            bwd_column<COUNT, 1>(g, c, blue, nidx, fx0, dy, cy2, vo0, vo1, vo2, bf, st, es, ngrad);
+            bwd_column<COUNT, 0>(g, c, blue, nidx, fx0, dy, cy2, vo0, vo1, vo2, bf, st, es, ngrad);
+            // v_xy = v_sigma (a dx + b dy, b dx + c dy) and v_conic = v_sigma
+            // / 2 (dx^2, dx dy, dy^2) are linear in these moments with the
+            // gaussian's own conic, the same in every tile: the projection
+            // backward applies the conic once per gaussian.  The opacity
+            // (logit) term is -v_sigma (1 - o).  v_rgb of a channel whose raw
+            // colour + 0.5 < 0 is dropped by its consumers.
+            const float so = es.s0 * (c.y - 1.f);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if (row == r && slot < WIN) {
+                    float4 a = s.sa[slot], b = s.sb[slot];
+                    a.x += es.s1;
+                    a.y += es.s2;
+                    a.z += es.s11;
+                    a.w += es.s12;
+                    b.x += es.s22;
+                    b.y += es.c0;
+                    b.z += es.c1;
+                    b.w += es.c2;
+                    s.sa[slot] = a;
+                    s.sb[slot] = b;
+                    s.sc[slot] += so;
                 }
                 __builtin_amdgcn_wave_barrier();
-                red8_write(v, lane, red);
-                __builtin_amdgcn_wave_barrier();
-                pend = true;
-                pofs = (uint32_t)__builtin_amdgcn_readfirstlane(__float_as_int(x.z));
-                puo = vsg * x.y;
             }
         }
-    }
-    if (pend) {   // the last evaluated step's sums
+        // the window's sums, consecutive lanes taking consecutive floats of a
+        // gaussian's nine; entries without a gradient add nothing
+        for (int k = lane; k < 9 * nw; k += 64) {
+            const int e = (int)((unsigned)k / 9u), q = k - 9 * e;
+            float* a = q < 8 ? reinterpret_cast<float*>(q < 4 ? s.sa : s.sb) + 4 * e + (q & 3) : s.sc + e;
+            const float v = *a;
+            *a = 0.f;
+            if (v != 0.f) atomicAdd(gacc + 9 * (size_t)s.gid[e] + q, v);
+        }
         __builtin_amdgcn_wave_barrier();
-        float4 pa, pb;
-        red8_issue(lane, red, pa, pb);
-        const float s = wave_sum_into_lane63(puo, red8_finish(pa, pb));
-        float* ap = reinterpret_cast<float*>(reinterpret_cast<char*>(gacc) + (pofs + kofs));
-        if (own) atomicAdd(ap, s);
+    }
     }
     if (COUNT && work) {
         unsigned long long* ws = work_slot(work);
@@ -787,14 +1017,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
 // define the algorithmic flops of the roofline; they change no state.
 __global__ __launch_bounds__(256) void k_raster_work(int W, int H, int tbx,
                                                      const Meta* __restrict__ meta, Items it,
-                                                     const int* __restrict__ tile_bins, Entries pk,
+                                                     Entries pk,
                                                      const int* __restrict__ final_idx,
                                                      ChunkBufs cb,
+                                                     const int* __restrict__ live_end,
                                                      unsigned long long* __restrict__ out) {
-    const int item = blockIdx.x;
-    if (item >= meta->n_items) return;
-    int t, K, cs, ce;
-    item_range(it, tile_bins, item, t, K, cs, ce);
+    if ((int)blockIdx.x >= meta->n_items) return;
+    const int4 rec = it.rec[blockIdx.x];
+    const int item = rec.x, t = rec.y & ITEM_TILE, cs = rec.z, ce = rec.w;
     const Px px = pixel_of(t, tbx, W, H);
     unsigned n[6] = {0u, 0u, 0u, 0u, 0u, 0u};
     if (px.inside) {
@@ -815,8 +1045,9 @@ __global__ __launch_bounds__(256) void k_raster_work(int W, int H, int tbx,
             ++n[2];
             T = nT;
         }
-        const int bf = K == 1 ? final_idx[(size_t)px.i * W + px.j]
-                              : cb.cidx[(size_t)item * TILE_PIX + px.lp];
+        const int bf = !(rec.y & ITEM_MULTI) ? final_idx[(size_t)px.i * W + px.j]
+                       : item < live_end[t]  ? cb.cidx[(size_t)item * TILE_PIX + px.lp]
+                                             : -1;
         for (int i = min(bf, ce - 1); i >= cs; --i) {
             ++n[3];
             const float4* r = pk.rec + 4 * (size_t)pk.ids[i];
@@ -841,15 +1072,15 @@ __global__ __launch_bounds__(256) void k_raster_work(int W, int H, int tbx,
 }  // namespace
 
 void launch_raster_work(hipStream_t s, const CamParams& p, int64_t max_items, const Meta* meta,
-                        Items it, const int* tile_bins, Entries pk, const int* final_idx,
-                        ChunkBufs cb, unsigned long long* out) {
+                        Items it, Entries pk, const int* final_idx,
+                        ChunkBufs cb, const int* live_end, unsigned long long* out) {
     if (max_items <= 0) return;
     hipLaunchKernelGGL(k_raster_work, dim3((unsigned)max_items), dim3(256), 0, s, p.W, p.H, p.tbx,
-                       meta, it, tile_bins, pk, final_idx, cb, out);
+                       meta, it, pk, final_idx, cb, live_end, out);
 }
 
 void launch_raster_fwd(hipStream_t s, const CamParams& p, int64_t max_items, const Meta* meta,
-                       Items it, const int* tile_bins, Entries pk, float* final_T, int* final_idx,
+                       Items it, Entries pk, float* final_T, int* final_idx,
                        float* out_img, ChunkBufs cb, unsigned long long* work, const int* chunked,
                        int* done) {
     if (max_items <= 0) return;
@@ -858,62 +1089,62 @@ void launch_raster_fwd(hipStream_t s, const CamParams& p, int64_t max_items, con
     // the counting variants only when pair counters are asked for
     if (work)
         hipLaunchKernelGGL(k_raster_fwd<true>, dim3((unsigned)max_items), dim3(256), 0, s, p.W, p.H,
-                           p.tbx, p.bg[0], p.bg[1], p.bg[2], meta, it, tile_bins, pk, final_T,
-                           final_idx, out_img, cb, work, FWD_P);
+                           p.tbx, p.bg[0], p.bg[1], p.bg[2], meta, it, pk, final_T,
+                           final_idx, out_img, cb, work);
     else
         hipLaunchKernelGGL(k_raster_fwd<false>, dim3((unsigned)max_items), dim3(256), 0, s, p.W, p.H,
-                           p.tbx, p.bg[0], p.bg[1], p.bg[2], meta, it, tile_bins, pk, final_T,
-                           final_idx, out_img, cb, work, FWD_P);
+                           p.tbx, p.bg[0], p.bg[1], p.bg[2], meta, it, pk, final_T,
+                           final_idx, out_img, cb, work);
     const int T = p.tbx * p.tby;
     hipLaunchKernelGGL(k_chunk_done, dim3((unsigned)std::min(T, 256)), dim3(256), 0, s, p.W, p.H,
                        p.tbx, meta, chunked, it, cb, done);
     const dim3 tg((unsigned)std::min<int64_t>(max_items, 1024));
     if (work)
         hipLaunchKernelGGL(k_raster_fwd_tail<true>, tg, dim3(256), 0, s, p.W, p.H, p.tbx, meta, it,
-                           tile_bins, pk, cb, work, FWD_P, (const int*)done);
+                           pk, cb, work, (const int*)done);
     else
         hipLaunchKernelGGL(k_raster_fwd_tail<false>, tg, dim3(256), 0, s, p.W, p.H, p.tbx, meta, it,
-                           tile_bins, pk, cb, work, FWD_P, (const int*)done);
+                           pk, cb, work, (const int*)done);
 }
 
-void launch_render_tiles(hipStream_t s, const CamParams& p, Items it, const int* tile_bins,
-                         Entries pk, float* final_T, int* final_idx, float* out_img,
+void launch_render_tiles(hipStream_t s, const CamParams& p, Items it, Entries pk, float* final_T, int* final_idx, float* out_img,
                          unsigned long long* work) {
     const int T = p.tbx * p.tby;
     if (T <= 0) return;
     if (work)
         hipLaunchKernelGGL(k_render_tiles<true>, dim3((unsigned)T), dim3(256), 0, s, p.W, p.H, p.tbx,
-                           p.bg[0], p.bg[1], p.bg[2], it, tile_bins, pk, final_T, final_idx, out_img,
+                           p.bg[0], p.bg[1], p.bg[2], it, pk, final_T, final_idx, out_img,
                            work);
     else
         hipLaunchKernelGGL(k_render_tiles<false>, dim3((unsigned)T), dim3(256), 0, s, p.W, p.H, p.tbx,
-                           p.bg[0], p.bg[1], p.bg[2], it, tile_bins, pk, final_T, final_idx, out_img,
+                           p.bg[0], p.bg[1], p.bg[2], it, pk, final_T, final_idx, out_img,
                            work);
 }
 
 void launch_raster_merge(hipStream_t s, const CamParams& p, const Meta* meta, const int* chunked,
                          Items it, float* final_T, int* final_idx, float* out_img, ChunkBufs cb,
-                         bool with_suffix, const int* done) {
+                         bool with_suffix, const int* done, int* live_end) {
     const int T = p.tbx * p.tby;
     hipLaunchKernelGGL(k_raster_merge, dim3(T), dim3(256), 0, s, p.W, p.H, p.tbx, p.bg[0], p.bg[1],
                        p.bg[2], meta, chunked, it, final_T, final_idx, out_img, cb,
-                       with_suffix ? 1 : 0, done, FWD_P);
+                       with_suffix ? 1 : 0, done, FWD_P, live_end);
 }
 
-void launch_raster_bwd(hipStream_t s, const CamParams& p, int64_t max_items, const Meta* meta,
-                       Items it, const int* tile_bins, Entries pk, const float* final_T,
-                       const int* final_idx, ChunkBufs cb, const float* v_out, float* gacc,
-                       unsigned long long* work, const LossFold& lf) {
-    // workgroup 0 folds the loss, the others take the items
-    const int64_t g = std::max<int64_t>(max_items, 0) + 1;
+void launch_raster_bwd(hipStream_t s, const CamParams& p, int64_t max_groups, const Meta* meta,
+                       Items it, Entries pk, const float* final_T,
+                       const int* final_idx, ChunkBufs cb, const int* live_end, const float* v_out,
+                       float* gacc, unsigned long long* work, const LossFold& lf) {
+    // workgroup 0 folds the loss, the others take the records' quadrants (eight
+    // records at a time)
+    const int64_t g = (std::max<int64_t>(max_groups, 0) + 7) / 8 * 32 + 1;
     if (work)
-        hipLaunchKernelGGL(k_raster_bwd<true>, dim3((unsigned)g), dim3(256), 0, s, p.W, p.H,
-                           p.tbx, p.bg[0], p.bg[1], p.bg[2], meta, it, tile_bins, pk, final_T,
-                           final_idx, cb, v_out, gacc, work, lf);
+        hipLaunchKernelGGL(k_raster_bwd<true>, dim3((unsigned)g), dim3(64), 0, s, p.W, p.H,
+                           p.tbx, p.bg[0], p.bg[1], p.bg[2], meta, it, pk, final_T,
+                           final_idx, cb, live_end, v_out, gacc, work, lf);
     else
-        hipLaunchKernelGGL(k_raster_bwd<false>, dim3((unsigned)g), dim3(256), 0, s, p.W, p.H,
-                           p.tbx, p.bg[0], p.bg[1], p.bg[2], meta, it, tile_bins, pk, final_T,
-                           final_idx, cb, v_out, gacc, work, lf);
+        hipLaunchKernelGGL(k_raster_bwd<false>, dim3((unsigned)g), dim3(64), 0, s, p.W, p.H,
+                           p.tbx, p.bg[0], p.bg[1], p.bg[2], meta, it, pk, final_T,
+                           final_idx, cb, live_end, v_out, gacc, work, lf);
 }
 
 }  // namespace msp

@@ -433,3 +433,43 @@ def test_scratch_reuse_across_sizes(dev):
     m2, _ = _render_and_compare(dev, little)
     m3, _ = _render_and_compare(dev, big)
     assert m2["total_isect"] < m1["total_isect"] == m3["total_isect"]
+
+
+def _block_scene(n, width, height, seed, needles=False, opaque=False):
+    """n gaussians over one corner of the image, most of them in the first
+    tiles: footprints from a pixel to several blocks, or needles up to the
+    image's size, of any direction."""
+    rng = np.random.default_rng(seed)
+    f = np.float32
+    sc = small_scene(n=n, width=width, height=height, seed_off=300 + seed % 50)
+    cam = sc.cameras[0]
+    # in front of the camera, at the image's first pixels
+    c2w = np.asarray(cam.cam_to_world, np.float64)
+    z = rng.uniform(2.0, 4.0, n)
+    u, v = rng.uniform(-2, 24, n), rng.uniform(-2, 24, n)
+    local = np.stack([(u - cam.cx) / cam.fx * z, -(v - cam.cy) / cam.fy * z, -z], 1)
+    sc.means = (local @ c2w[:3, :3].T + c2w[:3, 3]).astype(f)
+    px = z / cam.fx      # world size of a pixel
+    if needles:
+        s = np.stack([px * 10 ** rng.uniform(1.0, 2.5, n), px * 0.05, px * 0.02], 1)
+    else:
+        s = px[:, None] * 10 ** rng.uniform(-0.5, 1.0, (n, 3))
+    sc.scales = np.log(s).astype(f)
+    # opacities around 1/255 (logit -5.54) up to the 0.999 cap (logit 6.9)
+    sc.opacities = (rng.uniform(4.0, 9.0, (n, 1)) if opaque else rng.uniform(-6.0, 1.0, (n, 1))).astype(f)
+    return sc
+
+
+# rows of 16 entries, backward windows of 96, staged batches of 256, chunks of 512
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 33, 95, 97, 193, 257, 700])
+def test_raster_block_edges(dev, n):
+    """The rasteriser's 4x4 blocks: list lengths around its groups, windows
+    and batches, tiles cut by the image edge, entries at the alpha limits."""
+    _train_compare(dev, _block_scene(n, 43, 37, n))
+    _train_compare(dev, _block_scene(n, 43, 37, n + 1, needles=True))
+
+
+@pytest.mark.parametrize("kind", ["round", "needles", "opaque"])
+def test_raster_block_monolithic(dev, kind):
+    """The same where tiles are rasterised in one piece (400 tiles or more)."""
+    _train_compare(dev, _block_scene(900, 330, 321, 7, needles=kind == "needles", opaque=kind == "opaque"))
