@@ -635,11 +635,17 @@ __global__ __launch_bounds__(1024) void k_lists_and_items(int nsb, int S, const 
 }  // namespace
 
 void launch_depth_order(hipStream_t s, int N, uint32_t* dkey, uint32_t* dval, uint32_t* dkey2,
-                        uint32_t* dval2, int* radix_temp, const uint2* rect, uint2* rect_sorted,
-                        int* rcount, int* rtot, const SlotSum* ss, uint32_t** order_out) {
+                        uint32_t* dval2, int* radix_temp, int* rank, const uint2* rect,
+                        uint2* rect_sorted, int* rcount, int* rtot, const SlotSum* ss,
+                        uint32_t** order_out) {
     // the sort's last pass gathers the rectangles into depth order and
     // counts their super-tiles
     const RectGather rg{rect, rect_sorted, rcount};
+    if (N > 0 && N <= RANK_MAX) {
+        launch_rank_order(s, dkey, dval, N, rank, dval2, rtot, rg, *ss);
+        *order_out = dval2;
+        return;
+    }
     // culled gaussians (key 0xFFFFFFFF) go behind the visible ones in the
     // first pass and the later passes sort only the visible ones
     const bool flip = launch_radix_sort(s, dkey, dval, dkey2, dval2, N, 32, radix_temp, &rg, ss,

@@ -90,7 +90,7 @@ struct Ctx {
 
     // per gaussian
     Buf rec, radii, tiles_hit, rect, gacc;
-    Buf dkey, dval, dkey2, dval2, rect_sorted, hits, dtemp, stemp;
+    Buf dkey, dval, dkey2, dval2, rect_sorted, hits, dtemp, drank, stemp;
     // per tile
     Buf tcount, tscan, tile_bins, tile_K, tile_item0, l_chunked, tile_done, live_end;
     // per super-tile, per super-tile reference, per pair block
@@ -192,7 +192,7 @@ T* P(Buf& b) { return reinterpret_cast<T*>(b.p); }
 void free_all(Ctx* c) {
     Buf* bufs[] = {&c->rec, &c->radii, &c->tiles_hit, &c->rect, &c->rect_sorted,
                    &c->gacc, &c->dkey, &c->dval, &c->dkey2, &c->dval2, &c->hits,
-                   &c->dtemp, &c->stemp, &c->tcount, &c->tscan, &c->tile_done, &c->live_end, &c->tile_bins, &c->tile_K,
+                   &c->dtemp, &c->drank, &c->stemp, &c->tcount, &c->tscan, &c->tile_done, &c->live_end, &c->tile_bins, &c->tile_K,
                    &c->tile_item0, &c->l_chunked, &c->st_r0, &c->st_r1, &c->sstart,
                    &c->rkey, &c->rval, &c->rkey2, &c->rval2, &c->rtemp, &c->seg, &c->phist,
                    &c->tval, &c->bmask,
@@ -415,7 +415,8 @@ int forward(Ctx* c, const MsplatRenderArgs* a, bool training, float* dst_img = n
     ENSURE(c->dval2, Nn * 4);
     ENSURE(c->hits, Nn * 4);
     ENSURE(c->dtemp, (size_t)radix_temp_ints(N) * 4);
-    ENSURE(c->stemp, ((size_t)scan_block_count(N) + 8) * 4);
+    ENSURE(c->drank, (size_t)std::min(N, RANK_MAX) * 4);
+    ENSURE(c->stemp, (std::max<size_t>(scan_block_count(N), RANK_MAX / SCAN_BLOCK) + 8) * 4);
     ENSURE(c->tcount, (size_t)T * 4);
     ENSURE(c->tscan, (size_t)tile_scan_ints(T) * 4);
     const int nst = super_tiles(p.tbx, p.tby);
@@ -460,7 +461,7 @@ int forward(Ctx* c, const MsplatRenderArgs* a, bool training, float* dst_img = n
     const SlotSum totals{P<unsigned long long>(c->isect_d), c->isect_hd};
     launch_depth_order(c->stream, N, P<uint32_t>(c->dkey), P<uint32_t>(c->dval),
                        P<uint32_t>(c->dkey2), P<uint32_t>(c->dval2), P<int>(c->dtemp),
-                       P<uint2>(c->rect), P<uint2>(c->rect_sorted), P<int>(c->hits),
+                       P<int>(c->drank), P<uint2>(c->rect), P<uint2>(c->rect_sorted), P<int>(c->hits),
                        P<int>(c->stemp), &totals, &order);
     uint64_t word = 0;
     HIP_TRY(wait_totals(c, N, &word));

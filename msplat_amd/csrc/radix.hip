@@ -27,6 +27,8 @@
 #include "common.hpp"
 #include "kernels.hpp"
 
+#include <algorithm>
+
 namespace msp {
 
 namespace {
@@ -163,6 +165,97 @@ __global__ __launch_bounds__(256) void k_block_scan(const int* __restrict__ in,
     }
 }
 
+// The SlotSum job, by the first wave of one workgroup: lane k reads slot k's
+// pair, the wave sums them and lane 0 publishes the totals word.
+__device__ __forceinline__ void slot_sum(const SlotSum& ss) {
+    unsigned long long ti = 0, tr = 0;
+    for (int k = threadIdx.x; k < ISECT_SLOTS; k += 64) {
+        ti += __hip_atomic_load(ss.slots + (size_t)k * ISECT_STRIDE, __ATOMIC_RELAXED,
+                                __HIP_MEMORY_SCOPE_AGENT);
+        tr += __hip_atomic_load(ss.slots + (size_t)k * ISECT_STRIDE + 1, __ATOMIC_RELAXED,
+                                __HIP_MEMORY_SCOPE_AGENT);
+    }
+    for (int off = 32; off >= 1; off >>= 1) {
+        ti += __shfl_xor(ti, off, 64);
+        tr += __shfl_xor(tr, off, 64);
+    }
+    if (threadIdx.x == 0)
+        __hip_atomic_store(ss.out, totals_word(ti, tr), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Super-tiles of a rectangle as the projection packs it, 0 if it is empty.
+__device__ __forceinline__ int rect_span(uint2 r) {
+    const int x0 = (int)(r.x & 0xFFFFu), y0 = (int)(r.x >> 16);
+    const int x1 = (int)(r.y & 0xFFFFu), y1 = (int)(r.y >> 16);
+    return (x1 > x0 && y1 > y0) ? super_span(x0, y0, x1, y1) : 0;
+}
+
+// Ranks of up to RANK_MAX keys by comparing every key with every other:
+// workgroup (x, y) adds to rank[i], for its 256 keys i, the keys of its slice
+// of the others that come before (smaller, or equal with a smaller index, so
+// the order is a stable sort's).  The other keys are the same for the whole
+// workgroup: they come by scalar loads, and a comparison is two vector
+// instructions.  rank arrives zeroed (rank_scatter clears it again).  Also
+// clears the scan's block totals and does the SlotSum job.
+// Few keys leave a radix sort's passes bound by launches, not by work: 12
+// launches of 4-6 us for the depth order of 10k gaussians, 66 us, against two
+// here, 11 us.  The comparisons grow with the square of n.
+constexpr int RK_T = 256;
+__global__ __launch_bounds__(RK_T) void k_rank(const uint32_t* __restrict__ key, int n, int slice,
+                                               int* __restrict__ rank, int* __restrict__ tot,
+                                               SlotSum ss) {
+    if (blockIdx.x == 0 && blockIdx.y == 0) {
+        if (ss.out && threadIdx.x < 64) slot_sum(ss);
+        if ((int)threadIdx.x < RANK_MAX / SB) tot[threadIdx.x] = 0;
+    }
+    const int i0 = blockIdx.x * RK_T, i = i0 + threadIdx.x;
+    const int j0 = blockIdx.y * slice, j1 = min(j0 + slice, n);
+    const uint32_t k = i < n ? key[i] : 0u;
+    int c = 0;
+    // the slice's keys before this workgroup's, among them, and after them
+    const int a = min(max(i0, j0), j1), b = min(max(i0 + RK_T, j0), j1);
+    int j = j0;
+    for (; j + 16 <= a; j += 16)
+#pragma unroll
+        for (int u = 0; u < 16; ++u) c += key[j + u] <= k ? 1 : 0;
+    for (; j < a; ++j) c += key[j] <= k ? 1 : 0;
+    for (; j < b; ++j) {
+        const uint32_t o = key[j];
+        c += o < k || (o == k && j < i) ? 1 : 0;
+    }
+    for (; j + 16 <= j1; j += 16)
+#pragma unroll
+        for (int u = 0; u < 16; ++u) c += key[j + u] < k ? 1 : 0;
+    for (; j < j1; ++j) c += key[j] < k ? 1 : 0;
+    if (i < n && c) atomicAdd(&rank[i], c);
+}
+
+// The ranked values in order, with their rectangles and super-tile counts
+// (empty ones for the culled key 0xFFFFFFFF) and the counts' 1024-block totals.
+__global__ __launch_bounds__(RK_T) void k_rank_scatter(const uint32_t* __restrict__ key,
+                                                       const uint32_t* __restrict__ val, int n,
+                                                       int* __restrict__ rank,
+                                                       uint32_t* __restrict__ vout,
+                                                       int* __restrict__ tot, RectGather rg) {
+    __shared__ int s_tot[RANK_MAX / SB];
+    const int i = blockIdx.x * RK_T + threadIdx.x;
+    if ((int)threadIdx.x < RANK_MAX / SB) s_tot[threadIdx.x] = 0;
+    __syncthreads();
+    if (i < n) {
+        const int r = rank[i];
+        rank[i] = 0;
+        const uint2 rc = key[i] != 0xFFFFFFFFu ? rg.rect[i] : make_uint2(0u, 0u);
+        const int c = rect_span(rc);
+        vout[r] = val[i];
+        rg.rs[r] = rc;
+        rg.cnt[r] = c;
+        if (c) atomicAdd(&s_tot[r / SB], c);
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < RANK_MAX / SB && s_tot[threadIdx.x])
+        atomicAdd(&tot[threadIdx.x], s_tot[threadIdx.x]);
+}
+
 // Per-block digit counts.  D: digit slots (256, or 512 for a 9-bit or
 // culling pass).  LDS atomics on one address from many lanes of a wave are
 // serialised, so lanes that share a digit are counted with one atomic where
@@ -176,22 +269,7 @@ __global__ __launch_bounds__(RT) void k_radix_hist(const uint32_t* __restrict__ 
                                                    int* __restrict__ hist, int* __restrict__ dtot,
                                                    SlotSum ss) {
     __shared__ int h[D];
-    if (ss.out && blockIdx.x == 0 && threadIdx.x < 64) {
-        // lane k reads slot k's pair; the wave sums them
-        unsigned long long ti = 0, tr = 0;
-        for (int k = threadIdx.x; k < ISECT_SLOTS; k += 64) {
-            ti += __hip_atomic_load(ss.slots + (size_t)k * ISECT_STRIDE, __ATOMIC_RELAXED,
-                                    __HIP_MEMORY_SCOPE_AGENT);
-            tr += __hip_atomic_load(ss.slots + (size_t)k * ISECT_STRIDE + 1, __ATOMIC_RELAXED,
-                                    __HIP_MEMORY_SCOPE_AGENT);
-        }
-        for (int off = 32; off >= 1; off >>= 1) {
-            ti += __shfl_xor(ti, off, 64);
-            tr += __shfl_xor(tr, off, 64);
-        }
-        if (threadIdx.x == 0)
-            __hip_atomic_store(ss.out, totals_word(ti, tr), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
+    if (ss.out && blockIdx.x == 0 && threadIdx.x < 64) slot_sum(ss);
     const int64_t ne = pass_n(n, n_dev);
     const int nbe = (int)((ne + RB - 1) / RB);
     if ((int)blockIdx.x >= nbe) return;   // beyond the keys (the offsets scan only the blocks that hold some)
@@ -437,9 +515,7 @@ __global__ __launch_bounds__(RT) void k_radix_scatter(const uint32_t* __restrict
             const int p = tid + u * RT;
             const uint2 r = make_uint2(s_key[p], s_val[p]);
             rg.rs[opos[u]] = r;
-            const int x0 = (int)(r.x & 0xFFFFu), y0 = (int)(r.x >> 16);
-            const int x1 = (int)(r.y & 0xFFFFu), y1 = (int)(r.y >> 16);
-            rg.cnt[opos[u]] = (x1 > x0 && y1 > y0) ? super_span(x0, y0, x1, y1) : 0;
+            rg.cnt[opos[u]] = rect_span(r);
         }
     }
 }
@@ -484,6 +560,17 @@ void launch_scan_i32(hipStream_t s, const int* in, int* out, int64_t n, int* tot
 void launch_exclusive_scan_i32(hipStream_t s, const int* in, int* out, int64_t n, int* tot,
                                const uint32_t* gather, int* gathered) {
     launch_scan<false>(s, in, out, n, tot, gather, gathered);
+}
+
+void launch_rank_order(hipStream_t s, const uint32_t* key, const uint32_t* val, int n, int* rank,
+                       uint32_t* vout, int* tot, const RectGather& rg, const SlotSum& ss) {
+    const int nb = (n + RK_T - 1) / RK_T;
+    // about 2048 workgroups, with slices of 64 keys at least
+    const int slices = std::max(1, std::min((n + 63) / 64, (2048 + nb - 1) / nb));
+    const int slice = ((n + slices - 1) / slices + 15) & ~15;
+    hipLaunchKernelGGL(k_rank, dim3(nb, (n + slice - 1) / slice), dim3(RK_T), 0, s, key, n, slice, rank,
+                       tot, ss);
+    hipLaunchKernelGGL(k_rank_scatter, dim3(nb), dim3(RK_T), 0, s, key, val, n, rank, vout, tot, rg);
 }
 
 int64_t radix_temp_ints(int64_t n) {

@@ -473,3 +473,19 @@ def test_raster_block_edges(dev, n):
 def test_raster_block_monolithic(dev, kind):
     """The same where tiles are rasterised in one piece (400 tiles or more)."""
     _train_compare(dev, _block_scene(900, 330, 321, 7, needles=kind == "needles", opaque=kind == "opaque"))
+
+
+# one workgroup of ranks, several, the last ranked count and the first sorted one
+@pytest.mark.parametrize("n", [1, 2, 255, 256, 257, 1025, 24575, 24576, 24577])
+def test_depth_order_ties_and_culled(dev, n):
+    """Depth order of few gaussians: a handful of depths shared by all, some
+    of them behind the camera; ties keep index order."""
+    rng = np.random.default_rng(n)
+    sc = small_scene(n=n, width=100, height=60, seed_off=120)
+    cam = sc.cameras[0]
+    c2w = np.asarray(cam.cam_to_world, np.float64)
+    z = rng.choice([-1.0, 2.0, 2.0, 2.5, 3.0, 4.0], n)
+    z[0] = 2.0
+    local = np.stack([rng.uniform(-0.6, 0.6, n) * abs(z), rng.uniform(-0.4, 0.4, n) * abs(z), -z], 1)
+    sc.means = (local @ c2w[:3, :3].T + c2w[:3, 3]).astype(np.float32)
+    _render_and_compare(dev, sc)
