@@ -3,7 +3,7 @@
 // their super-tile references by super-tile, and by the nearest-neighbour
 // search to order points by cell.
 //
-// Sort: digits of up to 8 bits (9 for a sort of at most 9 bits, done in one
+// Sort (more than FUSE_BLOCKS blocks): digits of up to 8 bits (9 for a sort of at most 9 bits, done in one
 // pass), reduce-then-scan per pass over 2048-key blocks (512 threads x 4
 // keys):
 //   1. per-block digit histograms in LDS -> hist[digit][block], and the
@@ -41,6 +41,7 @@ constexpr int WK = RK * 64;        // keys per wave (RK rounds of 64)
 constexpr int SB = SCAN_BLOCK;     // elements per scan block
 constexpr int MAX_PASSES = 4;      // 32-bit keys in 8-bit digits
 constexpr int DMAX = 512;          // digit slots of the widest pass (9 bits, or 8 + the culled digit)
+constexpr int FUSE_BLOCKS = 64;    // most key blocks of a sort with one kernel a pass
 constexpr int DCOPIES = 16;        // copies of the digit totals (block b adds to copy b % 16)
 
 // Digit of key k in a pass: bits [shift, shift + width) (mask), or mask + 1
@@ -318,6 +319,53 @@ __global__ __launch_bounds__(RT) void k_radix_hist(const uint32_t* __restrict__ 
     }
 }
 
+// Sorts of at most FUSE_BLOCKS key blocks are launch bound (a kernel here
+// takes 4-6 us whatever it does), so they run one kernel a pass: the scatter
+// adds up the histograms of all blocks itself, and counts, while it writes
+// them out, the digits its keys have in the next pass at the blocks they land
+// in.  Histograms are block-major, D digits a row.  k_fused_first counts the
+// first pass's digits and clears the later passes' rows.  A 641x421 render with
+// three kernels a pass / one: 121 / 107 us for 25k gaussians, 137 / 130 for
+// 70k, 151 / 144 for 120k, 167 / 164 for 180k, 180 / 188 for 250k (adding up
+// every block's histogram grows with the square of the blocks): the line lies
+// at 64 blocks, 131072 keys.
+struct FusedPass {
+    const int* hist;     // this pass's counts
+    int* next;           // the next pass's, or null
+    int next_shift;
+    uint32_t next_mask;
+    int next_agg;        // rounds of equal counts to add up in the wave first
+    int* nvis;           // culling first pass: gets the number of visible keys
+    int* edge0;          // single-pass sort: output range of each digit, or null
+    int* edge1;
+};
+template <int D>
+__global__ __launch_bounds__(RT) void k_fused_first(const uint32_t* __restrict__ keys, int n, int shift,
+                                                    uint32_t mask, int cull, int* __restrict__ hist,
+                                                    int* __restrict__ later, int n_later, int later_row,
+                                                    int nb, SlotSum ss) {
+    __shared__ int h[D];
+    if (ss.out && blockIdx.x == 0 && threadIdx.x < 64) slot_sum(ss);
+    const int b = blockIdx.x, tid = threadIdx.x;
+    for (int p = 0; p < n_later; ++p)
+        for (int d = tid; d < later_row; d += RT) later[((size_t)p * nb + b) * later_row + d] = 0;
+    for (int d = tid; d < D; d += RT) h[d] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < RK; ++k) {
+        const int i = b * RB + k * RT + tid;
+        const bool ok = i < n;
+        const int d = ok ? digit_of(keys[i], shift, mask, cull != 0) : 0;
+        // the culled keys' digit, which many lanes share, by one atomic a wave
+        const bool cu = cull && ok && d == (int)mask + 1;
+        const uint64_t cm = wave_ballot(cu);
+        if (cm && (tid & 63) == (int)__builtin_ctzll(cm)) atomicAdd(&h[mask + 1], __popcll(cm));
+        if (ok && !cu) atomicAdd(&h[d], 1);
+    }
+    __syncthreads();
+    for (int d = tid; d < D; d += RT) hist[(size_t)b * D + d] = h[d];
+}
+
 // Exclusive scan of one value per thread over the NT threads of a block.
 template <int NT>
 __device__ __forceinline__ int block_exclusive_scan(int v, int* sh) {
@@ -385,7 +433,8 @@ __global__ __launch_bounds__(1024) void k_radix_offsets(int* __restrict__ hist, 
 // With RG (the depth order's last pass) the rectangles of the values go to
 // the same positions with their super-tile counts, and the positions past
 // the pass's keys (the culled tail) get empty ones.
-template <bool RG, int D>
+// FUSED: the offsets come from f.hist and the next pass is counted (FusedPass).
+template <bool RG, int D, bool FUSED>
 __global__ __launch_bounds__(RT) void k_radix_scatter(const uint32_t* __restrict__ kin,
                                                       const uint32_t* __restrict__ vin,
                                                       uint32_t* __restrict__ kout,
@@ -393,10 +442,10 @@ __global__ __launch_bounds__(RT) void k_radix_scatter(const uint32_t* __restrict
                                                       const int* __restrict__ n_dev, int shift,
                                                       uint32_t mask, int cull, int dbits,
                                                       int nblocks, const int* __restrict__ offs,
-                                                      int* __restrict__ dtot, RectGather rg) {
+                                                      int* __restrict__ dtot, RectGather rg, FusedPass f) {
     // The pass's digit totals were last read by the offsets kernel: block 0
     // clears them for the next sort that uses this scratch.
-    if (blockIdx.x == 0)
+    if (!FUSED && blockIdx.x == 0)
         for (int i = threadIdx.x; i < DCOPIES * D; i += RT) dtot[i] = 0;
     const int64_t ne = pass_n(n, n_dev);
     const int64_t bbase = (int64_t)blockIdx.x * RB;
@@ -425,7 +474,43 @@ __global__ __launch_bounds__(RT) void k_radix_scatter(const uint32_t* __restrict
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     // this block's scatter offset of digit tid, loaded now so that its latency
     // overlaps the key loads and the ranking
-    const int my_gofs = tid < nd ? offs[(size_t)tid * nblocks + rb] : 0;
+    int my_gofs = !FUSED && tid < nd ? offs[(size_t)tid * nblocks + rb] : 0;
+    if constexpr (FUSED) {
+        // digit tid % D: the keys in all blocks and in those before this one
+        // (two threads a digit where there are enough)
+        __shared__ int s_half[2][D];
+        constexpr int STEP = RT / D;
+        const int d = tid % D;
+        int total = 0, before = 0;
+#pragma unroll 16
+        for (int b = tid / D; b < nbe; b += STEP) {
+            const int c = f.hist[(size_t)b * D + d];
+            total += c;
+            before += b < rb ? c : 0;
+        }
+        if (STEP == 2) {
+            if (tid >= D) {
+                s_half[0][d] = total;
+                s_half[1][d] = before;
+            }
+            __syncthreads();
+            if (tid < D) {
+                total += s_half[0][d];
+                before += s_half[1][d];
+            } else {
+                total = 0;
+            }
+        }
+        const int start = block_exclusive_scan<RT>(total, scan_sh);
+        my_gofs = start + before;
+        if (rb == 0 && tid < nd) {
+            if (f.nvis && cl && tid == nd - 1) *f.nvis = start;
+            if (f.edge0 && total > 0) {
+                f.edge0[tid] = start;
+                f.edge1[tid] = start + total;
+            }
+        }
+    }
     for (int i = tid; i < RW * D; i += RT) (&wcnt[0][0])[i] = 0;
     __syncthreads();
     const int64_t wbase = kbase + (int64_t)w * WK;
@@ -497,6 +582,23 @@ __global__ __launch_bounds__(RT) void k_radix_scatter(const uint32_t* __restrict
         kout[pos] = k;
         vout[pos] = s_val[p];
         opos[u] = pos;
+        if constexpr (FUSED) {
+            if (f.next) {
+                int slot = (int)(pos / RB) * 256 + (int)((k >> f.next_shift) & f.next_mask);
+                bool left = !(cl && k == 0xFFFFFFFFu);
+                // the top byte of depth keys: lanes with the same count add once
+                for (int r = 0; r < f.next_agg; ++r) {
+                    const uint64_t act = wave_ballot(left);
+                    if (act == 0) break;
+                    const int first = (int)__builtin_ctzll(act);
+                    const bool mine = left && slot == __builtin_amdgcn_readlane(slot, first);
+                    const uint64_t same = wave_ballot(mine);
+                    if (lane == first) atomicAdd(&f.next[slot], __popcll(same));
+                    if (mine) left = false;
+                }
+                if (left) atomicAdd(&f.next[slot], 1);
+            }
+        }
     }
     if (RG) {
         // the rectangles take the keys' LDS places and go to the same
@@ -575,7 +677,8 @@ void launch_rank_order(hipStream_t s, const uint32_t* key, const uint32_t* val, 
 
 int64_t radix_temp_ints(int64_t n) {
     const int64_t nb = (n + RB - 1) / RB;
-    return DCOPIES * DMAX * MAX_PASSES + (int64_t)DMAX * nb + 16;
+    const int64_t row = nb <= FUSE_BLOCKS ? DMAX + 256 * (MAX_PASSES - 1) : DMAX;
+    return DCOPIES * DMAX * MAX_PASSES + row * nb + 16;
 }
 
 namespace {
@@ -592,12 +695,32 @@ void launch_pass(hipStream_t s, const uint32_t* ki, const uint32_t* vi, uint32_t
     hipLaunchKernelGGL(k_radix_offsets<D>, dim3(nd), dim3(1024), 0, s, hist, nb, n, n_dev,
                        (const int*)dt, edge0, edge1, cull ? nvis : nullptr, nd - 1);
     if (rg)
-        hipLaunchKernelGGL((k_radix_scatter<true, D>), dim3(nb), dim3(RT), 0, s, ki, vi, ko, vo, n, n_dev,
-                           shift, mask, cull ? 1 : 0, dbits, nb, (const int*)hist, dt, *rg);
+        hipLaunchKernelGGL((k_radix_scatter<true, D, false>), dim3(nb), dim3(RT), 0, s, ki, vi, ko, vo, n,
+                           n_dev, shift, mask, cull ? 1 : 0, dbits, nb, (const int*)hist, dt, *rg,
+                           FusedPass{});
     else
-        hipLaunchKernelGGL((k_radix_scatter<false, D>), dim3(nb), dim3(RT), 0, s, ki, vi, ko, vo, n,
+        hipLaunchKernelGGL((k_radix_scatter<false, D, false>), dim3(nb), dim3(RT), 0, s, ki, vi, ko, vo, n,
                            n_dev, shift, mask, cull ? 1 : 0, dbits, nb, (const int*)hist, dt,
-                           RectGather{});
+                           RectGather{}, FusedPass{});
+}
+
+// One pass of a fused sort (the first pass's counts, then the scatter).
+template <int D>
+void launch_fused_pass(hipStream_t s, const uint32_t* ki, const uint32_t* vi, uint32_t* ko, uint32_t* vo,
+                       int64_t n, const int* n_dev, int shift, uint32_t mask, bool cull, int dbits, int nb,
+                       bool first, int* hist, int* later, int n_later, const SlotSum& side, const FusedPass& f,
+                       const RectGather* rg) {
+    if (first)
+        hipLaunchKernelGGL(k_fused_first<D>, dim3(nb), dim3(RT), 0, s, ki, (int)n, shift, mask, cull ? 1 : 0,
+                           hist, later, n_later, 256, nb, side);
+    if (rg)
+        hipLaunchKernelGGL((k_radix_scatter<true, D, true>), dim3(nb), dim3(RT), 0, s, ki, vi, ko, vo, n,
+                           n_dev, shift, mask, cull ? 1 : 0, dbits, nb, (const int*)nullptr, (int*)nullptr, *rg,
+                           f);
+    else
+        hipLaunchKernelGGL((k_radix_scatter<false, D, true>), dim3(nb), dim3(RT), 0, s, ki, vi, ko, vo, n,
+                           n_dev, shift, mask, cull ? 1 : 0, dbits, nb, (const int*)nullptr, (int*)nullptr,
+                           RectGather{}, f);
 }
 
 }  // namespace
@@ -627,6 +750,8 @@ bool launch_radix_sort(hipStream_t s, uint32_t* k0, uint32_t* v0, uint32_t* k1, 
     int* dtot = temp;
     int* hist = temp + DCOPIES * DMAX * MAX_PASSES;
     int* nvis = hist + (size_t)DMAX * nb;
+    // (a fused sort's rows take DMAX + 3 x 256 ints a block, the count follows)
+    int* fused_nvis = hist + (size_t)(DMAX + 256 * (MAX_PASSES - 1)) * nb;
     // the digit totals arrive zeroed: fresh scratch is, and each pass's
     // scatter clears its own
     bool flip = false;
@@ -648,6 +773,27 @@ bool launch_radix_sort(hipStream_t s, uint32_t* k0, uint32_t* v0, uint32_t* k1, 
         // the top byte of depth keys: a wave's keys mostly share a digit
         const bool agg = cull && shift == 24;
         const RectGather* prg = rg && pass == passes - 1 ? rg : nullptr;
+        if (nb <= FUSE_BLOCKS) {
+            // rows of the first pass (up to DMAX digits), then 256 digits a row
+            int* rows0 = hist;
+            int* later = hist + (size_t)DMAX * nb;
+            auto rows = [&](int p) { return p == 0 ? rows0 : later + (size_t)(p - 1) * nb * 256; };
+            const int nshift = shift + width;
+            const int nwidth = pass + 1 < passes ? (bits - nshift + (passes - pass - 1) - 1) / (passes - pass - 1) : 0;
+            const FusedPass f{rows(pass), pass + 1 < passes ? rows(pass + 1) : nullptr, nshift,
+                              (1u << nwidth) - 1u, cull && nshift == 24 ? 6 : 0, fused_nvis, passes == 1 ? edge0 : nullptr,
+                              passes == 1 ? edge1 : nullptr};
+            const int* nd_dev = cull && pass > 0 ? fused_nvis : nullptr;
+            if (nd > 256)
+                launch_fused_pass<DMAX>(s, ki, vi, ko, vo, n, nd_dev, shift, mask, pcull, dbits, nb, pass == 0,
+                                        rows0, later, passes - 1, side, f, prg);
+            else
+                launch_fused_pass<256>(s, ki, vi, ko, vo, n, nd_dev, shift, mask, pcull, dbits, nb, pass == 0,
+                                       rows0, later, passes - 1, side, f, prg);
+            flip = !flip;
+            shift += width;
+            continue;
+        }
         int* e0 = passes == 1 ? edge0 : nullptr;
         int* e1 = passes == 1 ? edge1 : nullptr;
         if (nd > 256)

@@ -489,3 +489,19 @@ def test_depth_order_ties_and_culled(dev, n):
     local = np.stack([rng.uniform(-0.6, 0.6, n) * abs(z), rng.uniform(-0.4, 0.4, n) * abs(z), -z], 1)
     sc.means = (local @ c2w[:3, :3].T + c2w[:3, 3]).astype(np.float32)
     _render_and_compare(dev, sc)
+
+
+# one key block, the last count sorted with one kernel a pass, the next one
+@pytest.mark.parametrize("n", [26000, 131072, 131073])
+def test_depth_order_fused_passes(dev, n):
+    """Radix passes that count the next pass's digits: many equal depths (one
+    top byte, ties in index order), culled gaussians, several super-tiles."""
+    rng = np.random.default_rng(n)
+    sc = small_scene(n=n, width=300, height=270, seed_off=121, degree=0)
+    cam = sc.cameras[0]
+    c2w = np.asarray(cam.cam_to_world, np.float64)
+    z = np.where(rng.random(n) < 0.5, rng.choice([-1.0, 2.0, 2.5, 3.9], n), rng.uniform(2.0, 40.0, n))
+    local = np.stack([rng.uniform(-0.7, 0.7, n) * abs(z), rng.uniform(-0.6, 0.6, n) * abs(z), -z], 1)
+    sc.means = (local @ c2w[:3, :3].T + c2w[:3, 3]).astype(np.float32)
+    sc.scales -= 1.0
+    _render_and_compare(dev, sc)
