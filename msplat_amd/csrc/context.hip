@@ -123,7 +123,7 @@ struct Ctx {
     int* radii_dst = nullptr;   // the caller's radii_out of the current train step, or null
     int* count_h = nullptr;
     // densify scratch
-    Buf d_split, d_dup, d_sp, d_dp, d_keep, d_kp, d_tot, d_scratch, d_rnd, d_src;
+    Buf d_flags, d_tot, d_scratch, d_rnd, d_src;
 
     const uint32_t* sorted_ids = nullptr;   // tile-sorted gaussian ids (tval)
     Meta meta{};
@@ -200,8 +200,7 @@ void free_all(Ctx* c) {
                    &c->c_idx, &c->c_pT, &c->c_aC, &c->final_T, &c->final_idx, &c->out_img,
                    &c->v_rendered, &c->loss_part, &c->meta_d, &c->loss_d,
                    &c->count_d, &c->work_d, &c->isect_d, &c->eval_part, &c->eval_out, &c->knn_k, &c->knn_v, &c->knn_k2, &c->knn_v2,
-                   &c->knn_tmp, &c->knn_pts, &c->knn_box, &c->knn_frame, &c->d_split, &c->d_dup, &c->d_sp, &c->d_dp, &c->d_keep, &c->d_kp,
-                   &c->d_tot, &c->d_scratch, &c->d_rnd, &c->d_src};
+                   &c->knn_tmp, &c->knn_pts, &c->knn_box, &c->knn_frame, &c->d_flags, &c->d_tot, &c->d_scratch, &c->d_rnd, &c->d_src};
     for (Buf* b : bufs)
         if (b->p) { (void)hipFree(b->p); b->p = nullptr; b->bytes = 0; }
     if (c->meta_h) (void)hipHostFree(c->meta_h);
@@ -995,13 +994,9 @@ int msplat_hip_densify(const MsplatDensifyArgs* a, int32_t* new_count) {
     for (int g = 0; g < 6; ++g)
         if (!a->bufs[g] || !a->adam_exp_avg_buf[g] || !a->adam_exp_avg_sq_buf[g])
             if (!(g == 4 && a->fr_stride == 0)) return fail(MSPLAT_ERR_ARG, "null buffer %d", g);
-    ENSURE(c->d_split, (size_t)N * 4);
-    ENSURE(c->d_dup, (size_t)N * 4);
-    ENSURE(c->d_sp, (size_t)N * 4);
-    ENSURE(c->d_dp, (size_t)N * 4);
-    ENSURE(c->d_keep, (size_t)worst * 4);
-    ENSURE(c->d_kp, (size_t)worst * 4);
-    ENSURE(c->d_tot, (size_t)scan_block_count(worst) * 4 + 64);
+    ENSURE(c->d_flags, (size_t)N);
+    ENSURE(c->d_tot, (size_t)densify_total_ints(N) * 4);
+    ENSURE(c->d_src, (size_t)worst * 8);   // a gaussian leaves at most three rows
     ENSURE(c->count_d, 16);
     stage_begin(c);
     stage_mark(c, S_DENSIFY);
@@ -1023,10 +1018,8 @@ int msplat_hip_densify(const MsplatDensifyArgs* a, int32_t* new_count) {
     hp.check_huge = a->check_huge;
     hp.half_max_dim = a->half_max_dim;
     hp.fr = a->fr_stride;
-    launch_densify(c->stream, hp, a->xys_grad_norm, a->vis_counts, a->max_2d_size, a->bufs,
-                   a->adam_exp_avg_buf, a->adam_exp_avg_sq_buf, rnd, P<int>(c->d_split),
-                   P<int>(c->d_dup), P<int>(c->d_sp), P<int>(c->d_dp), P<int>(c->d_keep),
-                   P<int>(c->d_kp), P<int>(c->d_tot), P<int>(c->count_d));
+    launch_densify(c->stream, hp, a->xys_grad_norm, a->vis_counts, a->max_2d_size, a->bufs[1], a->bufs[5],
+                   P<uint8_t>(c->d_flags), P<int>(c->d_tot), P<uint2>(c->d_src), P<int>(c->count_d));
     HIP_TRY(hipGetLastError());
     // rows after appending and rows kept size the compaction exactly
     HIP_TRY(hipMemcpyAsync(c->count_h, c->count_d.p, 8, hipMemcpyDeviceToHost, c->stream));
@@ -1035,11 +1028,9 @@ int msplat_hip_densify(const MsplatDensifyArgs* a, int32_t* new_count) {
     if (rows < 0 || rows > worst || kept < 0 || kept > rows)
         return fail(MSPLAT_ERR_HIP, "densify counts out of range: %d rows, %d kept (N = %d)", rows,
                     kept, N);
-    ENSURE(c->d_src, (size_t)std::max(kept, 1) * 4);
     ENSURE(c->d_scratch, (size_t)densify_workspace_floats(kept, a->fr_stride) * 4);
-    launch_densify_compact(c->stream, rows, kept, a->fr_stride, a->bufs, a->adam_exp_avg_buf,
-                           a->adam_exp_avg_sq_buf, P<int>(c->d_keep), P<int>(c->d_kp),
-                           P<int>(c->d_src), P<float>(c->d_scratch));
+    launch_densify_compact(c->stream, kept, a->fr_stride, a->bufs, a->adam_exp_avg_buf,
+                           a->adam_exp_avg_sq_buf, P<uint2>(c->d_src), rnd, P<float>(c->d_scratch));
     HIP_TRY(hipGetLastError());
     stage_mark(c, S_END);
     HIP_TRY(hipStreamSynchronize(c->stream));

@@ -112,8 +112,7 @@ void launch_project_fwd(hipStream_t s, const CamParams& p, const float* means,
                         uint32_t* dkey, uint32_t* dval, float* gacc,
                         unsigned long long* total_isect);
 
-// Scans and radix sort (radix.hip).  With `gather` the scanned values are
-// in[gather[i]], also stored to gathered[i] (n ints).
+// Block totals and radix sort (radix.hip).
 constexpr int SCAN_BLOCK = 1024;   // elements per scan block
 int64_t scan_block_count(int64_t n);
 // Above this many 1024-element blocks a scan runs its block totals through a
@@ -123,9 +122,6 @@ constexpr int SCAN_DIRECT_BLOCKS = 2048;
 // turned into exclusive block offsets when there are more than
 // SCAN_DIRECT_BLOCKS blocks (the consumer then reads tot[b] directly).
 void launch_block_totals(hipStream_t s, const int* in, int64_t n, int* tot);
-void launch_scan_i32(hipStream_t s, const int* in, int* out, int64_t n, int* block_tot);
-void launch_exclusive_scan_i32(hipStream_t s, const int* in, int* out, int64_t n, int* block_tot,
-                               const uint32_t* gather = nullptr, int* gathered = nullptr);
 int64_t radix_temp_ints(int64_t n);
 // Optional side job of a sort's first kernel, for the depth order: its
 // workgroup 0 sums the projection's ISECT_SLOTS counter pairs and writes the
@@ -340,18 +336,19 @@ struct DensifyHP {
 };
 void launch_randn(hipStream_t s, float* dst, int64_t n, uint64_t seed);
 void launch_clamp_max(hipStream_t s, float* p, int64_t n, float hi);
-// Classify, split / duplicate append, cull flags and keep scan; writes
-// counts_out[0] = rows after appending, counts_out[1] = rows kept.
+// Decides which rows the N gaussians leave (flags: a byte each; tot:
+// densify_total_ints(N)) and records the source of each kept row in src (at
+// most 3 N); counts_out[0] = rows after the reference's appending,
+// counts_out[1] = rows kept.
+int64_t densify_total_ints(int64_t N);
 void launch_densify(hipStream_t s, const DensifyHP& hp, const float* gnorm, const float* vis,
-                    const float* max2d, float* const bufs[6], float* const m[6],
-                    float* const v[6], const float* rnd, int* split, int* dup, int* sp,
-                    int* dp, int* keep, int* kp, int* block_tot, int* counts_out);
-// Stable compaction of the cnt kept rows (of `rows` rows) of all 18 buffers
-// through a workspace of densify_workspace_floats(cnt, fr) floats.
+                    const float* max2d, const float* scales, const float* opac, uint8_t* flags, int* tot,
+                    uint2* src, int* counts_out);
+// Forms the cnt kept rows of all 18 buffers, one set at a time, in a workspace
+// of densify_workspace_floats(cnt, fr) floats and copies them back.
 int64_t densify_workspace_floats(int cnt, int fr);
-void launch_densify_compact(hipStream_t s, int rows, int cnt, int fr, float* const bufs[6],
-                            float* const m[6], float* const v[6], const int* keep,
-                            const int* kp, int* src_of, float* ws);
+void launch_densify_compact(hipStream_t s, int cnt, int fr, float* const bufs[6], float* const m[6],
+                            float* const v[6], const uint2* src, const float* rnd, float* ws);
 
 // Evaluation images: RGBA8 display conversion and PSNR / L1 / SSIM.
 struct EvalWindow {

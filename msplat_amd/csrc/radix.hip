@@ -69,29 +69,16 @@ __device__ __forceinline__ int block_sum(int v, int* sh) {
 }
 __device__ __forceinline__ int block_sum_256(int v, int* sh) { return block_sum<256>(v, sh); }
 
-// Value i of a scan's input: in[i], or in[gather[i]].
-__device__ __forceinline__ int scan_in(const int* __restrict__ in,
-                                       const uint32_t* __restrict__ gather, int64_t i) {
-    return gather ? in[gather[i]] : in[i];
-}
-
-// Block totals of the scan input; with `gather` the input is in[gather[i]],
-// which is also written to gathered[i] for the later passes.
+// Totals of the 1024-element blocks of in.
 __global__ __launch_bounds__(256) void k_block_reduce(const int* __restrict__ in, int64_t n,
-                                                      int* __restrict__ tot,
-                                                      const uint32_t* __restrict__ gather,
-                                                      int* __restrict__ gathered) {
+                                                      int* __restrict__ tot) {
     __shared__ int sh[4];
     const int64_t base = (int64_t)blockIdx.x * SB;
     int v = 0;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         const int64_t i = base + k * 256 + threadIdx.x;
-        if (i < n) {
-            const int x = scan_in(in, gather, i);
-            if (gathered) gathered[i] = x;
-            v += x;
-        }
+        if (i < n) v += in[i];
     }
     const int t = block_sum_256(v, sh);
     if (threadIdx.x == 0) tot[blockIdx.x] = t;
@@ -119,51 +106,6 @@ __global__ __launch_bounds__(1024) void k_scan_totals(int* __restrict__ tot, int
         run += v;
     }
     if (threadIdx.x == 1023) tot[nb] = s[1023];
-}
-
-// Scan of each 1024-element block plus its offset; inclusive or exclusive.
-// With PREFIX the block sums the totals of the blocks before it itself (tot
-// holds plain block totals); otherwise tot holds the scanned offsets.
-template <bool INCLUSIVE, bool PREFIX>
-__global__ __launch_bounds__(256) void k_block_scan(const int* __restrict__ in,
-                                                    int* __restrict__ out, int64_t n,
-                                                    const int* __restrict__ tot,
-                                                    const uint32_t* __restrict__ gather) {
-    __shared__ int ts[256];
-    __shared__ int sh[4];
-    const int64_t base = (int64_t)blockIdx.x * SB;
-    const int t = threadIdx.x;
-    int boff = 0;
-    if (PREFIX) {
-        int acc = 0;
-        for (int b = t; b < (int)blockIdx.x; b += 256) acc += tot[b];
-        boff = block_sum_256(acc, sh);
-    } else {
-        boff = tot[blockIdx.x];
-    }
-    int v[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int64_t i = base + 4 * t + k;
-        v[k] = i < n ? scan_in(in, gather, i) : 0;
-    }
-    const int s4 = v[0] + v[1] + v[2] + v[3];
-    ts[t] = s4;
-    __syncthreads();
-    for (int off = 1; off < 256; off <<= 1) {
-        const int x = t >= off ? ts[t - off] : 0;
-        __syncthreads();
-        ts[t] += x;
-        __syncthreads();
-    }
-    int run = ts[t] - s4 + boff;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int64_t i = base + 4 * t + k;
-        if (INCLUSIVE) run += v[k];
-        if (i < n) out[i] = run;
-        if (!INCLUSIVE) run += v[k];
-    }
 }
 
 // The SlotSum job, by the first wave of one workgroup: lane k reads slot k's
@@ -628,40 +570,11 @@ inline unsigned blocks_for(int64_t n, int per) { return (unsigned)((n + per - 1)
 
 int64_t scan_block_count(int64_t n) { return (n + SB - 1) / SB; }
 
-template <bool INCLUSIVE>
-void launch_scan(hipStream_t s, const int* in, int* out, int64_t n, int* tot,
-                 const uint32_t* gather, int* gathered) {
-    if (n <= 0) return;
-    const int nb = (int)scan_block_count(n);
-    hipLaunchKernelGGL(k_block_reduce, dim3(nb), dim3(256), 0, s, in, n, tot, gather, gathered);
-    if (gather) {   // the block scans read the gathered copy
-        in = gathered;
-        gather = nullptr;
-    }
-    if (nb <= SCAN_DIRECT_BLOCKS) {
-        hipLaunchKernelGGL((k_block_scan<INCLUSIVE, true>), dim3(nb), dim3(256), 0, s, in, out, n,
-                           (const int*)tot, gather);
-    } else {
-        hipLaunchKernelGGL(k_scan_totals, dim3(1), dim3(1024), 0, s, tot, nb);
-        hipLaunchKernelGGL((k_block_scan<INCLUSIVE, false>), dim3(nb), dim3(256), 0, s, in, out, n,
-                           (const int*)tot, gather);
-    }
-}
-
 void launch_block_totals(hipStream_t s, const int* in, int64_t n, int* tot) {
     if (n <= 0) return;
     const int nb = (int)scan_block_count(n);
-    hipLaunchKernelGGL(k_block_reduce, dim3(nb), dim3(256), 0, s, in, n, tot, nullptr, nullptr);
+    hipLaunchKernelGGL(k_block_reduce, dim3(nb), dim3(256), 0, s, in, n, tot);
     if (nb > SCAN_DIRECT_BLOCKS) hipLaunchKernelGGL(k_scan_totals, dim3(1), dim3(1024), 0, s, tot, nb);
-}
-
-void launch_scan_i32(hipStream_t s, const int* in, int* out, int64_t n, int* tot) {
-    launch_scan<true>(s, in, out, n, tot, nullptr, nullptr);
-}
-
-void launch_exclusive_scan_i32(hipStream_t s, const int* in, int* out, int64_t n, int* tot,
-                               const uint32_t* gather, int* gathered) {
-    launch_scan<false>(s, in, out, n, tot, gather, gathered);
 }
 
 void launch_rank_order(hipStream_t s, const uint32_t* key, const uint32_t* val, int n, int* rank,

@@ -411,6 +411,52 @@ def test_densify_parity(dev, misaligned):
         assert_bits_equal(g.v[i][:nn_o].cpu().numpy(), vs[i][:nn_o], f"densified exp_avg_sq {i}")
 
 
+@pytest.mark.parametrize("n", [1, 1023, 1024, 1025, 2049])
+@pytest.mark.parametrize("screen", [0, 1])
+def test_densify_block_edges(dev, n, screen):
+    """Row numbering at the edges of its 1024-gaussian blocks, with gaussians
+    that are split, duplicated, both (by screen size alone) and culled in every
+    mixture, at SH degree 1: bit-equal to the oracle."""
+    torch = pytest.importorskip("torch")
+    sc = small_scene(n=n, seed_off=86)
+    st = synthetic.Stream(synthetic.BASE_SEED + 87 + n)
+    params = [np.ascontiguousarray(p.reshape(n, -1)[:, :9] if i == 4 else p)
+              for i, p in enumerate(sc.params())]
+    params[4] = params[4].reshape(n, 3, 3)
+    params[1] = (params[1] + 1.5 * (st.uniform(n) < 0.4)[:, None]).astype(np.float32)
+    g = dev.DeviceGaussians.from_arrays(params, 1, capacity=3 * n)
+    m0 = [(st.uniform(b.numel()).reshape(tuple(b.shape)) * 0.1).astype(np.float32) for b in g.bufs]
+    for i in range(6):
+        g.m[i].copy_(torch.from_numpy(m0[i]))
+        g.v[i].copy_(torch.from_numpy(m0[i] * 0.5))
+    vis = np.floor(st.uniform(n) * 4).astype(np.float32)
+    gnorm = (st.uniform(n) * 8e-6 * vis).astype(np.float32)
+    max2d = (st.uniform(n) * 0.2).astype(np.float32)
+    for dst, a in ((g.vis, vis), (g.gnorm, gnorm), (g.max2d, max2d)):
+        dst[:n].copy_(torch.from_numpy(a))
+    rnd = (st.uniform(6 * n) * 2 - 1).astype(np.float32)
+    kw = dict(grad_thresh=2e-4, size_thresh=0.05, screen_thresh=0.05, check_screen=screen, cull_alpha=0.4,
+              cull_scale=0.1, cull_screen=0.15, check_huge=1, half_max_dim=0.5 * 160)
+    bufs = [b.cpu().numpy().copy() for b in g.bufs]
+    ms = [a.copy() for a in m0]
+    vs = [(a * 0.5).astype(np.float32) for a in m0]
+    oa = orc.OrcDensifyArgs()
+    oa.N = n
+    oa.grad_thresh, oa.size_thresh, oa.screen_thresh, oa.check_screen = 2e-4, 0.05, 0.05, screen
+    oa.cull_alpha_thresh, oa.cull_scale_thresh, oa.cull_screen_size, oa.check_huge = 0.4, 0.1, 0.15, 1
+    oa.half_max_dim, oa.fr_stride = 0.5 * 160, 9
+    nn_o, split, dup, keep = orc.densify(oa, gnorm, vis, max2d, bufs, ms, vs, rnd)
+    if n > 1000:
+        assert split.sum() > 0 and dup.sum() > 0 and (keep == 0).sum() > split.sum()
+        assert (split.astype(bool) & dup.astype(bool)).any() == bool(screen)
+    nn_g = dev.densify(g, random_samples=torch.from_numpy(rnd).cuda(), **kw)
+    assert nn_g == nn_o, (nn_g, nn_o)
+    for i in range(6):
+        assert_bits_equal(g.bufs[i][:nn_o].cpu().numpy(), bufs[i][:nn_o], f"densified param {i}")
+        assert_bits_equal(g.m[i][:nn_o].cpu().numpy(), ms[i][:nn_o], f"densified exp_avg {i}")
+        assert_bits_equal(g.v[i][:nn_o].cpu().numpy(), vs[i][:nn_o], f"densified exp_avg_sq {i}")
+
+
 def test_randn_statistics(dev):
     torch = pytest.importorskip("torch")
     from msplat_amd import _abi
