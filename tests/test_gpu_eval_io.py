@@ -60,6 +60,19 @@ def test_image_metrics_match_oracle(mods, shape, ws, sigma):
         assert abs(got[k] - want[k]) <= 1e-6 * max(1.0, abs(want[k])), (k, got[k], want[k])
 
 
+@pytest.mark.parametrize("ws", [1, 3, 5, 7, 9, 11])
+def test_image_metrics_tile_edges(mods, ws):
+    """Every window size at images around its 64x16 tiles.  The sums are exact
+    to fp64 rounding, and psnr, l1 and ssim are rounded once more: 1e-6."""
+    torch, device, _ = mods
+    for shape in ((1, 1), (16, 64), (15, 63), (17, 65), (33, 130)):
+        a, b = _pair(*shape, seed=shape[1] + ws)
+        got = device.image_metrics(torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda(), ws, 1.5)
+        want = orc.image_metrics(a, b, ws, 1.5)
+        for k in ("psnr", "ssim", "l1"):
+            assert abs(got[k] - want[k]) <= 1e-6 * max(1.0, abs(want[k])), (shape, k, got[k], want[k])
+
+
 def test_image_metrics_identical_images(mods):
     torch, device, _ = mods
     a, _ = _pair(48, 80, 3)
