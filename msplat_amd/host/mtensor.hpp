@@ -103,16 +103,23 @@ public:
         MTensor t;
         t.shape_ = std::move(shape);
         t.dtype_ = dt;
-        size_t bytes = (size_t)t.numel() * dtype_size(dt);
+        if (t.nbytes() <= kMappedBytes) return mapped(std::move(t.shape_), dt);
         void* p = nullptr;
-        if (bytes <= kMappedBytes) {
-            check(msplat_hip_alloc_mapped(&p, bytes ? bytes : 16), "alloc mapped");
-            t.mem_ = std::shared_ptr<void>(p, [](void* q) { msplat_hip_free_mapped(q); });
-            t.mapped_ = true;
-        } else {
-            check(msplat_hip_alloc(&p, bytes), "alloc");
-            t.mem_ = std::shared_ptr<void>(p, [](void* q) { msplat_hip_free(q); });
-        }
+        check(msplat_hip_alloc(&p, t.nbytes()), "alloc");
+        t.mem_ = std::shared_ptr<void>(p, [](void* q) { msplat_hip_free(q); });
+        t.ptr_ = p;
+        return t;
+    }
+    // A mapped tensor of any size, for results that a kernel writes once and
+    // the host reads.
+    static MTensor mapped(std::vector<int64_t> shape, DType dt) {
+        MTensor t;
+        t.shape_ = std::move(shape);
+        t.dtype_ = dt;
+        void* p = nullptr;
+        check(msplat_hip_alloc_mapped(&p, t.nbytes() ? t.nbytes() : 16), "alloc mapped");
+        t.mem_ = std::shared_ptr<void>(p, [](void* q) { msplat_hip_free_mapped(q); });
+        t.mapped_ = true;
         t.ptr_ = p;
         return t;
     }

@@ -185,6 +185,26 @@ public:
         model->renderTo(cam, current_step, dst, w, h);
     }
 
+    // The same as display bytes in host memory (out NULL: size only).  The
+    // image and the bytes are kept for the next frame, for as long as frames
+    // stay at this size: allocating and freeing them took longer than the
+    // conversion, and each free waits for the GPU.  The conversion writes the
+    // bytes straight to mapped host memory.
+    void render_pose_rgba8(const float camToWorld[16], int ref, uint8_t* out, int& w, int& h) {
+        render_pose_to(camToWorld, ref, nullptr, w, h);
+        if (!out) return;
+        const int64_t n = (int64_t)w * h;
+        if (frame.numel() != 3 * n) {
+            frame.reset();
+            frame_rgba.reset();
+            frame = gpu_empty({3 * n}, DType::Float32);
+            frame_rgba = MTensor::mapped({n}, DType::Int32);   // 4 bytes per pixel
+        }
+        render_pose_to(camToWorld, ref, frame.data<float>(), w, h);
+        check(msplat_hip_image_to_rgba8(frame.data<float>(), n, frame_rgba.data<uint8_t>()), "rgba8");
+        frame_rgba.copy_to_host(out, (size_t)n * 4);
+    }
+
     // Trainer::render (msplat_api.mm:168-186): a training or held-out camera
     // at the current step's resolution; an empty tensor when out of range.
     MTensor render_camera(int i, bool use_test) {
@@ -222,6 +242,7 @@ private:
     std::vector<Camera> test_cameras;
     std::vector<MTensor> test_images;
     std::vector<std::map<int, MTensor>> gpu_images;
+    MTensor frame, frame_rgba;   // of the latest render_pose_rgba8
     std::vector<size_t> cam_indices;
     size_t cam_iter_pos = 0;
     std::mt19937 rng;
@@ -495,7 +516,8 @@ MsplatPixelBuffer msplat_trainer_render_pose(MsplatTrainer t, const float camToW
 }
 
 // Trainer::renderFromPoseToBuffer (msplat_api.mm:207-238): the RGBA8
-// conversion runs on the GPU and 4 bytes per pixel are copied.
+// conversion runs on the GPU and 4 bytes per pixel are copied; without a
+// buffer only the size is determined.
 void msplat_trainer_render_pose_to_buffer(MsplatTrainer t, const float camToWorld[16],
                                           int refCameraIndex, uint8_t* outRGBA, int* outWidth,
                                           int* outHeight) {
@@ -505,15 +527,10 @@ void msplat_trainer_render_pose_to_buffer(MsplatTrainer t, const float camToWorl
         return;
     }
     guarded_void([&]() {
-        msplat::MTensor img = T(t)->render_pose(camToWorld, refCameraIndex);
-        const int h = (int)img.size(0), w = (int)img.size(1);
+        int w = 0, h = 0;
+        T(t)->render_pose_rgba8(camToWorld, refCameraIndex, outRGBA, w, h);
         if (outWidth) *outWidth = w;
         if (outHeight) *outHeight = h;
-        if (!outRGBA) return;
-        const int64_t n = (int64_t)w * h;
-        msplat::MTensor rgba = msplat::gpu_empty({n}, msplat::DType::Int32);   // 4 bytes per pixel
-        msplat::check(msplat_hip_image_to_rgba8(img.data<float>(), n, rgba.data<uint8_t>()), "rgba8");
-        rgba.copy_to_host(outRGBA, (size_t)n * 4);
     });
 }
 
