@@ -188,3 +188,27 @@ def test_png_read_write_bytes(tmp_path):
     Image.fromarray(b[..., 0], "L").save(tmp_path / "g.png")      # grey: replicated channels
     g = image_io.imread_rgb(str(tmp_path / "g.png"))
     assert np.array_equal(g, np.repeat(b[..., :1], 3, axis=2).astype(np.float32) / np.float32(255))
+
+
+@pytest.mark.parametrize("scale", [0.0, 0.01, 0.3, 3.0, 1e19])
+def test_library_rectangle_equals_the_oracles(scale):
+    """The library's crop rectangle, found four points at a time and stopped
+    where an iteration changes nothing, over lenses whose iteration settles,
+    wanders and overflows: the oracle's 20 plain iterations, exactly."""
+    import ctypes
+    import os
+    from msplat_amd import _abi
+    if not os.path.exists(_abi.LIB_PATH):
+        pytest.skip("libmsplat_hip.so not built")
+    lib = _abi.load()
+    rng = np.random.default_rng(11)
+    for _ in range(60):
+        w, h = (int(v) for v in rng.integers(1, 5000, 2))
+        f = max(w, h) * rng.uniform(0.3, 2.0)
+        intr = np.array([f, f * rng.uniform(0.9, 1.1), w * rng.uniform(0.3, 0.7), h * rng.uniform(0.3, 0.7)],
+                        np.float32)
+        dist = (rng.normal(size=5) * scale * np.array([1, 0.5, 0.02, 0.02, 0.2])).astype(np.float32)
+        roi = (ctypes.c_int32 * 4)()
+        fp = ctypes.POINTER(ctypes.c_float)
+        _abi.check(lib.msplat_undistort_roi(w, h, intr.ctypes.data_as(fp), dist.ctypes.data_as(fp), roi))
+        assert list(roi) == list(orc.undistort_roi(w, h, intr, dist)), (w, h, intr, dist)
