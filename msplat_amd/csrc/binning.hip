@@ -520,7 +520,7 @@ __global__ __launch_bounds__(TS_T) void k_tile_offsets(int T, int nb,
     if (tid < 96 && s_cls[tid]) atomicAdd(&it.cls[64 * (tid >> 5) + (tid & 31)], s_cls[tid]);
     // the projection's intersection and reference counters, copied to the
     // host earlier on the stream, cleared for the next frame
-    if (b == 0 && tid < 2 * ISECT_SLOTS) isect[(size_t)(tid >> 1) * ISECT_STRIDE + (tid & 1)] = 0ull;
+    if (b == 0 && tid < 4 * ISECT_SLOTS) isect[(size_t)(tid >> 2) * ISECT_STRIDE + (tid & 3)] = 0ull;
     if (b == nb - 1 && tid == 0) {
         int mx = 0;
         for (int i = 0; i < nb; ++i) mx = max(mx, tot[3 * i + 2]);
@@ -646,15 +646,22 @@ void launch_depth_order(hipStream_t s, int N, uint32_t* dkey, uint32_t* dval, ui
         *order_out = dval2;
         return;
     }
-    // culled gaussians (key 0xFFFFFFFF) go behind the visible ones in the
-    // first pass and the later passes sort only the visible ones
-    const bool flip = launch_radix_sort(s, dkey, dval, dkey2, dval2, N, 32, radix_temp, &rg, ss,
-                                        nullptr, nullptr, true);
-    uint32_t* order = flip ? dval2 : dval;
-    *order_out = order;
+    // three passes (FAR_BITS), the result in dkey2, dval2; the first leaves out
+    // culled gaussians (key 0xFFFFFFFF)
+    launch_radix_sort(s, dkey, dval, dkey2, dval2, N, FAR_BITS, radix_temp, &rg, ss, nullptr, nullptr, true);
+    *order_out = dval2;
     if (N <= 0) return;
     // the block totals of the super-tile counts in depth order (the reference
     // emission finishes their scan)
+    launch_block_totals(s, rcount, N, rtot);
+}
+
+void launch_depth_order_far(hipStream_t s, int N, uint32_t* dkey, uint32_t* dval, uint32_t* dkey2,
+                            uint32_t* dval2, int* radix_temp, const uint2* rect, uint2* rect_sorted,
+                            int* rcount, int* rtot, uint32_t** order_out) {
+    if (N <= RANK_MAX) return;   // ranked by all bits
+    launch_radix_far(s, dkey2, dval2, dkey, dval, N, radix_temp, RectGather{rect, rect_sorted, rcount});
+    *order_out = dval;
     launch_block_totals(s, rcount, N, rtot);
 }
 

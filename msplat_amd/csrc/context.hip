@@ -344,6 +344,8 @@ CamParams cam_params(const MsplatRenderArgs* a) {
     p.tbx = a->tile_bounds[0];
     p.tby = a->tile_bounds[1];
     p.clip = a->clip_thresh;
+    p.key0 = 0;
+    if (p.clip > 0.f) std::memcpy(&p.key0, &p.clip, 4);
     p.degree = (int)a->degree;
     p.dtu = (int)std::min(a->degrees_to_use, a->degree);
     p.rest_per = (sh_bases(p.degree) - 1) * 3;
@@ -475,6 +477,11 @@ int forward(Ctx* c, const MsplatRenderArgs* a, bool training, float* dst_img = n
     if (I64 > (int64_t)0x7FFFFFFF - 4096)
         return fail(MSPLAT_ERR_ARG, "%lld tile intersections exceed the 32-bit index range",
                     (long long)I64);
+    if (word >> 62 & 1)
+        launch_depth_order_far(c->stream, N, P<uint32_t>(c->dkey), P<uint32_t>(c->dval),
+                               P<uint32_t>(c->dkey2), P<uint32_t>(c->dval2), P<int>(c->dtemp),
+                               P<uint2>(c->rect), P<uint2>(c->rect_sorted), P<int>(c->hits),
+                               P<int>(c->stemp), &order);
     const size_t I = (size_t)std::max<int64_t>(I64, 1);
     const size_t R = (size_t)std::max<int64_t>(R64, 1);
     const size_t NS = (size_t)segments_bound(R64, nst);

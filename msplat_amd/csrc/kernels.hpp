@@ -17,6 +17,7 @@ struct CamParams {
     int W, H;
     int tbx, tby;
     float clip;
+    uint32_t key0;   // depth keys: the depth's bits less these (the near plane's, if it is positive)
     int degree;          // SH degree of the stored coefficients
     int dtu;             // degrees_to_use (clamped to degree)
     int rest_per;        // floats per gaussian in features_rest
@@ -98,11 +99,12 @@ struct ChunkBufs {
     float* aC;           // x3
 };
 
-// Intersection-total counters of the projection: ISECT_SLOTS u64 counter
-// pairs ISECT_STRIDE u64 apart (one 128-byte line each); the first of a pair
-// counts (gaussian, tile) pairs, the second (gaussian, super-tile)
-// references; the totals are the sums over the slots, formed by the first
-// kernel of the depth sort (SlotSum) for the host.
+// Counters of the projection: ISECT_SLOTS slots of u64 counters ISECT_STRIDE
+// u64 apart (one 128-byte line each); a slot's first counts (gaussian, tile)
+// pairs, the second (gaussian, super-tile) references, the third is set where
+// a depth key takes more than FAR_BITS bits; the totals over the slots are
+// formed by the first kernel of the depth sort (SlotSum) for the host.
+constexpr int FAR_BITS = 27;
 constexpr int ISECT_SLOTS = 64;
 constexpr int ISECT_STRIDE = 16;
 constexpr size_t ISECT_BYTES = (size_t)ISECT_SLOTS * ISECT_STRIDE * 8;
@@ -131,17 +133,17 @@ struct SlotSum {
     const unsigned long long* slots;
     unsigned long long* out;
 };
-// Bit 63 set (so that a zeroed word means "not yet"), the intersection total
-// in bits 31..61 and the reference total in bits 0..30, each saturated at
-// 2^31 - 1.
-__host__ __device__ inline unsigned long long totals_word(unsigned long long i, unsigned long long r) {
+// Bit 63 set (so that a zeroed word means "not yet"), bit 62 if a depth key
+// takes more than FAR_BITS bits, the intersection total in bits 31..61 and the
+// reference total in bits 0..30, each saturated at 2^31 - 1.
+__host__ __device__ inline unsigned long long totals_word(unsigned long long i, unsigned long long r, bool far) {
     const unsigned long long cap = 0x7FFFFFFFull;
-    return (1ull << 63) | ((i < cap ? i : cap) << 31) | (r < cap ? r : cap);
+    return (1ull << 63) | ((far ? 1ull : 0ull) << 62) | ((i < cap ? i : cap) << 31) | (r < cap ? r : cap);
 }
 // Optional epilogue of a sort's last pass, for the depth order: output
 // position i also gets rs[i] = rect[value] and cnt[i] = the super-tile count
-// of that rectangle (both zero for the culled key 0xFFFFFFFF, and at the
-// positions of a culling sort's culled tail).
+// of that rectangle (both zero at the positions of a culling sort's culled
+// tail).
 struct RectGather {
     const uint2* rect;
     uint2* rs;
@@ -160,6 +162,8 @@ bool launch_radix_sort(hipStream_t s, uint32_t* k0, uint32_t* v0, uint32_t* k1, 
                        int64_t n, int bits, int* temp, const RectGather* rg = nullptr,
                        const SlotSum* ss = nullptr, int* edge0 = nullptr, int* edge1 = nullptr,
                        bool cull = false);
+void launch_radix_far(hipStream_t s, const uint32_t* ki, const uint32_t* vi, uint32_t* ko, uint32_t* vo,
+                      int64_t n, int* temp, const RectGather& rg);
 
 // Super-tiles: SUPER x SUPER tiles of the tile grid.  A gaussian's tile
 // rectangle is cut into one reference per super-tile it overlaps; the
@@ -187,6 +191,11 @@ __host__ __device__ inline int super_span(int x0, int y0, int x1, int y1) {
 void launch_depth_order(hipStream_t s, int N, uint32_t* dkey, uint32_t* dval, uint32_t* dkey2,
                         uint32_t* dval2, int* radix_temp, int* rank, const uint2* rect, uint2* rect_sorted,
                         int* rcount, int* rtot, const SlotSum* ss, uint32_t** order_out);
+// What the depth order still lacks where the totals word says that a key takes
+// more than FAR_BITS bits (the same arguments).
+void launch_depth_order_far(hipStream_t s, int N, uint32_t* dkey, uint32_t* dval, uint32_t* dkey2,
+                            uint32_t* dval2, int* radix_temp, const uint2* rect, uint2* rect_sorted,
+                            int* rcount, int* rtot, uint32_t** order_out);
 
 // Scratch of launch_tile_lists for R references, S super-tiles, NS =
 // segments_bound(R, S) segments and T tiles.

@@ -190,6 +190,9 @@ __global__ __launch_bounds__(PROJ_T) void k_project_fwd(
     // Intersection and reference totals for the host: one atomic each per
     // workgroup, on one of ISECT_SLOTS counter pairs so that workgroups do
     // not queue on one address.
+    const bool far = area > 0 && (__float_as_uint(ge.z) - p.key0) >> FAR_BITS != 0;
+    unsigned long long* slot = total_isect + (size_t)(blockIdx.x % ISECT_SLOTS) * ISECT_STRIDE;
+    if (wave_ballot(far) && (threadIdx.x & 63) == 0) atomicOr(slot + 2, 1ull);
     int v = area, vr = ge.nref;
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
@@ -207,8 +210,7 @@ __global__ __launch_bounds__(PROJ_T) void k_project_fwd(
 #pragma unroll
         for (int k = 0; k < PROJ_T / 64; ++k) t += s_tot[threadIdx.x][k];
         if (t)
-            atomicAdd(total_isect + (size_t)(blockIdx.x % ISECT_SLOTS) * ISECT_STRIDE + threadIdx.x,
-                      (unsigned long long)t);
+            atomicAdd(slot + threadIdx.x, (unsigned long long)t);
     }
 }
 
@@ -304,7 +306,7 @@ __device__ __forceinline__ void project_col(const CamParams& p, int g, V3 pw, co
     rec[1] = make_float4(cc, sigmoid(ol), col[0], col[1]);
     rec[2] = make_float4(col[2], ex, ey, e.z);
     rec[3] = make_float4(dir.x, dir.y, dir.z, 0.f);
-    dkey[g] = __float_as_uint(e.z);
+    dkey[g] = __float_as_uint(e.z) - p.key0;
 }
 
 }  // namespace

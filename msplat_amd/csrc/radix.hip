@@ -3,9 +3,8 @@
 // their super-tile references by super-tile, and by the nearest-neighbour
 // search to order points by cell.
 //
-// Sort (more than FUSE_BLOCKS blocks): digits of up to 8 bits (9 for a sort of at most 9 bits, done in one
-// pass), reduce-then-scan per pass over 2048-key blocks (512 threads x 4
-// keys):
+// Sort (more than FUSE_BLOCKS blocks): digits of up to 9 bits,
+// reduce-then-scan per pass over 2048-key blocks (512 threads x 4 keys):
 //   1. per-block digit histograms in LDS -> hist[digit][block], and the
 //      digit totals over all blocks (one global atomic per block and digit)
 //   2. one workgroup per digit scans its row of hist and adds the keys of
@@ -17,13 +16,15 @@
 //      runs (coalesced stores).
 // Stability makes the result independent of how work is scheduled: equal keys
 // keep their input order.
-// The depth order sorts with "cull" set: in the first pass the key
-// 0xFFFFFFFF (a culled gaussian) is a digit of its own after all others, so
-// the culled keys end up behind the visible ones in input order, and the
-// later passes sort only the visible keys (their count, written by the first
-// pass, is read on the device).  The visible keys get the order a full sort
-// of all keys gives them; the culled tail is left where the first pass put
-// it, and the last pass writes empty rectangles for it.
+// The depth order sorts with "cull" set: the first pass leaves out the keys
+// 0xFFFFFFFF (culled gaussians), and the later passes sort only the visible
+// keys (their count, written by the first pass, is read on the device).  The
+// last pass writes empty rectangles behind them.
+// Depth keys are the bits of the depth less those of the near plane, and the
+// depth order sorts their low 27 bits in three passes: depths up to 65536 times
+// the near plane.  A fourth (launch_radix_far) follows where the projection
+// found a key beyond; the host learns that while the first passes run.  Four
+// passes of 8 bits for all took 13 us more at 500k gaussians, 11 at 120k.
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -39,16 +40,23 @@ constexpr int RK = 4;              // keys per thread
 constexpr int RB = RT * RK;        // keys per block
 constexpr int WK = RK * 64;        // keys per wave (RK rounds of 64)
 constexpr int SB = SCAN_BLOCK;     // elements per scan block
-constexpr int MAX_PASSES = 4;      // 32-bit keys in 8-bit digits
-constexpr int DMAX = 512;          // digit slots of the widest pass (9 bits, or 8 + the culled digit)
+constexpr int MAX_PASSES = 4;      // 32-bit keys in digits of 8 or 9 bits
+constexpr int DBITS = 9;           // bits of the widest digit
+constexpr int DMAX = 1 << DBITS;   // its digit slots
 constexpr int FUSE_BLOCKS = 64;    // most key blocks of a sort with one kernel a pass
+// Groups of equal digits that a wave of depth keys counts with one atomic before
+// the rest add one each: a 641x421 render of a wall at one depth (120k gaussians)
+// takes 196 us with none and 116 with one; more cost 0.5 us each on spread depths
+// and gain nothing.
+constexpr int AGG_ROUNDS = 1;
 constexpr int DCOPIES = 16;        // copies of the digit totals (block b adds to copy b % 16)
 
-// Digit of key k in a pass: bits [shift, shift + width) (mask), or mask + 1
-// for the culled key 0xFFFFFFFF when cull is set.
-__device__ __forceinline__ int digit_of(uint32_t k, int shift, uint32_t mask, bool cull) {
-    return (cull && k == 0xFFFFFFFFu) ? (int)mask + 1 : (int)((k >> shift) & mask);
+// Digit of key k in a pass: bits [shift, shift + width) (mask).
+__device__ __forceinline__ int digit_of(uint32_t k, int shift, uint32_t mask) {
+    return (int)((k >> shift) & mask);
 }
+// Whether a pass with cull leaves key k out.
+__device__ __forceinline__ bool culled(uint32_t k, bool cull) { return cull && k == 0xFFFFFFFFu; }
 
 // Keys a pass covers: n, or the count the culling first pass wrote.
 __device__ __forceinline__ int64_t pass_n(int64_t n, const int* n_dev) {
@@ -109,21 +117,24 @@ __global__ __launch_bounds__(1024) void k_scan_totals(int* __restrict__ tot, int
 }
 
 // The SlotSum job, by the first wave of one workgroup: lane k reads slot k's
-// pair, the wave sums them and lane 0 publishes the totals word.
+// counters, the wave sums them and lane 0 publishes the totals word.
 __device__ __forceinline__ void slot_sum(const SlotSum& ss) {
-    unsigned long long ti = 0, tr = 0;
+    unsigned long long ti = 0, tr = 0, far = 0;
     for (int k = threadIdx.x; k < ISECT_SLOTS; k += 64) {
         ti += __hip_atomic_load(ss.slots + (size_t)k * ISECT_STRIDE, __ATOMIC_RELAXED,
                                 __HIP_MEMORY_SCOPE_AGENT);
         tr += __hip_atomic_load(ss.slots + (size_t)k * ISECT_STRIDE + 1, __ATOMIC_RELAXED,
                                 __HIP_MEMORY_SCOPE_AGENT);
+        far |= __hip_atomic_load(ss.slots + (size_t)k * ISECT_STRIDE + 2, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
     }
+    const bool any_far = wave_ballot(far != 0) != 0;
     for (int off = 32; off >= 1; off >>= 1) {
         ti += __shfl_xor(ti, off, 64);
         tr += __shfl_xor(tr, off, 64);
     }
     if (threadIdx.x == 0)
-        __hip_atomic_store(ss.out, totals_word(ti, tr), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(ss.out, totals_word(ti, tr, any_far), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Super-tiles of a rectangle as the projection packs it, 0 if it is empty.
@@ -199,12 +210,10 @@ __global__ __launch_bounds__(RK_T) void k_rank_scatter(const uint32_t* __restric
         atomicAdd(&tot[threadIdx.x], s_tot[threadIdx.x]);
 }
 
-// Per-block digit counts.  D: digit slots (256, or 512 for a 9-bit or
-// culling pass).  LDS atomics on one address from many lanes of a wave are
-// serialised, so lanes that share a digit are counted with one atomic where
-// that is common: the culled keys' digit of a culling pass, and with agg (the
-// top byte of depth keys, where a wave's keys mostly share one or two
-// digits) up to four groups of equal digits; the lanes left add one each.
+// Per-block digit counts.  D: digit slots (256, or 512 for a 9-bit pass).
+// LDS atomics on one address from many lanes of a wave are serialised, so with
+// agg (the top bits of depth keys) AGG_ROUNDS groups of equal digits are counted
+// with one atomic each.
 template <int D>
 __global__ __launch_bounds__(RT) void k_radix_hist(const uint32_t* __restrict__ keys, int64_t n,
                                                    const int* __restrict__ n_dev, int shift,
@@ -225,20 +234,11 @@ __global__ __launch_bounds__(RT) void k_radix_hist(const uint32_t* __restrict__ 
 #pragma unroll
     for (int k = 0; k < RK; ++k) {
         const int64_t i = base + k * RT + threadIdx.x;
-        const bool ok = i < ne;
-        const int d = ok ? digit_of(keys[i], shift, mask, cl) : 0;
-        bool left = ok;
-        if (cl) {
-            // the culled keys' digit (about a third of the keys): one atomic
-            // for all of the wave's lanes that hold it
-            const bool cu = ok && d == (int)mask + 1;
-            const uint64_t cm = wave_ballot(cu);
-            if (cm && (int)(threadIdx.x & 63) == (int)__builtin_ctzll(cm))
-                atomicAdd(&h[mask + 1], __popcll(cm));
-            if (cu) left = false;
-        }
+        const uint32_t key = i < ne ? keys[i] : 0u;
+        const int d = digit_of(key, shift, mask);
+        bool left = i < ne && !culled(key, cl);
         if (agg) {
-            for (int r = 0; r < 4; ++r) {
+            for (int r = 0; r < AGG_ROUNDS; ++r) {
                 const uint64_t act = wave_ballot(left);
                 if (act == 0) break;
                 // the lowest lane still left picks the digit of this round
@@ -252,7 +252,7 @@ __global__ __launch_bounds__(RT) void k_radix_hist(const uint32_t* __restrict__ 
         if (left) atomicAdd(&h[d], 1);
     }
     __syncthreads();
-    const int nd = (int)mask + 1 + (cl ? 1 : 0);
+    const int nd = (int)mask + 1;
     if ((int)threadIdx.x < nd) {
         const int c = h[threadIdx.x];
         hist[(size_t)threadIdx.x * nblocks + rb] = c;
@@ -265,10 +265,10 @@ __global__ __launch_bounds__(RT) void k_radix_hist(const uint32_t* __restrict__ 
 // takes 4-6 us whatever it does), so they run one kernel a pass: the scatter
 // adds up the histograms of all blocks itself, and counts, while it writes
 // them out, the digits its keys have in the next pass at the blocks they land
-// in.  Histograms are block-major, D digits a row.  k_fused_first counts the
+// in.  Histograms are block-major, DMAX digits a row.  k_fused_first counts the
 // first pass's digits and clears the later passes' rows.  A 641x421 render with
-// three kernels a pass / one: 121 / 107 us for 25k gaussians, 137 / 130 for
-// 70k, 151 / 144 for 120k, 167 / 164 for 180k, 180 / 188 for 250k (adding up
+// three kernels a pass / one: 113 / 102 us for 25k gaussians, 127 / 120 for
+// 70k, 139 / 132 for 120k, 154 / 154 for 180k, 169 / 174 for 250k (adding up
 // every block's histogram grows with the square of the blocks): the line lies
 // at 64 blocks, 131072 keys.
 struct FusedPass {
@@ -277,35 +277,29 @@ struct FusedPass {
     int next_shift;
     uint32_t next_mask;
     int next_agg;        // rounds of equal counts to add up in the wave first
-    int* nvis;           // culling first pass: gets the number of visible keys
+    int* nvis;           // culling pass: gets the number of visible keys
     int* edge0;          // single-pass sort: output range of each digit, or null
     int* edge1;
 };
-template <int D>
 __global__ __launch_bounds__(RT) void k_fused_first(const uint32_t* __restrict__ keys, int n, int shift,
                                                     uint32_t mask, int cull, int* __restrict__ hist,
-                                                    int* __restrict__ later, int n_later, int later_row,
-                                                    int nb, SlotSum ss) {
-    __shared__ int h[D];
+                                                    int* __restrict__ later, int n_later, int nb,
+                                                    SlotSum ss) {
+    static_assert(RT == DMAX, "a thread a digit");
+    __shared__ int h[DMAX];
     if (ss.out && blockIdx.x == 0 && threadIdx.x < 64) slot_sum(ss);
     const int b = blockIdx.x, tid = threadIdx.x;
-    for (int p = 0; p < n_later; ++p)
-        for (int d = tid; d < later_row; d += RT) later[((size_t)p * nb + b) * later_row + d] = 0;
-    for (int d = tid; d < D; d += RT) h[d] = 0;
+    for (int p = 0; p < n_later; ++p) later[((size_t)p * nb + b) * DMAX + tid] = 0;
+    h[tid] = 0;
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < RK; ++k) {
         const int i = b * RB + k * RT + tid;
-        const bool ok = i < n;
-        const int d = ok ? digit_of(keys[i], shift, mask, cull != 0) : 0;
-        // the culled keys' digit, which many lanes share, by one atomic a wave
-        const bool cu = cull && ok && d == (int)mask + 1;
-        const uint64_t cm = wave_ballot(cu);
-        if (cm && (tid & 63) == (int)__builtin_ctzll(cm)) atomicAdd(&h[mask + 1], __popcll(cm));
-        if (ok && !cu) atomicAdd(&h[d], 1);
+        const uint32_t key = i < n ? keys[i] : 0u;
+        if (i < n && !culled(key, cull != 0)) atomicAdd(&h[digit_of(key, shift, mask)], 1);
     }
     __syncthreads();
-    for (int d = tid; d < D; d += RT) hist[(size_t)b * D + d] = h[d];
+    hist[(size_t)b * DMAX + tid] = h[tid];
 }
 
 // Exclusive scan of one value per thread over the NT threads of a block.
@@ -332,16 +326,16 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int* sh) {
 // digit d in the blocks before b (exclusive scan of the row over the blocks
 // that hold keys of this pass).
 // With edge0 (a single-pass sort) the digit's output range [start, end)
-// also goes to edge0[d], edge1[d] when the digit occurs.  With nvis the
-// workgroup of digit cull_digit (the culled key's) writes its start, the
-// number of visible keys, there.
+// also goes to edge0[d], edge1[d] when the digit occurs.  With nvis (a culling
+// pass) the last digit's workgroup writes its end, the number of visible keys,
+// there.
 template <int D>
 __global__ __launch_bounds__(1024) void k_radix_offsets(int* __restrict__ hist, int nblocks,
                                                         int64_t n, const int* __restrict__ n_dev,
                                                         const int* __restrict__ dtot,
                                                         int* __restrict__ edge0,
                                                         int* __restrict__ edge1,
-                                                        int* __restrict__ nvis, int cull_digit) {
+                                                        int* __restrict__ nvis) {
     __shared__ int sh[16];
     const int d = blockIdx.x, t = threadIdx.x;
     int lower = 0;
@@ -351,7 +345,6 @@ __global__ __launch_bounds__(1024) void k_radix_offsets(int* __restrict__ hist, 
     }
     int carry = block_sum<1024>(lower, sh);
     const int start = carry;
-    if (nvis && d == cull_digit && t == 0) *nvis = start;
     const int nbe = (int)((pass_n(n, n_dev) + RB - 1) / RB);
     int* row = hist + (size_t)d * nblocks;
     for (int c = 0; c < nbe; c += 1024) {
@@ -361,6 +354,7 @@ __global__ __launch_bounds__(1024) void k_radix_offsets(int* __restrict__ hist, 
         if (i < nbe) row[i] = carry + ex;
         carry += block_sum<1024>(v, sh);
     }
+    if (nvis && d == (int)gridDim.x - 1 && t == 0) *nvis = carry;
     if (edge0 && t == 0 && carry > start) {
         edge0[d] = start;
         edge1[d] = carry;
@@ -368,7 +362,7 @@ __global__ __launch_bounds__(1024) void k_radix_offsets(int* __restrict__ hist, 
 }
 
 // One LSD pass over the digit of each key (digit_of: dbits bits, at most D
-// values).  Keys are ranked stably inside the block (each wave ranks its RB/4
+// values; with cull the keys 0xFFFFFFFF are left out).  Keys are ranked stably inside the block (each wave ranks its RB/4
 // consecutive keys in 64-key rounds by ballot-matching the digit bits and
 // keeps per-digit running counts), reordered by digit in LDS, and written out
 // in digit runs so that neighbouring lanes store neighbouring addresses.
@@ -411,8 +405,9 @@ __global__ __launch_bounds__(RT) void k_radix_scatter(const uint32_t* __restrict
     __shared__ int dstart[D];
     __shared__ int gofs[D];
     __shared__ int scan_sh[RW];
+    __shared__ int s_nvalid;
     const bool cl = cull != 0;
-    const int nd = (int)mask + 1 + (cl ? 1 : 0);
+    const int nd = (int)mask + 1;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     // this block's scatter offset of digit tid, loaded now so that its latency
     // overlaps the key loads and the ranking
@@ -426,7 +421,7 @@ __global__ __launch_bounds__(RT) void k_radix_scatter(const uint32_t* __restrict
         int total = 0, before = 0;
 #pragma unroll 16
         for (int b = tid / D; b < nbe; b += STEP) {
-            const int c = f.hist[(size_t)b * D + d];
+            const int c = f.hist[(size_t)b * DMAX + d];
             total += c;
             before += b < rb ? c : 0;
         }
@@ -446,7 +441,7 @@ __global__ __launch_bounds__(RT) void k_radix_scatter(const uint32_t* __restrict
         const int start = block_exclusive_scan<RT>(total, scan_sh);
         my_gofs = start + before;
         if (rb == 0 && tid < nd) {
-            if (f.nvis && cl && tid == nd - 1) *f.nvis = start;
+            if (cl && tid == nd - 1) *f.nvis = start + total;
             if (f.edge0 && total > 0) {
                 f.edge0[tid] = start;
                 f.edge1[tid] = start + total;
@@ -463,11 +458,11 @@ __global__ __launch_bounds__(RT) void k_radix_scatter(const uint32_t* __restrict
 #pragma unroll
     for (int j = 0; j < RK; ++j) {
         const int64_t i = wbase + j * 64 + lane;
-        const bool ok = i < ne;
-        key[j] = ok ? kin[i] : 0u;
-        val[j] = ok ? vin[i] : 0u;
-        if (RG) rc[j] = ok && key[j] != 0xFFFFFFFFu ? rg.rect[val[j]] : make_uint2(0u, 0u);
-        const int d = ok ? digit_of(key[j], shift, mask, cl) : D;
+        key[j] = i < ne ? kin[i] : 0u;
+        val[j] = i < ne ? vin[i] : 0u;
+        const bool ok = i < ne && !culled(key[j], cl);
+        if (RG) rc[j] = ok ? rg.rect[val[j]] : make_uint2(0u, 0u);
+        const int d = ok ? digit_of(key[j], shift, mask) : D;
         dig[j] = d;
         uint64_t peers = wave_ballot(ok);
         if (!ok) peers = ~peers;
@@ -498,6 +493,7 @@ __global__ __launch_bounds__(RT) void k_radix_scatter(const uint32_t* __restrict
     }
     const int start = block_exclusive_scan<RT>(cnt, scan_sh);
     if (tid < D) dstart[tid] = start;
+    if (tid == RT - 1) s_nvalid = start + cnt;
     __syncthreads();
     int lpos[RK];      // each key's place in the block's digit order
 #pragma unroll
@@ -511,7 +507,7 @@ __global__ __launch_bounds__(RT) void k_radix_scatter(const uint32_t* __restrict
         s_val[p] = val[j];
     }
     __syncthreads();
-    const int nvalid = (int)min((int64_t)RB, ne - kbase);
+    const int nvalid = s_nvalid;
     int64_t opos[RK];  // output position of block element tid + u RT
 #pragma unroll
     for (int u = 0; u < RK; ++u) {
@@ -519,16 +515,16 @@ __global__ __launch_bounds__(RT) void k_radix_scatter(const uint32_t* __restrict
         opos[u] = -1;
         if (p >= nvalid) continue;
         const uint32_t k = s_key[p];
-        const int d = digit_of(k, shift, mask, cl);
+        const int d = digit_of(k, shift, mask);
         const int64_t pos = (int64_t)gofs[d] + (p - dstart[d]);
         kout[pos] = k;
         vout[pos] = s_val[p];
         opos[u] = pos;
         if constexpr (FUSED) {
             if (f.next) {
-                int slot = (int)(pos / RB) * 256 + (int)((k >> f.next_shift) & f.next_mask);
-                bool left = !(cl && k == 0xFFFFFFFFu);
-                // the top byte of depth keys: lanes with the same count add once
+                const int slot = (int)(pos / RB) * DMAX + digit_of(k, f.next_shift, f.next_mask);
+                bool left = true;
+                // depth keys: lanes with the same count add once
                 for (int r = 0; r < f.next_agg; ++r) {
                     const uint64_t act = wave_ballot(left);
                     if (act == 0) break;
@@ -590,8 +586,8 @@ void launch_rank_order(hipStream_t s, const uint32_t* key, const uint32_t* val, 
 
 int64_t radix_temp_ints(int64_t n) {
     const int64_t nb = (n + RB - 1) / RB;
-    const int64_t row = nb <= FUSE_BLOCKS ? DMAX + 256 * (MAX_PASSES - 1) : DMAX;
-    return DCOPIES * DMAX * MAX_PASSES + row * nb + 16;
+    const int64_t rows = nb <= FUSE_BLOCKS ? nb * MAX_PASSES : nb;
+    return DCOPIES * DMAX * MAX_PASSES + rows * DMAX + 16;
 }
 
 namespace {
@@ -602,11 +598,11 @@ void launch_pass(hipStream_t s, const uint32_t* ki, const uint32_t* vi, uint32_t
                  int64_t n, const int* n_dev, int shift, uint32_t mask, bool cull, int dbits, bool agg,
                  int nb, int* hist, int* dt, const SlotSum& side, int* edge0, int* edge1, int* nvis,
                  const RectGather* rg) {
-    const int nd = (int)mask + 1 + (cull ? 1 : 0);
+    const int nd = (int)mask + 1;
     hipLaunchKernelGGL(k_radix_hist<D>, dim3(nb), dim3(RT), 0, s, ki, n, n_dev, shift, mask,
                        cull ? 1 : 0, agg ? 1 : 0, nb, hist, dt, side);
     hipLaunchKernelGGL(k_radix_offsets<D>, dim3(nd), dim3(1024), 0, s, hist, nb, n, n_dev,
-                       (const int*)dt, edge0, edge1, cull ? nvis : nullptr, nd - 1);
+                       (const int*)dt, edge0, edge1, cull ? nvis : nullptr);
     if (rg)
         hipLaunchKernelGGL((k_radix_scatter<true, D, false>), dim3(nb), dim3(RT), 0, s, ki, vi, ko, vo, n,
                            n_dev, shift, mask, cull ? 1 : 0, dbits, nb, (const int*)hist, dt, *rg,
@@ -624,8 +620,8 @@ void launch_fused_pass(hipStream_t s, const uint32_t* ki, const uint32_t* vi, ui
                        bool first, int* hist, int* later, int n_later, const SlotSum& side, const FusedPass& f,
                        const RectGather* rg) {
     if (first)
-        hipLaunchKernelGGL(k_fused_first<D>, dim3(nb), dim3(RT), 0, s, ki, (int)n, shift, mask, cull ? 1 : 0,
-                           hist, later, n_later, 256, nb, side);
+        hipLaunchKernelGGL(k_fused_first, dim3(nb), dim3(RT), 0, s, ki, (int)n, shift, mask, cull ? 1 : 0,
+                           hist, later, n_later, nb, side);
     if (rg)
         hipLaunchKernelGGL((k_radix_scatter<true, D, true>), dim3(nb), dim3(RT), 0, s, ki, vi, ko, vo, n,
                            n_dev, shift, mask, cull ? 1 : 0, dbits, nb, (const int*)nullptr, (int*)nullptr, *rg,
@@ -636,89 +632,84 @@ void launch_fused_pass(hipStream_t s, const uint32_t* ki, const uint32_t* vi, ui
                            RectGather{}, f);
 }
 
+// Scratch layout: the digit totals first, at a fixed place whatever n is
+// (DCOPIES x DMAX per pass; each pass's scatter clears its totals for the next
+// sort on this scratch), then the per-block histograms (a fused sort has one
+// set of rows per pass), then the visible count of a culling sort.
+struct RadixTemp {
+    int *dtot, *hist, *nvis;
+    RadixTemp(int* temp, int nb)
+        : dtot(temp), hist(temp + DCOPIES * DMAX * MAX_PASSES),
+          nvis(hist + (size_t)DMAX * nb * (nb <= FUSE_BLOCKS ? MAX_PASSES : 1)) {}
+};
+
 }  // namespace
 
 // Sorts (k0, v0) by the bits [0, bits) of the keys; ping-pongs with (k1, v1).
-// A sort of at most 9 bits takes one pass; otherwise the bits are split into
-// ceil(bits / 8) passes of equal width (fewer digit values give longer runs
-// per digit and block).  Returns true when the result ends up in (k1, v1).
-// With rg the last pass also writes each output position's rectangle and
-// super-tile count (RectGather); with ss the first kernel also does the
-// SlotSum job; with edge0 / edge1 and one pass each occurring key value k
-// gets its output range [edge0[k], edge1[k]) (entries of absent values are
-// not written).  With cull (32-bit depth keys) the keys 0xFFFFFFFF are put
-// behind the others by the first pass and the later passes sort only the
-// others; positions [visible, n) of the result then hold no sorted keys,
-// and rg marks them empty.
+// The bits are split into ceil(bits / 9) passes of equal width (fewer digit
+// values give longer runs per digit and block).  Returns true when the result
+// ends up in (k1, v1).  With rg the last pass also writes each output
+// position's rectangle and super-tile count (RectGather); with ss the first
+// kernel also does the SlotSum job; with edge0 / edge1 and one pass each
+// occurring key value k gets its output range [edge0[k], edge1[k]) (entries of
+// absent values are not written).  With cull the keys 0xFFFFFFFF are left out
+// by the first pass and the later passes sort only the others; positions
+// [visible, n) of the result then hold nothing, and rg marks them empty.
 bool launch_radix_sort(hipStream_t s, uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1,
                        int64_t n, int bits, int* temp, const RectGather* rg, const SlotSum* ss,
                        int* edge0, int* edge1, bool cull) {
     if (n <= 0 || bits <= 0) return false;
     const int nb = (int)((n + RB - 1) / RB);
-    const int passes = bits <= 9 ? 1 : (bits + 7) / 8;
-    // Scratch layout: the digit totals first, at a fixed place whatever n is
-    // (DCOPIES x DMAX per pass; each pass's scatter clears its totals for the
-    // next sort on this scratch), then the per-block histograms, then the
-    // visible count of a culling sort.
-    int* dtot = temp;
-    int* hist = temp + DCOPIES * DMAX * MAX_PASSES;
-    int* nvis = hist + (size_t)DMAX * nb;
-    // (a fused sort's rows take DMAX + 3 x 256 ints a block, the count follows)
-    int* fused_nvis = hist + (size_t)(DMAX + 256 * (MAX_PASSES - 1)) * nb;
+    const int passes = (bits + DBITS - 1) / DBITS;
+    const RadixTemp t(temp, nb);
     // the digit totals arrive zeroed: fresh scratch is, and each pass's
     // scatter clears its own
     bool flip = false;
     int shift = 0;
     for (int pass = 0; pass < passes; ++pass) {
-        const int width = (bits - shift + (passes - pass) - 1) / (passes - pass);
+        auto width_at = [&](int p, int sh) { return (bits - sh + (passes - p) - 1) / (passes - p); };
+        const int width = width_at(pass, shift);
         const uint32_t mask = (1u << width) - 1u;
-        const bool pcull = cull && pass == 0;
-        const int nd = (int)mask + 1 + (pcull ? 1 : 0);
-        int dbits = 0;
-        while ((1 << dbits) < nd) ++dbits;
+        const bool pcull = cull && pass == 0, last = pass == passes - 1;
         uint32_t* ki = flip ? k1 : k0;
         uint32_t* vi = flip ? v1 : v0;
         uint32_t* ko = flip ? k0 : k1;
         uint32_t* vo = flip ? v0 : v1;
-        int* dt = dtot + DCOPIES * DMAX * pass;
         const SlotSum side = ss && pass == 0 ? *ss : SlotSum{nullptr, nullptr};
-        const int* n_dev = cull && pass > 0 ? nvis : nullptr;
-        // the top byte of depth keys: a wave's keys mostly share a digit
-        const bool agg = cull && shift == 24;
-        const RectGather* prg = rg && pass == passes - 1 ? rg : nullptr;
-        if (nb <= FUSE_BLOCKS) {
-            // rows of the first pass (up to DMAX digits), then 256 digits a row
-            int* rows0 = hist;
-            int* later = hist + (size_t)DMAX * nb;
-            auto rows = [&](int p) { return p == 0 ? rows0 : later + (size_t)(p - 1) * nb * 256; };
-            const int nshift = shift + width;
-            const int nwidth = pass + 1 < passes ? (bits - nshift + (passes - pass - 1) - 1) / (passes - pass - 1) : 0;
-            const FusedPass f{rows(pass), pass + 1 < passes ? rows(pass + 1) : nullptr, nshift,
-                              (1u << nwidth) - 1u, cull && nshift == 24 ? 6 : 0, fused_nvis, passes == 1 ? edge0 : nullptr,
-                              passes == 1 ? edge1 : nullptr};
-            const int* nd_dev = cull && pass > 0 ? fused_nvis : nullptr;
-            if (nd > 256)
-                launch_fused_pass<DMAX>(s, ki, vi, ko, vo, n, nd_dev, shift, mask, pcull, dbits, nb, pass == 0,
-                                        rows0, later, passes - 1, side, f, prg);
-            else
-                launch_fused_pass<256>(s, ki, vi, ko, vo, n, nd_dev, shift, mask, pcull, dbits, nb, pass == 0,
-                                       rows0, later, passes - 1, side, f, prg);
-            flip = !flip;
-            shift += width;
-            continue;
-        }
+        const int* n_dev = cull && pass > 0 ? t.nvis : nullptr;
         int* e0 = passes == 1 ? edge0 : nullptr;
         int* e1 = passes == 1 ? edge1 : nullptr;
-        if (nd > 256)
-            launch_pass<DMAX>(s, ki, vi, ko, vo, n, n_dev, shift, mask, pcull, dbits, agg, nb, hist, dt,
-                              side, e0, e1, nvis, prg);
-        else
-            launch_pass<256>(s, ki, vi, ko, vo, n, n_dev, shift, mask, pcull, dbits, agg, nb, hist, dt,
-                             side, e0, e1, nvis, prg);
+        const RectGather* prg = last ? rg : nullptr;
+        if (nb <= FUSE_BLOCKS) {
+            auto rows = [&](int p) { return t.hist + (size_t)p * nb * DMAX; };
+            const int nshift = shift + width;
+            const FusedPass f{rows(pass), last ? nullptr : rows(pass + 1), nshift,
+                              last ? 0u : (1u << width_at(pass + 1, nshift)) - 1u,
+                              cull ? AGG_ROUNDS : 0, t.nvis, e0, e1};
+            auto go = mask >= 256 ? launch_fused_pass<DMAX> : launch_fused_pass<256>;
+            go(s, ki, vi, ko, vo, n, n_dev, shift, mask, pcull, width, nb, pass == 0, rows(0), rows(1),
+               passes - 1, side, f, prg);
+        } else {
+            auto go = mask >= 256 ? launch_pass<DMAX> : launch_pass<256>;
+            go(s, ki, vi, ko, vo, n, n_dev, shift, mask, pcull, width, cull && last, nb, t.hist,
+               t.dtot + DCOPIES * DMAX * pass, side, e0, e1, t.nvis, prg);
+        }
         flip = !flip;
         shift += width;
     }
     return flip;
+}
+
+// The pass over the bits from FAR_BITS on, after a culling sort of those below
+// on the same scratch.
+void launch_radix_far(hipStream_t s, const uint32_t* ki, const uint32_t* vi, uint32_t* ko, uint32_t* vo,
+                      int64_t n, int* temp, const RectGather& rg) {
+    const int nb = (int)((n + RB - 1) / RB);
+    const RadixTemp t(temp, nb);
+    constexpr int W = 32 - FAR_BITS;
+    launch_pass<256>(s, ki, vi, ko, vo, n, t.nvis, FAR_BITS, (1u << W) - 1u, false, W, true, nb, t.hist,
+                     t.dtot + DCOPIES * DMAX * (MAX_PASSES - 1), SlotSum{nullptr, nullptr}, nullptr, nullptr,
+                     nullptr, &rg);
 }
 
 }  // namespace msp

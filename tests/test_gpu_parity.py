@@ -551,3 +551,20 @@ def test_depth_order_fused_passes(dev, n):
     sc.means = (local @ c2w[:3, :3].T + c2w[:3, 3]).astype(np.float32)
     sc.scales -= 1.0
     _render_and_compare(dev, sc)
+
+
+@pytest.mark.parametrize("n", [26000, 131073])
+@pytest.mark.parametrize("clip", [1e-5, 0.0])
+def test_depth_order_far_keys(dev, n, clip):
+    """Depths more than 65536 times the near plane take a fourth radix pass:
+    depths on both sides of it, ties and culled gaussians."""
+    rng = np.random.default_rng(n)
+    sc = small_scene(n=n, width=300, height=270, seed_off=122, degree=0)
+    c2w = np.asarray(sc.cameras[0].cam_to_world, np.float64)
+    z = np.where(rng.random(n) < 0.3, rng.choice([-1.0, 0.6, 0.66, 3.9], n), np.exp(rng.uniform(-1.2, 3.5, n)))
+    local = np.stack([rng.uniform(-0.7, 0.7, n) * abs(z), rng.uniform(-0.6, 0.6, n) * abs(z), -z], 1)
+    sc.means = (local @ c2w[:3, :3].T + c2w[:3, 3]).astype(np.float32)
+    sc.scales -= 1.5
+    keys = z[z > 0].astype(np.float32).view(np.uint32) - (np.float32(clip).view(np.uint32) if clip > 0 else 0)
+    assert len(np.unique(keys >> 27)) > 1 and (keys >> 27).max() > 0
+    parity.render_and_compare(dev, sc.params(), 0, sc.cameras[0], clip=clip)
