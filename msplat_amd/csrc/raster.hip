@@ -19,10 +19,9 @@
 // with these MI355X differences: each loaded entry carries a conservative
 // mask of the tile's sixteen 4x4 blocks it can reach and a row of lanes walks
 // only the entries of its own block; a workgroup-wide vote stops the forward once
-// every pixel of the item has terminated; the backward reduces each
-// gaussian's per-pixel terms across the 64 lanes of a wave (eight of them
-// transposed through LDS, the ninth by DPP) and nine lanes issue one float
-// atomic each.
+// every pixel of the item has terminated; the backward holds 16 entries in a
+// row's lanes, scans what a pixel carries from one to the next, and adds a
+// window's gradient sums to memory with consecutive lanes on consecutive floats.
 #include "common.hpp"
 #include "kernels.hpp"
 

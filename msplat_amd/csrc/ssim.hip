@@ -40,69 +40,62 @@ constexpr int WIN = 11;
 // Tile of TX x TY output pixels, NT threads, and the regions of its passes
 // (rows / columns relative to the tile's first output pixel (x0, y0)):
 //   input (gt, render)    rows -10 .. TY+9,  columns -10 .. TX+9   IN_H x IN_W
-//   horizontal sums       rows -10 .. TY+9,  columns -5 .. TX+4    HS_H x HS_W
+//   horizontal sums       rows -10 .. TY+9,  columns -5 .. TX+4    IN_H x FD_W
 //   fields f1, f2, f3     rows -5 .. TY+4,   columns -5 .. TX+4    FD_H x FD_W
 //   horizontal backward   rows -5 .. TY+4,   columns 0 .. TX-1     FD_H x TX
 //   vertical backward     rows 0 .. TY-1,    columns 0 .. TX-1     the outputs
 // For 32 x 32 outputs the horizontal sums are evaluated 2.13 times per
-// output, the fields 1.72 times and the horizontal backward 1.31 times.  The
-// two sum passes take two neighbouring positions per item (along the row for
-// the horizontal sums, down the column for the vertical ones): the twelve
-// inputs of the pair are read once instead of eleven per position, and the
-// vertical pass's 21 x 42 items take one round of the 1024 threads.
-constexpr int TX = 32, TY = 32, NT = 1024;
-constexpr int IN_W = TX + 4 * HALF;   // 52
-constexpr int IN_H = TY + 4 * HALF;   // 52
-constexpr int HS_W = TX + 2 * HALF;   // 42
-constexpr int HS_H = IN_H;            // 52
-constexpr int FD_W = HS_W;            // 42
-constexpr int FD_H = TY + 2 * HALF;   // 42
-// LDS layouts, chosen so that most of the passes' accesses are free of bank
-// conflicts (64 banks of 4 bytes; a wave's 8-byte reads are served 32 lanes at a time,
-// its 16-byte reads 16 lanes at a time):
-//  * input: (gt, render) of a position as one float2, rows IN_S float2 apart.
-//    The horizontal pass gives lane l the position pair p + l of a row-major
-//    walk over the HS_H x HS_W / 2 pairs and reads its inputs 16 bytes (two
-//    positions) at a time, so 16 lanes cover at most two row pieces, pairs
-//    [a, 21) of one row and [0, a - 5) of the next; IN_S = 74 = 10 (mod 32)
-//    puts the second piece on exactly the 16-byte bank groups the first
-//    leaves.
-//  * horizontal sums: (mu_x, mu_y, E[x^2], E[y^2]) as a float4 and E[xy] as a
-//    float, row-major over HS_H x HS_W (the vertical pass's lanes read
-//    consecutive positions).  Lanes share bank groups where the vertical
-//    pass's items wrap to the row pair below and in the horizontal pass's
-//    two float4 stores per lane; layouts without those conflicts were
-//    measured no faster.
-//  * fields (f1, f2, f3) as one float4 per position, row-major over
-//    FD_H x FD_W: the horizontal backward's 16-lane quarters read 16
-//    consecutive positions of one row.
-//  * horizontal backward (h1, h2, h3) as one float4 per position, row-major
-//    over FD_H x TX: the vertical backward's lanes read consecutive columns.
+// output, the fields 1.72 times and the horizontal backward 1.31 times (16 x
+// 16: 3.66, 2.64 and 1.63 times).
+// Bound by vector issue, LDS reads and the latency between barriers, so every
+// pass's item takes a run of neighbouring positions: KH of a row for the
+// horizontal sums, KV of a column for the vertical ones, KB of a row and KO of
+// a column for the backward passes.  A run's inputs (ten more than its
+// positions) are read once, where one position an item reads eleven each, and
+// its positions are independent chains of multiply-adds.
+// LDS layouts (64 banks of 4 bytes; 16-byte reads are served 16 lanes at a
+// time): in the two horizontal passes consecutive lanes take consecutive rows,
+// whose strides are odd numbers of 16-byte groups, and in the two vertical
+// ones consecutive columns, so that neither reads nor writes share banks
+// (but where a wave wraps from one run to the next).
+//  * input: (gt, render) of a position as one float2, read two at a time
+//  * horizontal sums: (mu_x, mu_y, E[x^2], E[y^2]) as a float4 and E[xy] as a float
+//  * fields (f1, f2, f3) and horizontal backward (h1, h2, h3) as a float4 each
 // The input and the fields share one LDS area, the horizontal sums and the
-// horizontal backward another (each pass reads one and writes the other):
-// 74.5 KB, two workgroups per CU; 1024 threads each (at most 64 VGPRs) make
-// that eight waves per SIMD, which hide the passes' LDS latency and barriers
-// better than 512 threads (four waves per SIMD) did.
-constexpr int IN_S = 74;
-constexpr int LDS_A = IN_H * IN_S * 8;                  // input; the fields (FD_H x FD_W x 16) fit
-constexpr int LDS_B = HS_H * HS_W * (16 + 4);           // horizontal sums; the backward (FD_H x TX x 16) fits
-static_assert(FD_H * FD_W * 16 <= LDS_A, "fields overflow the input's area");
-static_assert(FD_H * TX * 16 <= LDS_B, "horizontal backward overflows the sums' area");
-static_assert(HS_W % 2 == 0 && FD_H % 2 == 0 && IN_S % 2 == 0, "two positions per item, 16-byte aligned");
-constexpr int NPOS = (IN_H * IN_W + NT - 1) / NT;      // input positions per thread
-constexpr int NOUT = TX * TY / NT;                      // output pixels per thread
+// horizontal backward another (each pass reads one and writes the other).
+template <int TX_, int TY_, int NT_, int KH_, int KV_, int KB_, int KO_, int WAVES_>
+struct Tile {
+    static constexpr int TX = TX_, TY = TY_, NT = NT_, KH = KH_, KV = KV_, KB = KB_, KO = KO_;
+    static constexpr int WAVES = WAVES_;                                   // per SIMD
+    static constexpr int IN_W = TX + 4 * HALF, IN_H = TY + 4 * HALF;
+    static constexpr int FD_W = TX + 2 * HALF, FD_H = TY + 2 * HALF;
+    static constexpr int NH = (FD_W + KH - 1) / KH, NV = (FD_H + KV - 1) / KV;   // runs
+    static constexpr int odd(int v) { return v | 1; }
+    static constexpr int IN_S = 2 * odd((NH * KH + 2 * HALF + 1) / 2);      // row strides
+    static constexpr int HS_S = odd(FD_W), FD_S = odd(FD_W), HB_S = odd(TX);
+    static constexpr int HS_H = NV * KV + 2 * HALF;                         // rows the runs read
+    static constexpr int cmax(int a, int b) { return a > b ? a : b; }
+    static constexpr int LDS_A = cmax(IN_H * IN_S * 8, FD_H * FD_S * 16);
+    static constexpr int LDS_B = cmax(HS_H * HS_S * (16 + 4), FD_H * HB_S * 16);
+    static constexpr int NPOS = (IN_H * IN_W + NT - 1) / NT;                // input positions per thread
+    static_assert(KH % 2 == 0 && TX % KB == 0 && TY % KO == 0, "runs");
+    static_assert(TX * TY / KO <= NT, "one run of outputs per thread");
+};
 
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void k_ssim_tile(int W, int H, const float* __restrict__ img,
-                                                  const float* __restrict__ gt, float w_ssim,
-                                                  float inv_n, float* __restrict__ v_rendered,
-                                                  float* __restrict__ loss_part) {
-    __shared__ __align__(16) char lds_a[LDS_A];
-    __shared__ __align__(16) char lds_b[LDS_B];
+template <class G>
+__global__ __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(G::WAVES))) void k_ssim_tile(
+    int W, int H, const float* __restrict__ img, const float* __restrict__ gt, float w_ssim,
+    float inv_n, float* __restrict__ v_rendered, float* __restrict__ loss_part) {
+    constexpr int TX = G::TX, TY = G::TY, NT = G::NT, KH = G::KH, KV = G::KV, KB = G::KB, KO = G::KO;
+    constexpr int IN_W = G::IN_W, IN_H = G::IN_H, FD_W = G::FD_W, FD_H = G::FD_H, NPOS = G::NPOS;
+    constexpr int IN_S = G::IN_S, HS_S = G::HS_S, FD_S = G::FD_S, HB_S = G::HB_S;
+    __shared__ __align__(16) char lds_a[G::LDS_A];
+    __shared__ __align__(16) char lds_b[G::LDS_B];
     __shared__ float s_red[3][NT / 64];
     float2* s_in = reinterpret_cast<float2*>(lds_a);
     float4* s_f = reinterpret_cast<float4*>(lds_a);
     float4* s_h4 = reinterpret_cast<float4*>(lds_b);
-    float* s_h1 = reinterpret_cast<float*>(lds_b + HS_H * HS_W * 16);
+    float* s_h1 = reinterpret_cast<float*>(lds_b + G::HS_H * HS_S * 16);
     float4* s_hb = reinterpret_cast<float4*>(lds_b);
     const int t = threadIdx.x;
     const int x0 = blockIdx.x * TX, y0 = blockIdx.y * TY;
@@ -117,30 +110,25 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void k_
         const int iy = i / IN_W, ix = i - iy * IN_W;
         const int gy = y0 - 2 * HALF + iy, gx = x0 - 2 * HALF + ix;
         const bool in = i < IN_H * IN_W && gx >= 0 && gx < W && gy >= 0 && gy < H;
+        const size_t q = in ? ((size_t)gy * W + gx) * 3 : 0;
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            const size_t q = ((size_t)gy * W + gx) * 3 + c;
-            rg[k][c] = in ? gt[q] : 0.f;
-            rr[k][c] = in ? img[q] : 0.f;
+            rg[k][c] = gt[q + c];
+            rr[k][c] = img[q + c];
         }
-    }
-    // this thread's output pixels: column t % TX, rows t / TX + (NT / TX) j
-    const int ox = t % TX, oy0 = t / TX;
-    float og[NOUT][3], orr[NOUT][3], vr[NOUT][3];
-    bool oin[NOUT];
-#pragma unroll
-    for (int j = 0; j < NOUT; ++j) {
-        const int gx = x0 + ox, gy = y0 + oy0 + (NT / TX) * j;
-        oin[j] = gx < W && gy < H;
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            const size_t q = ((size_t)gy * W + gx) * 3 + c;
-            og[j][c] = oin[j] ? gt[q] : 0.f;
-            orr[j][c] = oin[j] ? img[q] : 0.f;
-            vr[j][c] = 0.f;
+            rg[k][c] = in ? rg[k][c] : 0.f;
+            rr[k][c] = in ? rr[k][c] : 0.f;
         }
-        if (oin[j]) cnt += 1.f;
     }
+    // this thread's output pixels: column ox, rows oy .. oy + KO - 1
+    const int ox = t % TX, oy = (t / TX) * KO;
+    const int gox = x0 + ox, goy = y0 + oy;
+    const int n_out = oy < TY && gox < W ? min(KO, H - goy) : 0;   // may be negative
+    float vr[KO][3] = {};
+#pragma unroll
+    for (int u = 0; u < KO; ++u) cnt += u < n_out ? 1.f : 0.f;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
         // the previous channel's vertical backward has read the horizontal
@@ -157,27 +145,25 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void k_
         }
         __syncthreads();
         // horizontal zero-padded sums (ssim_h_fwd, .metal:3094-3114) at the
-        // in-image positions; zero elsewhere.  An item takes two neighbouring
-        // positions: their twelve inputs are six 16-byte reads (each position
-        // adds its eleven terms in the reference's order).
-        for (int i = t; i < HS_H * (HS_W / 2); i += NT) {
-            const int hy = i / (HS_W / 2), hx = 2 * (i - hy * (HS_W / 2));
+        // in-image positions; zero elsewhere.  Input k of a run is term k - u
+        // of the sums of its position u, each added in the reference's order.
+        // (A last run may read past the input's columns, for positions past
+        // FD_W that it does not store.)
+        for (int i = t; i < IN_H * G::NH; i += NT) {
+            const int hg = i / IN_H, hy = i - hg * IN_H, hx = KH * hg;
             const int gy = y0 - 2 * HALF + hy, gx = x0 - HALF + hx;
             const bool rin = gy >= 0 && gy < H;
-            const bool in0 = rin && gx >= 0 && gx < W, in1 = rin && gx + 1 >= 0 && gx + 1 < W;
-            // inputs hx + k, k = 0..11, read two at a time: input k is term k
-            // of the first position's sums and term k - 1 of the second's
-            float acc[2][5] = {};
+            float acc[KH][5] = {};
             const float4* row = reinterpret_cast<const float4*>(s_in + hy * IN_S + hx);
 #pragma unroll
-            for (int q = 0; q < (WIN + 1) / 2; ++q) {
+            for (int q = 0; q < (KH + WIN - 1) / 2; ++q) {
                 const float4 f = row[q];
 #pragma unroll
                 for (int e = 0; e < 2; ++e) {
                     const int k = 2 * q + e;
                     const float gv = e ? f.z : f.x, rv = e ? f.w : f.y;
 #pragma unroll
-                    for (int u = 0; u < 2; ++u) {
+                    for (int u = 0; u < KH; ++u) {
                         const int d = k - u;
                         if (d < 0 || d >= WIN) continue;
                         const float w = GAUSS_1D[d];
@@ -190,61 +176,51 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void k_
                     }
                 }
             }
-            float a[2][5];
+            const int o = hy * HS_S + hx;
 #pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const bool in = u == 0 ? in0 : in1;
-#pragma unroll
-                for (int r = 0; r < 5; ++r) a[u][r] = in ? acc[u][r] : 0.f;
+            for (int u = 0; u < KH; ++u) {
+                const bool in = rin && gx + u >= 0 && gx + u < W;
+                if (FD_W % KH != 0 && hx + u >= FD_W) continue;
+                s_h4[o + u] = make_float4(in ? acc[u][0] : 0.f, in ? acc[u][1] : 0.f, in ? acc[u][2] : 0.f,
+                                          in ? acc[u][3] : 0.f);
+                s_h1[o + u] = in ? acc[u][4] : 0.f;
             }
-            const int o = hy * HS_W + hx;
-            s_h4[o] = make_float4(a[0][0], a[0][1], a[0][2], a[0][3]);
-            s_h4[o + 1] = make_float4(a[1][0], a[1][1], a[1][2], a[1][3]);
-            *reinterpret_cast<float2*>(s_h1 + o) = make_float2(a[0][4], a[1][4]);
         }
         __syncthreads();
         // vertical sums, SSIM and the derivative fields (.metal:3243-3300)
         // at the centres of the in-image rows (the fields of other rows are
-        // never read: their horizontal backward is zero).  An item takes two
-        // rows of one column: twelve rows of sums serve both.
-        for (int i = t; i < (FD_H / 2) * FD_W; i += NT) {
-            const int fy0 = 2 * (i / FD_W), fx = i - (i / FD_W) * FD_W;
+        // never read: their horizontal backward is zero).  Row k of a run is
+        // term k - u of the sums of its row u, each added in order.
+        for (int i = t; i < G::NV * FD_W; i += NT) {
+            const int fy0 = KV * (i / FD_W), fx = i - (i / FD_W) * FD_W;
             const int gx = x0 - HALF + fx;
-            // rows fy0 + k, k = 0..11: row k is term k of the first row's
-            // sums and term k - 1 of the second's, each added in order
-            float acc[2][5] = {};
+            float acc[KV][5] = {};
 #pragma unroll
-            for (int k = 0; k < WIN + 1; ++k) {
-                const float4 q = s_h4[(fy0 + k) * HS_W + fx];
-                const float q4 = s_h1[(fy0 + k) * HS_W + fx];
-                if (k < WIN) {
-                    const float w = GAUSS_1D[k];
-                    acc[0][0] = fmaf(w, q.x, acc[0][0]);
-                    acc[0][1] = fmaf(w, q.y, acc[0][1]);
-                    acc[0][2] = fmaf(w, q.z, acc[0][2]);
-                    acc[0][3] = fmaf(w, q.w, acc[0][3]);
-                    acc[0][4] = fmaf(w, q4, acc[0][4]);
+            for (int k = 0; k < KV + WIN - 1; ++k) {
+                const float4 q = s_h4[(fy0 + k) * HS_S + fx];
+                const float q4 = s_h1[(fy0 + k) * HS_S + fx];
+#pragma unroll
+                for (int u = 0; u < KV; ++u) {
+                    const int d = k - u;
+                    if (d < 0 || d >= WIN) continue;
+                    const float w = GAUSS_1D[d];
+                    acc[u][0] = fmaf(w, q.x, acc[u][0]);
+                    acc[u][1] = fmaf(w, q.y, acc[u][1]);
+                    acc[u][2] = fmaf(w, q.z, acc[u][2]);
+                    acc[u][3] = fmaf(w, q.w, acc[u][3]);
+                    acc[u][4] = fmaf(w, q4, acc[u][4]);
+                    // the sums are formed row by row (without this the compiler
+                    // sinks them into the per-row validity test and keeps all
+                    // rows in registers, which spills)
+                    asm volatile("" : "+v"(acc[u][0]), "+v"(acc[u][1]), "+v"(acc[u][2]), "+v"(acc[u][3]),
+                                 "+v"(acc[u][4]));
                 }
-                if (k > 0) {
-                    const float w = GAUSS_1D[k - 1];
-                    acc[1][0] = fmaf(w, q.x, acc[1][0]);
-                    acc[1][1] = fmaf(w, q.y, acc[1][1]);
-                    acc[1][2] = fmaf(w, q.z, acc[1][2]);
-                    acc[1][3] = fmaf(w, q.w, acc[1][3]);
-                    acc[1][4] = fmaf(w, q4, acc[1][4]);
-                }
-                // the sums are formed row by row (without this the compiler
-                // sinks them into the per-row validity test and keeps all
-                // twelve rows in registers, which spills)
-                asm volatile("" : "+v"(acc[0][0]), "+v"(acc[0][1]), "+v"(acc[0][2]), "+v"(acc[0][3]),
-                             "+v"(acc[0][4]), "+v"(acc[1][0]), "+v"(acc[1][1]), "+v"(acc[1][2]),
-                             "+v"(acc[1][3]), "+v"(acc[1][4]));
             }
 #pragma unroll
-            for (int u = 0; u < 2; ++u) {
+            for (int u = 0; u < KV; ++u) {
                 const int fy = fy0 + u;
                 const int gy = y0 - HALF + fy;
-                if (gy < 0 || gy >= H) continue;
+                if (gy < 0 || gy >= H || (FD_H % KV != 0 && fy >= FD_H)) continue;
                 const float mx = acc[u][0], my = acc[u][1], sx = acc[u][2], sy = acc[u][3],
                             cxy = acc[u][4];
                 const float sxs = sx - mx * mx, sys = sy - my * my, sxy = cxy - mx * my;
@@ -253,62 +229,82 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void k_
                 const float iCD = 1.0f / (Cd * D);
                 const float dmu = 2.0f * B * (mx * Cd - A * my) / (Cd * Cd * D);
                 const float dsyq = -A * B * iCD / D, dsxy = 2.0f * A * iCD;
-                s_f[fy * FD_W + fx] = make_float4(dmu - 2.0f * my * dsyq - mx * dsxy, 2.0f * dsyq, dsxy, 0.f);
+                s_f[fy * FD_S + fx] = make_float4(dmu - 2.0f * my * dsyq - mx * dsxy, 2.0f * dsyq, dsxy, 0.f);
                 // the tile's own in-image outputs add their SSIM to the loss
                 if (fy >= HALF && fy < HALF + TY && fx >= HALF && fx < HALF + TX && gx >= 0 && gx < W)
                     ssim_sum += (A * B) / (Cd * D);
             }
         }
+        // this thread's output pixels of the channel, for the last pass
+        float og[KO], orr[KO];
+#pragma unroll
+        for (int u = 0; u < KO; ++u) {
+            const size_t q = u < n_out ? ((size_t)(goy + u) * W + gox) * 3 + c : 0;
+            og[u] = gt[q];
+            orr[u] = img[q];
+        }
         __syncthreads();
         // mirrored horizontal backward at the in-image rows of the tile's
-        // columns +- 5 rows (zero at rows outside the image)
-        for (int i = t; i < FD_H * TX; i += NT) {
-            const int by = i / TX, bx = i - by * TX;
+        // columns +- 5 rows (zero at rows outside the image, whose fields are
+        // not formed)
+        for (int i = t; i < FD_H * (TX / KB); i += NT) {
+            const int bg = i / FD_H, by = i - bg * FD_H, bx = KB * bg;
             const int gy = y0 - HALF + by;
-            float h1 = 0.f, h2 = 0.f, h3 = 0.f;
+            float h[KB][3] = {};
             if (gy >= 0 && gy < H) {
-                const float4* fr = s_f + by * FD_W + bx;
+                const float4* fr = s_f + by * FD_S + bx;
 #pragma unroll
-                for (int d = 0; d < WIN; ++d) {
-                    const float w = GAUSS_1D[WIN - 1 - d];
-                    const float4 f = fr[d];
-                    h1 = fmaf(w, f.x, h1);
-                    h2 = fmaf(w, f.y, h2);
-                    h3 = fmaf(w, f.z, h3);
+                for (int k = 0; k < KB + WIN - 1; ++k) {
+                    const float4 f = fr[k];
+#pragma unroll
+                    for (int u = 0; u < KB; ++u) {
+                        const int d = k - u;
+                        if (d < 0 || d >= WIN) continue;
+                        const float w = GAUSS_1D[WIN - 1 - d];
+                        h[u][0] = fmaf(w, f.x, h[u][0]);
+                        h[u][1] = fmaf(w, f.y, h[u][1]);
+                        h[u][2] = fmaf(w, f.z, h[u][2]);
+                    }
                 }
             }
-            s_hb[i] = make_float4(h1, h2, h3, 0.f);
+#pragma unroll
+            for (int u = 0; u < KB; ++u) s_hb[by * HB_S + bx + u] = make_float4(h[u][0], h[u][1], h[u][2], 0.f);
         }
         __syncthreads();
         // mirrored vertical backward (.metal:3443-3463) and the L1 term
+        if (n_out > 0) {
+            float f[KO][3] = {};
+            const float4* hr = s_hb + oy * HB_S + ox;
 #pragma unroll
-        for (int j = 0; j < NOUT; ++j) {
-            if (!oin[j]) continue;
-            const int oy = oy0 + (NT / TX) * j;
-            float f1 = 0.f, f2 = 0.f, f3 = 0.f;
-            const float4* hr = s_hb + oy * TX + ox;
+            for (int k = 0; k < KO + WIN - 1; ++k) {
+                const float4 h = hr[k * HB_S];
 #pragma unroll
-            for (int d = 0; d < WIN; ++d) {
-                const float w = GAUSS_1D[WIN - 1 - d];
-                const float4 h = hr[d * TX];
-                f1 = fmaf(w, h.x, f1);
-                f2 = fmaf(w, h.y, f2);
-                f3 = fmaf(w, h.z, f3);
+                for (int u = 0; u < KO; ++u) {
+                    const int d = k - u;
+                    if (d < 0 || d >= WIN) continue;
+                    const float w = GAUSS_1D[WIN - 1 - d];
+                    f[u][0] = fmaf(w, h.x, f[u][0]);
+                    f[u][1] = fmaf(w, h.y, f[u][1]);
+                    f[u][2] = fmaf(w, h.z, f[u][2]);
+                }
             }
-            const float r = orr[j][c], g = og[j][c];
-            const float v_ssim = f1 + r * f2 + g * f3;
-            const float v_l1 = (g > r) ? -1.0f : ((g < r) ? 1.0f : 0.0f);
-            vr[j][c] = inv_n * (-w_ssim * v_ssim + (1.0f - w_ssim) * v_l1);
-            l1_sum += fabsf(g - r);
+#pragma unroll
+            for (int u = 0; u < KO; ++u) {
+                const float r = orr[u], g = og[u];
+                const float v_ssim = f[u][0] + r * f[u][1] + g * f[u][2];
+                const float v_l1 = (g > r) ? -1.0f : ((g < r) ? 1.0f : 0.0f);
+                vr[u][c] = inv_n * (-w_ssim * v_ssim + (1.0f - w_ssim) * v_l1);
+                l1_sum += u < n_out ? fabsf(g - r) : 0.f;
+            }
         }
     }
 #pragma unroll
-    for (int j = 0; j < NOUT; ++j) {
-        if (!oin[j]) continue;
-        const size_t q = ((size_t)(y0 + oy0 + (NT / TX) * j) * W + x0 + ox) * 3;
-        v_rendered[q + 0] = vr[j][0];
-        v_rendered[q + 1] = vr[j][1];
-        v_rendered[q + 2] = vr[j][2];
+    for (int u = 0; u < KO; ++u) {
+        if (u >= n_out) continue;
+        const size_t q = ((size_t)(goy + u) * W + gox) * 3;
+        v_rendered[q + 0] = vr[u][0];
+        v_rendered[q + 1] = vr[u][1];
+        v_rendered[q + 2] = vr[u][2];
     }
     // Workgroup partials of (sum SSIM, sum L1, pixels).
     const float a = wave_sum(ssim_sum), b = wave_sum(l1_sum), n = wave_sum(cnt);
@@ -326,14 +322,44 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void k_
     }
 }
 
+// The tile by the size of the image.  A call takes about as long as its
+// rounds of workgroups: 256 CUs hold two of the larger tiles each.
+//  * 16 x 16 while every tile gets a CU of its own: the chain of passes is
+//    shortest (256x256: 11.1 us, against 15.0 with 32 x 24 and 18.0 with 32 x 32)
+//  * else 32 x 32, which recomputes the least halo, or 32 x 24, whose round
+//    takes 5/6 of the time, whichever makes less of the rounds (1297x840: 61.2
+//    us in three rounds against 64.7 in three; 2594x1680: 204 us in nine against
+//    220 in twelve; 800x600: 28.4 us in one against 33.2 in two)
+// One pass position per item and 32 x 32 tiles for all took 19.3 us at
+// 256x256, 30.3 at 648x420, 67.8 at 1297x840 and 217 at 2594x1680.
+using TileS = Tile<16, 16, 512, 2, 2, 1, 1, 8>;
+using TileM = Tile<32, 24, 512, 4, 3, 4, 2, 4>;
+using TileL = Tile<32, 32, 512, 6, 4, 4, 2, 4>;
+constexpr int CUS = 256;
+
+template <class G>
+int tiles(int W, int H) {
+    return ((W + G::TX - 1) / G::TX) * ((H + G::TY - 1) / G::TY);
+}
+
+template <class G>
+int run(hipStream_t s, int H, int W, const float* img, const float* gt, float w, float inv_n,
+        float* v_rendered, float* loss_part) {
+    const dim3 grid((W + G::TX - 1) / G::TX, (H + G::TY - 1) / G::TY);
+    hipLaunchKernelGGL(k_ssim_tile<G>, grid, dim3(G::NT), 0, s, W, H, img, gt, w, inv_n, v_rendered,
+                       loss_part);
+    return tiles<G>(W, H);
+}
+
 }  // namespace
 
 int launch_ssim(hipStream_t s, int H, int W, const float* img, const float* gt, float w,
                 float inv_n, float* v_rendered, float* loss_part) {
-    const dim3 grid((W + TX - 1) / TX, (H + TY - 1) / TY);
-    hipLaunchKernelGGL(k_ssim_tile, grid, dim3(NT), 0, s, W, H, img, gt, w, inv_n, v_rendered,
-                       loss_part);
-    return (int)(grid.x * grid.y);
+    const auto rounds = [](int n) { return (n + 2 * CUS - 1) / (2 * CUS); };
+    if (tiles<TileS>(W, H) <= CUS) return run<TileS>(s, H, W, img, gt, w, inv_n, v_rendered, loss_part);
+    if (5 * rounds(tiles<TileM>(W, H)) < 6 * rounds(tiles<TileL>(W, H)))
+        return run<TileM>(s, H, W, img, gt, w, inv_n, v_rendered, loss_part);
+    return run<TileL>(s, H, W, img, gt, w, inv_n, v_rendered, loss_part);
 }
 
 }  // namespace msp

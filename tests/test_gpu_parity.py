@@ -199,6 +199,15 @@ def test_train_step_tiny_odd_images(dev, width, height):
     _train_compare(dev, small_scene(n=300, width=width, height=height, seed_off=95 + width))
 
 
+# loss tiles of 16x16 (up to 256 of them), 32x24 and 32x32; sizes at and around tile edges
+@pytest.mark.parametrize("width,height", [(16, 16), (49, 31), (256, 256), (257, 256), (321, 337), (637, 607),
+                                          (640, 608)])
+def test_train_step_loss_tiles(dev, width, height):
+    """Each tile shape of the loss kernel, whole and cut by the image's
+    edges; the loss gradient image must stay bit-exact."""
+    _train_compare(dev, small_scene(n=1500, width=width, height=height, seed_off=130 + width))
+
+
 def test_train_step_partial_edge_tiles_chunked(dev):
     """Partial edge tiles in chunk mode (fewer than 400 tiles) with
     multi-chunk tiles: prefix / suffix backward at the image border."""
