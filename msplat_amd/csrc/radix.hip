@@ -173,6 +173,12 @@ __global__ __launch_bounds__(RK_T) void k_rank(const uint32_t* __restrict__ key,
 #pragma unroll
         for (int u = 0; u < 16; ++u) c += key[j + u] <= k ? 1 : 0;
     for (; j < a; ++j) c += key[j] <= k ? 1 : 0;
+    for (; j + 16 <= b; j += 16)
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const uint32_t o = key[j + u];
+            c += o < k || (o == k && j + u < i) ? 1 : 0;
+        }
     for (; j < b; ++j) {
         const uint32_t o = key[j];
         c += o < k || (o == k && j < i) ? 1 : 0;
