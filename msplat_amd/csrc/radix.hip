@@ -153,7 +153,10 @@ __device__ __forceinline__ int rect_span(uint2 r) {
 // clears the scan's block totals and does the SlotSum job.
 // Few keys leave a radix sort's passes bound by launches, not by work: 12
 // launches of 4-6 us for the depth order of 10k gaussians, 66 us, against two
-// here, 11 us.  The comparisons grow with the square of n.
+// here, 13 and 4 us.  The comparisons grow with the square of n.  The
+// workgroup's own keys go sixteen at a time like the others: one scalar load
+// waited for after the other, they made the diagonal workgroups last and the
+// launch 18.7 us.
 constexpr int RK_T = 256;
 __global__ __launch_bounds__(RK_T) void k_rank(const uint32_t* __restrict__ key, int n, int slice,
                                                int* __restrict__ rank, int* __restrict__ tot,
