@@ -68,14 +68,19 @@ __device__ __forceinline__ unsigned long long* work_slot(unsigned long long* wor
 // Conservative block mask of one entry: bit 4 w + r is set when the entry can
 // reach alpha >= 1/255 at a pixel of the 4x4 block of row r of wave w, in the
 // tile at (tx0, ty0).  The reach is the ellipse sigma < min(5.55, ln(255 o)),
-// with a margin far above fp32 rounding on that threshold and 1/32 pixel
-// around the blocks.  For the tile's four strips of 4 pixel rows, the part of
-// the ellipse inside a strip spans an interval of x whose ends are the
-// ellipse's extremes with their offset dy clamped to the strip (the ellipse
-// is convex); the blocks of the strip that meet the interval are set.  Entries
-// outside a block are exactly the ones the per-pixel tests would skip there,
-// so culling them changes no result.  About 140 vector instructions (the four
-// exact quadrant minima that a coarser mask of 8x8 quadrants took were 250).
+// with margins on that threshold and of 1/32 pixel around the blocks.  For the
+// tile's four strips of 4 pixel rows, the part of the ellipse inside a strip
+// spans an interval of x whose ends are the ellipse's extremes with their
+// offset dy clamped to the strip (the ellipse is convex); the blocks of the
+// strip that meet the interval are set.  Entries outside a block are ones the
+// per-pixel tests skip there, so culling them changes no result.
+// The threshold's margin covers what a pixel's computed sigma may be below its
+// value: the terms a dx^2, c dy^2 and b dx dy of a needle cancel, each up to 2
+// kappa sigma with kappa = a c / (a c - b^2), and the roundings that fwd_step
+// makes on them add up to at most 17 u kappa sigma (u = 2^-24; the bound is
+// taken 1.08 times).  Where that is half of sigma (needles of 1000 pixels and
+// more), nothing is culled.  About 140 vector instructions (the four exact
+// quadrant minima that a coarser mask of 8x8 quadrants took were 250).
 __device__ __forceinline__ int block_mask(float x, float y, float a, float b, float c, float o,
                                           int tx0, int ty0) {
     if (!(o >= 0.0039f)) return o == o ? 0 : 0xFFFF;   // alpha <= o < 1/255 everywhere
@@ -87,8 +92,11 @@ __device__ __forceinline__ int block_mask(float x, float y, float a, float b, fl
         !(c < 1e30f) || !(fabsf(x) < 1e30f) || !(fabsf(y) < 1e30f))
         return 0xFFFF;
     constexpr float M = 0.03125f;
-    const float thr2 = 2.f * (fminf(5.55f, __logf(255.f * o) + 0.05f) * 1.002f + 1e-3f);
     const float ia = __builtin_amdgcn_rcpf(a), id = __builtin_amdgcn_rcpf(det);
+    const float err = 1.1e-6f * (a * c * id);     // of sigma, relative
+    if (!(err < 0.5f)) return 0xFFFF;
+    // sigma (1 - err) <= t holds up to sigma = t / (1 - err) <= t (1 + 2 err)
+    const float thr2 = 2.f * (fminf(5.55f, __logf(255.f * o) + 0.05f) * 1.002f + 1e-3f) * fmaf(2.f, err, 1.f);
     // offsets d = centre - pixel: at offset dy the ellipse spans dx = (-b dy
     // -+ sqrt(a thr2 - det dy^2)) / a; its largest dx lies at dy = -k
     const float k = b * __builtin_amdgcn_rcpf(c) * __builtin_amdgcn_sqrtf(c * thr2 * id);

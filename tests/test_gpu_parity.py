@@ -577,3 +577,42 @@ def test_depth_order_far_keys(dev, n, clip):
     keys = z[z > 0].astype(np.float32).view(np.uint32) - (np.float32(clip).view(np.uint32) if clip > 0 else 0)
     assert len(np.unique(keys >> 27)) > 1 and (keys >> 27).max() > 0
     parity.render_and_compare(dev, sc.params(), 0, sc.cameras[0], clip=clip)
+
+
+def _needle_scene(width, height, angles, seed, n=400):
+    """n thin gaussians (sd across below the pixel blur) whose sd along the
+    given screen angles is 100 to 2000 pixels, each reaching the image with a
+    part up to 3 sd from its centre."""
+    rng = np.random.default_rng(seed)
+    f = np.float32
+    sc = small_scene(n=n, width=width, height=height, seed_off=360)
+    cam = sc.cameras[0]
+    c2w = np.asarray(cam.cam_to_world, np.float64)
+    z = rng.uniform(2.0, 4.0, n)
+    sd, th = 10 ** rng.uniform(2.0, 3.3, n), rng.uniform(*angles, n)
+    along = rng.uniform(-3.0, 3.0, n) * sd
+    u = rng.uniform(0, width, n) + along * np.cos(th)
+    v = rng.uniform(0, height, n) - along * np.sin(th)
+    local = np.stack([(u - cam.cx) / cam.fx * z, -(v - cam.cy) / cam.fy * z, -z], 1)
+    sc.means = (local @ c2w[:3, :3].T + c2w[:3, 3]).astype(f)
+    px = z / cam.fx      # world size of a pixel
+    sc.scales = np.log(np.stack([px * sd, px * 0.05, px * 0.02], 1)).astype(f)
+    # the camera's axes turned by th about the line of sight
+    d = np.cos(th)[:, None] * c2w[:3, 0] + np.sin(th)[:, None] * c2w[:3, 1]
+    b = np.broadcast_to(c2w[:3, 2], d.shape)
+    R = np.stack([d, np.cross(b, d), b], 2)
+    w = 0.5 * np.sqrt(np.maximum(1e-9, 1 + R[:, 0, 0] + R[:, 1, 1] + R[:, 2, 2]))
+    sc.quats = np.stack([w, (R[:, 2, 1] - R[:, 1, 2]) / (4 * w), (R[:, 0, 2] - R[:, 2, 0]) / (4 * w),
+                         (R[:, 1, 0] - R[:, 0, 1]) / (4 * w)], 1).astype(f)
+    sc.opacities = rng.uniform(-5.0, 8.0, (n, 1)).astype(f)
+    return sc
+
+
+# near an axis, along a wide and a tall image, and at any angle
+@pytest.mark.parametrize("width,height,angles", [(2000, 64, (-0.3, 0.3)), (64, 2000, (1.3, 1.9)),
+                                                 (420, 410, (-1.5, 1.5))])
+def test_raster_long_needles(dev, width, height, angles):
+    """Needles hundreds of pixels long, whose terms of sigma cancel: a pixel's
+    computed sigma is off by more than rounding of its value, and the block
+    masks have to let through every entry that a pixel takes all the same."""
+    _train_compare(dev, _needle_scene(width, height, angles, width))
