@@ -656,20 +656,35 @@ template <int N>
 __device__ __forceinline__ float row_bcast(float v) {
     return __int_as_float(row_bcast<N>(__float_as_int(v)));
 }
-// acc + a's value in lane N of the row x b, rounded once.  The compiler does
-// not fold the broadcast into a multiply-add by itself.  a must have been
-// written at least two instructions before (settled()).
-template <int N>
-__device__ __forceinline__ void row_fmac(float& acc, float a, float b) {
-    asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
-        : "+v"(acc) : "v"(a), "v"(b), "n"(N));
+// The colour terms of a column's four pixels, lane X + 4 y of each row holding
+// pixel y's (v0, v1, v2): rv[y] = v0 r + v1 g + v2 b, and c0, c1, c2 become
+// their value + sum over y of (v0, v1, v2) fac[y], every product and sum rounded
+// once.  The compiler does not fold a broadcast into a multiply-add by itself.
+// One block with the DPP wait states in front: the compiler's hazard logic
+// does not look inside, and may place a copy of v0, v1 or v2 right before it.
+#define MSP_COLOUR(op, d0, d1, d2, d3, v, s0, s1, s2, s3)                               \
+    op " " d0 ", " v ", " s0 " row_newbcast:%[n0] row_mask:0xf bank_mask:0xf\n\t"       \
+    op " " d1 ", " v ", " s1 " row_newbcast:%[n1] row_mask:0xf bank_mask:0xf\n\t"       \
+    op " " d2 ", " v ", " s2 " row_newbcast:%[n2] row_mask:0xf bank_mask:0xf\n\t"       \
+    op " " d3 ", " v ", " s3 " row_newbcast:%[n3] row_mask:0xf bank_mask:0xf\n\t"
+#define MSP_COLOUR_RV(op, v, s) MSP_COLOUR(op, "%0", "%1", "%2", "%3", v, s, s, s, s)
+#define MSP_COLOUR_SUM(d, v) MSP_COLOUR("v_fmac_f32_dpp", d, d, d, d, v, "%[f0]", "%[f1]", "%[f2]", "%[f3]")
+template <int X>
+__device__ __forceinline__ void column_colours(float v0, float v1, float v2, float r, float g, float b,
+                                               const float (&fac)[4], float (&rv)[4], float& c0, float& c1,
+                                               float& c2) {
+    asm("s_nop 1\n\t"
+        MSP_COLOUR_RV("v_mul_f32_dpp", "%[v0]", "%[r]") MSP_COLOUR_RV("v_fmac_f32_dpp", "%[v1]", "%[g]")
+        MSP_COLOUR_RV("v_fmac_f32_dpp", "%[v2]", "%[b]") MSP_COLOUR_SUM("%[c0]", "%[v0]")
+        MSP_COLOUR_SUM("%[c1]", "%[v1]") MSP_COLOUR_SUM("%[c2]", "%[v2]")
+        : "=&v"(rv[0]), "=&v"(rv[1]), "=&v"(rv[2]), "=&v"(rv[3]), [c0] "+v"(c0), [c1] "+v"(c1), [c2] "+v"(c2)
+        : [v0] "v"(v0), [v1] "v"(v1), [v2] "v"(v2), [r] "v"(r), [g] "v"(g), [b] "v"(b), [f0] "v"(fac[0]),
+          [f1] "v"(fac[1]), [f2] "v"(fac[2]), [f3] "v"(fac[3]), [n0] "n"(X), [n1] "n"(X + 4), [n2] "n"(X + 8),
+          [n3] "n"(X + 12));
 }
-// A point after which a, b and c may be read through DPP, and before which
-// the compiler forms no broadcast of them or of d (a loop's broadcasts are
-// not hoisted into registers of their own).
-__device__ __forceinline__ void settled(float& a, float& b, float& c, int& d) {
-    asm volatile("s_nop 1" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
-}
+// A point before which the compiler forms no broadcast of d (a loop's
+// broadcasts are not hoisted into registers of their own).
+__device__ __forceinline__ void keep_in_loop(int& d) { asm volatile("" : "+v"(d)); }
 // The value of the lane before within the row; lane 0 gets first.
 __device__ __forceinline__ float row_before(float v, float first) {
     return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(first), __float_as_int(v), 0x111,
@@ -755,16 +770,12 @@ __device__ __forceinline__ void bwd_column(float4 g, float4 c, float blue, int n
         constexpr int y = decltype(yc)::value, p = 4 * y + X;
         Tn[y] = st.T[p] * P[y];
         fac[y] = ag[y] * Tn[y];
-        RV[y] = row_bcast<p>(vo0) * c.z;
-        row_fmac<p>(RV[y], vo1, c.w);
-        row_fmac<p>(RV[y], vo2, blue);
-        S[y] = fac[y] * RV[y];
-        row_fmac<p>(es.c0, vo0, fac[y]);
-        row_fmac<p>(es.c1, vo1, fac[y]);
-        row_fmac<p>(es.c2, vo2, fac[y]);
         st.T[p] = row_bcast<15>(Tn[y]);
     };
     for_each_to<4>(terms);
+    column_colours<X>(vo0, vo1, vo2, c.z, c.w, blue, fac, RV, es.c0, es.c1, es.c2);
+#pragma unroll
+    for (int y = 0; y < 4; ++y) S[y] = fac[y] * RV[y];
     MSP_ROW_SCAN4("v_add_f32_dpp", S);
     float s = 0.f, t = 0.f;     // the column's sums of v and v dy
     auto sums = [&](auto yc) {
@@ -966,7 +977,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
                 cy2[y] = c.x * dy[y] * dy[y];
             }
             EntrySums es{};
-            settled(vo0, vo1, vo2, bf);
+            keep_in_loop(bf);
             bwd_column<COUNT, 3>(g, c, blue, nidx, fx0, dy, cy2, vo0, vo1, vo2, bf, st, es, ngrad);
             bwd_column<COUNT, 2>(g, c, blue, nidx, fx0, dy, cy2, vo0, vo1, vo2, bf, st, es, ngrad);
             bwd_column<COUNT, 1>(g, c, blue, nidx, fx0, dy, cy2, vo0, vo1, vo2, bf, st, es, ngrad);
