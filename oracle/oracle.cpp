@@ -606,7 +606,7 @@ struct BwdBounds { float* mag; float* err; uint8_t* quad; };
 //                              dx^2 / 2 ..., fac |v_out_k|, |1 - o|)
 // so err accumulates (8 d + 24) x magnitude; the per-gaussian summation of
 // the terms adds (n_w + 10) x the gaussian's total magnitude (done by the
-// caller): a tree of at most 10 levels inside a wave plus n_w float atomics,
+// caller): at most 10 additions inside a wave plus n_w float atomics,
 // one per 8x8 quadrant and entry with a gradient.
 inline void raster_pixel_bwd(const Entry* ent, int s, int bin_final, float px, float py,
                              float T, const float* buf0, float T_final, const float* bg,

@@ -616,3 +616,35 @@ def test_raster_long_needles(dev, width, height, angles):
     computed sigma is off by more than rounding of its value, and the block
     masks have to let through every entry that a pixel takes all the same."""
     _train_compare(dev, _needle_scene(width, height, angles, width))
+
+
+def test_raster_backward_equal_terms(dev):
+    """A gaussian as flat as a constant gives each of the 64 pixels of an 8x8
+    image the same colour and opacity term x, 1/64 of a 1x1 image's term, so the
+    two differ by rounding alone.  On the 1x1 image x is rounded once (u = 2^-24,
+    relative).  Of the 8x8 image's sums of four, 2 x loses nothing that matters,
+    3 x up to 3/4 u of 4 x and 4 x up to u; four equal sums in a chain, and four
+    of these again, add up to 4 times a sum exactly (3 s is off by at most half
+    a unit in the last place of 4 s, and adding s rounds that away, ties to
+    even).  So 2.75 u; a chain of 16 terms is off by more than 4 u."""
+    torch = pytest.importorskip("torch")
+    f = np.float32
+    rng = np.random.default_rng(5)
+    worst = 0.0
+    for logit in rng.uniform(-3.0, 3.0, 24):
+        got = []
+        for size in (1, 8):
+            sc = small_scene(n=1, width=size, height=size, seed_off=370, degree=0)
+            c2w = np.asarray(sc.cameras[0].cam_to_world, np.float64)
+            sc.means = (c2w[:3, 3] - 3.0 * c2w[:3, 2])[None].astype(f)
+            sc.scales = np.full((1, 3), np.log(1e5), f)
+            sc.f_dc = np.full((1, 3), 0.3, f)
+            sc.opacities = np.full((1, 1), logit, f)
+            g = dev.DeviceGaussians.from_arrays(sc.params(), 0)
+            gt = torch.zeros((size, size, 3), dtype=torch.float32, device="cuda")
+            dev.train_step(g, camera.prepare_cam(sc.cameras[0]), 0, np.zeros(3, f), gt, 0.0, LRS, 1)
+            got.append(np.concatenate([dev.intermediate("v_rgb"), dev.intermediate("v_opacity")]).astype(np.float64))
+        assert (got[0] != 0).all()
+        worst = max(worst, float(np.abs(got[1] / got[0] - 1).max()))
+        print(f"logit {logit:.3f}: {got[0]} {got[1]} off by {worst * 2 ** 24:.2f} u", flush=True)
+    assert worst <= 2.75 * 2.0 ** -24, worst * 2 ** 24
