@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "dataset.hpp"
+#include "frame_buffers.hpp"
 #include "model.hpp"
 #include "jpeg_decode.hpp"
 #include "png_decode.hpp"
@@ -194,15 +195,10 @@ public:
         render_pose_to(camToWorld, ref, nullptr, w, h);
         if (!out) return;
         const int64_t n = (int64_t)w * h;
-        if (frame.numel() != 3 * n) {
-            frame.reset();
-            frame_rgba.reset();
-            frame = gpu_empty({3 * n}, DType::Float32);
-            frame_rgba = MTensor::mapped({n}, DType::Int32);   // 4 bytes per pixel
-        }
-        render_pose_to(camToWorld, ref, frame.data<float>(), w, h);
-        check(msplat_hip_image_to_rgba8(frame.data<float>(), n, frame_rgba.data<uint8_t>()), "rgba8");
-        frame_rgba.copy_to_host(out, (size_t)n * 4);
+        frame.fit(n);
+        render_pose_to(camToWorld, ref, frame.image.data<float>(), w, h);
+        check(msplat_hip_image_to_rgba8(frame.image.data<float>(), n, frame.rgba.data<uint8_t>()), "rgba8");
+        frame.rgba.copy_to_host(out, (size_t)n * 4);
     }
 
     // Trainer::render (msplat_api.mm:168-186): a training or held-out camera
@@ -242,7 +238,7 @@ private:
     std::vector<Camera> test_cameras;
     std::vector<MTensor> test_images;
     std::vector<std::map<int, MTensor>> gpu_images;
-    MTensor frame, frame_rgba;   // of the latest render_pose_rgba8
+    FrameBuffers frame;   // of the latest render_pose_rgba8
     std::vector<size_t> cam_indices;
     size_t cam_iter_pos = 0;
     std::mt19937 rng;

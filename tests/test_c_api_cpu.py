@@ -303,3 +303,63 @@ def test_bindings_shim_has_every_reference_prototype(tmp_path):
     host = os.path.join(ROOT, "msplat_amd", "host")
     subprocess.check_call([cxx, "-std=c++17", "-fsyntax-only", "-I", host, "-I", os.path.join(ROOT, "include"),
                            str(src)])
+
+
+FRAME_BUFFERS_PROGRAM = r"""
+#include <cstdio>
+#include <cstdlib>
+#include "frame_buffers.hpp"
+static int live = 0;
+static bool fail_device = false, fail_mapped = false;
+extern "C" {
+const char* msplat_hip_last_error(void) { return "out of memory"; }
+int msplat_hip_alloc(void** p, size_t n) {
+    if (fail_device) return MSPLAT_ERR_NOMEM;
+    ++live; *p = std::malloc(n); return MSPLAT_OK;
+}
+int msplat_hip_alloc_mapped(void** p, size_t n) {
+    if (fail_mapped) return MSPLAT_ERR_NOMEM;
+    ++live; *p = std::malloc(n); return MSPLAT_OK;
+}
+int msplat_hip_free(void* p) { --live; std::free(p); return MSPLAT_OK; }
+int msplat_hip_free_mapped(void* p) { --live; std::free(p); return MSPLAT_OK; }
+}
+#define CHECK(x) do { if (!(x)) { std::printf("line %d: %s\n", __LINE__, #x); return 1; } } while (0)
+static bool fits(msplat::FrameBuffers& f, int64_t n) {
+    try { f.fit(n); } catch (const std::exception&) { return false; }
+    return f.image.data_ptr() && f.rgba.data_ptr() && f.image.numel() == 3 * n && f.rgba.numel() == n;
+}
+int main() {
+    {
+        msplat::FrameBuffers f;
+        CHECK(fits(f, 1000) && live == 2);
+        void* kept = f.rgba.data_ptr();
+        CHECK(fits(f, 1000) && live == 2 && f.rgba.data_ptr() == kept);
+        for (bool* fail : {&fail_mapped, &fail_device}) {
+            *fail = true;
+            CHECK(!fits(f, 2000) && live == 0);
+            CHECK(!fits(f, 2000) && live == 0);     // still failing, not a null buffer
+            *fail = false;
+            CHECK(fits(f, 2000) && live == 2);      // memory is free again
+            CHECK(fits(f, 500) && live == 2);       // smaller
+        }
+    }
+    CHECK(live == 0);
+    return 0;
+}
+"""
+
+
+def test_frame_buffers_survive_a_failed_allocation(tmp_path):
+    """The display frame's kept buffers: reused at one size, given back before
+    others are taken, and taken again after a call whose allocation failed."""
+    cxx = shutil.which("g++")
+    if not cxx:
+        pytest.skip("no host C++ compiler")
+    src = tmp_path / "frames.cpp"
+    src.write_text(FRAME_BUFFERS_PROGRAM)
+    exe = str(tmp_path / "frames")
+    subprocess.check_call([cxx, "-std=c++17", "-Wall", "-I", os.path.join(ROOT, "msplat_amd", "host"), "-o", exe,
+                           str(src)])
+    r = subprocess.run([exe], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout

@@ -114,6 +114,29 @@ def test_render_to_rgba8_buffer(mods):
     assert_bits_equal(rgba, orc.image_to_rgba8(img), "render_pose_to_buffer")
 
 
+def test_display_frames_of_changing_pose_and_size(mods):
+    """One trainer's frames, whose buffers are kept from call to call: another
+    pose at the same size, other sizes (smaller, larger, the first again) and
+    another resolution of the schedule, each against its own float render."""
+    _, _, trainer = mods
+    sc = small_scene(n=1500, seed_off=640)
+    poses = [camera.look_at(np.array(p)) for p in ((3.5, 1.0, -3.0), (-2.0, 2.5, 4.0), (0.5, -3.0, 4.0))]
+    sc.cameras += [camera.pinhole(w, h, 60.0, poses[0]) for w, h in ((97, 51), (230, 171))]
+    tg = [target_for(sc, (c.height, c.width), seed_off=650 + i) for i, c in enumerate(sc.cameras)]
+    cfg = trainer.TrainingConfig(iterations=1000, sh_degree=3, sh_degree_interval=0, num_downscales=1,
+                                 resolution_schedule=2, warmup_length=10_000, shuffle_cameras=False)
+    tr = trainer.GaussianTrainer(sc.params(), sc.cameras, tg, cfg)
+    shapes = set()
+    for step in range(4):
+        for ref, pose in ((0, 0), (0, 1), (1, 1), (2, 2), (2, 0), (0, 2)):
+            rgba = tr.render_from_pose_rgba8(poses[pose], ref)
+            assert_bits_equal(rgba, orc.image_to_rgba8(tr.render_from_pose(poses[pose], ref)),
+                              f"frame of camera {ref}, pose {pose}, step {step}")
+            shapes.add(rgba.shape)
+        tr.step()
+    assert len(shapes) == 6, shapes
+
+
 def test_trainer_evaluate(mods):
     _, _, trainer = mods
     sc, tg, tr = _trainer(trainer, cams=2)
