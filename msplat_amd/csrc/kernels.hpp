@@ -130,8 +130,9 @@ int64_t radix_temp_ints(int64_t n);
 // two totals to *out (coherent host memory) as one 64-bit word,
 // totals_word(I, R), which the host polls.
 struct SlotSum {
-    const unsigned long long* slots;
-    unsigned long long* out;
+    const unsigned long long* slots = nullptr;
+    unsigned long long* out = nullptr;
+    int* far = nullptr;   // gets 1 if a depth key takes more than FAR_BITS bits, else 0
 };
 // Bit 63 set (so that a zeroed word means "not yet"), bit 62 if a depth key
 // takes more than FAR_BITS bits, the intersection total in bits 31..61 and the
@@ -145,9 +146,10 @@ __host__ __device__ inline unsigned long long totals_word(unsigned long long i, 
 // of that rectangle (both zero at the positions of a culling sort's culled
 // tail).
 struct RectGather {
-    const uint2* rect;
-    uint2* rs;
-    int* cnt;
+    const uint2* rect = nullptr;
+    uint2* rs = nullptr;
+    int* cnt = nullptr;
+    const int* skip = nullptr;   // nothing is written where this holds nonzero
 };
 // Up to RANK_MAX keys are ordered by ranking (all pairs compared) instead.  A
 // 256x256 render took, sorted / ranked: 98 / 44 us for 2k gaussians, 115 / 63

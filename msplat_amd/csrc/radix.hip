@@ -23,8 +23,13 @@
 // Depth keys are the bits of the depth less those of the near plane, and the
 // depth order sorts their low 27 bits in three passes: depths up to 65536 times
 // the near plane.  A fourth (launch_radix_far) follows where the projection
-// found a key beyond; the host learns that while the first passes run.  Four
-// passes of 8 bits for all took 13 us more at 500k gaussians, 11 at 120k.
+// found a key beyond; the host learns that while the first passes run, and the
+// third pass, which a flag on the device tells the same, leaves the rectangles to
+// the fourth.  Four passes of 8 bits for all took 13 us more at 500k gaussians, 11
+// at 120k.  Renders with some points beyond (or a near plane of 0), with four
+// passes of 8 bits / now / the same scene without: 171 / 154 / 136 us for 120k at
+// 641x421, 266 / 254 / 236 for 500k and 412 / 398 / 375 for 1.5M at 1297x840, 2187
+// / 2150 / 2102 for 6M at 4946x3286 (2230 where the third pass gathered too).
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -135,6 +140,7 @@ __device__ __forceinline__ void slot_sum(const SlotSum& ss) {
     }
     if (threadIdx.x == 0)
         __hip_atomic_store(ss.out, totals_word(ti, tr, any_far), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (ss.far && threadIdx.x == 0) *ss.far = any_far ? 1 : 0;
 }
 
 // Super-tiles of a rectangle as the projection packs it, 0 if it is empty.
@@ -394,7 +400,8 @@ __global__ __launch_bounds__(RT) void k_radix_scatter(const uint32_t* __restrict
         for (int i = threadIdx.x; i < DCOPIES * D; i += RT) dtot[i] = 0;
     const int64_t ne = pass_n(n, n_dev);
     const int64_t bbase = (int64_t)blockIdx.x * RB;
-    if (RG) {
+    const bool gather = RG && !(rg.skip && *rg.skip);
+    if (gather) {
         // output positions [ne, n) of this block's range: the culled tail
         for (int64_t p = max(bbase, ne) + threadIdx.x; p < min(bbase + RB, n); p += RT) {
             rg.rs[p] = make_uint2(0u, 0u);
@@ -470,7 +477,7 @@ __global__ __launch_bounds__(RT) void k_radix_scatter(const uint32_t* __restrict
         key[j] = i < ne ? kin[i] : 0u;
         val[j] = i < ne ? vin[i] : 0u;
         const bool ok = i < ne && !culled(key[j], cl);
-        if (RG) rc[j] = ok ? rg.rect[val[j]] : make_uint2(0u, 0u);
+        if (RG) rc[j] = gather && ok ? rg.rect[val[j]] : make_uint2(0u, 0u);
         const int d = ok ? digit_of(key[j], shift, mask) : D;
         dig[j] = d;
         uint64_t peers = wave_ballot(ok);
@@ -547,7 +554,7 @@ __global__ __launch_bounds__(RT) void k_radix_scatter(const uint32_t* __restrict
             }
         }
     }
-    if (RG) {
+    if (gather) {
         // the rectangles take the keys' LDS places and go to the same
         // output positions, with their super-tile counts
         __syncthreads();
@@ -644,12 +651,13 @@ void launch_fused_pass(hipStream_t s, const uint32_t* ki, const uint32_t* vi, ui
 // Scratch layout: the digit totals first, at a fixed place whatever n is
 // (DCOPIES x DMAX per pass; each pass's scatter clears its totals for the next
 // sort on this scratch), then the per-block histograms (a fused sort has one
-// set of rows per pass), then the visible count of a culling sort.
+// set of rows per pass), then the visible count of a culling sort
+// and whether launch_radix_far follows it.
 struct RadixTemp {
-    int *dtot, *hist, *nvis;
+    int *dtot, *hist, *nvis, *far;
     RadixTemp(int* temp, int nb)
         : dtot(temp), hist(temp + DCOPIES * DMAX * MAX_PASSES),
-          nvis(hist + (size_t)DMAX * nb * (nb <= FUSE_BLOCKS ? MAX_PASSES : 1)) {}
+          nvis(hist + (size_t)DMAX * nb * (nb <= FUSE_BLOCKS ? MAX_PASSES : 1)), far(nvis + 1) {}
 };
 
 }  // namespace
@@ -663,7 +671,8 @@ struct RadixTemp {
 // occurring key value k gets its output range [edge0[k], edge1[k]) (entries of
 // absent values are not written).  With cull the keys 0xFFFFFFFF are left out
 // by the first pass and the later passes sort only the others; positions
-// [visible, n) of the result then hold nothing, and rg marks them empty.
+// [visible, n) of the result then hold nothing, and rg marks them empty, unless
+// the SlotSum job finds that launch_radix_far has to follow: rg is left to that.
 bool launch_radix_sort(hipStream_t s, uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1,
                        int64_t n, int bits, int* temp, const RectGather* rg, const SlotSum* ss,
                        int* edge0, int* edge1, bool cull) {
@@ -684,11 +693,12 @@ bool launch_radix_sort(hipStream_t s, uint32_t* k0, uint32_t* v0, uint32_t* k1, 
         uint32_t* vi = flip ? v1 : v0;
         uint32_t* ko = flip ? k0 : k1;
         uint32_t* vo = flip ? v0 : v1;
-        const SlotSum side = ss && pass == 0 ? *ss : SlotSum{nullptr, nullptr};
+        const SlotSum side = ss && pass == 0 ? SlotSum{ss->slots, ss->out, t.far} : SlotSum{};
         const int* n_dev = cull && pass > 0 ? t.nvis : nullptr;
         int* e0 = passes == 1 ? edge0 : nullptr;
         int* e1 = passes == 1 ? edge1 : nullptr;
-        const RectGather* prg = last ? rg : nullptr;
+        const RectGather lrg = rg ? RectGather{rg->rect, rg->rs, rg->cnt, ss ? t.far : nullptr} : RectGather{};
+        const RectGather* prg = last && rg ? &lrg : nullptr;
         if (nb <= FUSE_BLOCKS) {
             auto rows = [&](int p) { return t.hist + (size_t)p * nb * DMAX; };
             const int nshift = shift + width;
@@ -717,7 +727,7 @@ void launch_radix_far(hipStream_t s, const uint32_t* ki, const uint32_t* vi, uin
     const RadixTemp t(temp, nb);
     constexpr int W = 32 - FAR_BITS;
     launch_pass<256>(s, ki, vi, ko, vo, n, t.nvis, FAR_BITS, (1u << W) - 1u, false, W, true, nb, t.hist,
-                     t.dtot + DCOPIES * DMAX * (MAX_PASSES - 1), SlotSum{nullptr, nullptr}, nullptr, nullptr,
+                     t.dtot + DCOPIES * DMAX * (MAX_PASSES - 1), SlotSum{}, nullptr, nullptr,
                      nullptr, &rg);
 }
 

@@ -579,6 +579,16 @@ def test_depth_order_far_keys(dev, n, clip):
     parity.render_and_compare(dev, sc.params(), 0, sc.cameras[0], clip=clip)
 
 
+@pytest.mark.parametrize("n", [26000, 131073])
+def test_depth_order_far_and_near_in_turn(dev, n):
+    """Whether a fourth pass follows is decided anew for each frame: the near
+    plane moves back and forth, so that the same depths need it and do not."""
+    sc = small_scene(n=n, width=300, height=270, seed_off=123, degree=0)
+    sc.scales -= 1.0
+    for clip in (1e-5, 0.01, 0.01, 0.0, 0.01, 1e-5):
+        parity.render_and_compare(dev, sc.params(), 0, sc.cameras[0], clip=clip, label=f"clip {clip}")
+
+
 def _needle_scene(width, height, angles, seed, n=400):
     """n thin gaussians (sd across below the pixel blur) whose sd along the
     given screen angles is 100 to 2000 pixels, each reaching the image with a
