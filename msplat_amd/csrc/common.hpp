@@ -141,25 +141,10 @@ __device__ __forceinline__ float dpp(float v) {
 // int and first turns the condition into a 0/1 value).
 __device__ __forceinline__ uint64_t wave_ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
 
-// Lane masks of single compares (one v_cmp writing an SGPR pair), to be
-// combined with scalar ands; lane_of(mask) turns a mask back into the
-// per-lane condition without a vector instruction.  Predicates: "u"
-// versions are true for NaN operands, as !(a < b) is.
-__device__ __forceinline__ uint64_t mask_lt(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 4); }
+// Lane mask of a single compare (one v_cmp writing an SGPR pair); lane_of(mask)
+// turns a mask back into the per-lane condition without a vector instruction.
 __device__ __forceinline__ uint64_t mask_le(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 5); }
-__device__ __forceinline__ uint64_t mask_uge(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 11); }
-__device__ __forceinline__ uint64_t mask_ult(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 12); }
-__device__ __forceinline__ uint64_t mask_ge_i(int a, int b) { return __builtin_amdgcn_sicmp(a, b, 39); }
 __device__ __forceinline__ bool lane_of(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
-
-// Index of the lowest set bit of a nonzero wave-uniform mask, cleared from the
-// mask: s_ff1 then s_bitset0, two scalar ALU instructions where m &= m - 1
-// takes a 64-bit decrement and an and.
-__device__ __forceinline__ int pop_low_bit(uint64_t& m) {
-    int bit;
-    asm volatile("s_ff1_i32_b64 %0, %1\n\ts_bitset0_b64 %1, %0" : "=&s"(bit), "+s"(m));
-    return bit;
-}
 
 // Sum over the 64 lanes; every lane gets the total.  All lanes must be active.
 __device__ __forceinline__ float wave_sum(float v) {
@@ -172,48 +157,6 @@ __device__ __forceinline__ float wave_sum(float v) {
     const float r2 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32));
     const float r3 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 48));
     return (r0 + r1) + (r2 + r3);
-}
-
-// Sum over the 64 lanes, total in lane 63: row sums by row DPP, then the
-// gfx9 row_bcast:15 / row_bcast:31 adds carry rows 0..2 into row 3 (rows
-// outside the row mask keep their value).  The two masked adds are written
-// as assembly because the compiler does not fold a row-masked DPP move into
-// the add; the s_nop 1 before each covers the VALU-write -> DPP-read hazard
-// (two wait states) and the one after covers a DPP reader that may follow.
-// All lanes must be active.
-__device__ __forceinline__ float wave_sum_to_last(float v) {
-    v += dpp<0xB1>(v);                 // quad_perm [1,0,3,2]
-    v += dpp<0x4E>(v);                 // quad_perm [2,3,0,1]
-    v += dpp<0x124>(v);                // row_ror:4
-    v += dpp<0x128>(v);                // row_ror:8  -> row sums
-    asm volatile(
-        "s_nop 1\n\t"
-        "v_add_f32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
-        "s_nop 1\n\t"
-        "v_add_f32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
-        "s_nop 1"
-        : "+v"(v));
-    return v;
-}
-
-// The same sum with its total written into lane 63 of dst: the last masked
-// add goes to dst in row 3, bank 3 only (lanes 60..63: row_mask selects the
-// 16-lane row, bank_mask the group of four lanes within it), so lanes 60..62
-// of dst receive partial sums and every other lane keeps its dst value.
-// All lanes must be active.
-__device__ __forceinline__ float wave_sum_into_lane63(float v, float dst) {
-    v += dpp<0xB1>(v);                 // quad_perm [1,0,3,2]
-    v += dpp<0x4E>(v);                 // quad_perm [2,3,0,1]
-    v += dpp<0x124>(v);                // row_ror:4
-    v += dpp<0x128>(v);                // row_ror:8  -> row sums
-    asm volatile(
-        "s_nop 1\n\t"
-        "v_add_f32_dpp %1, %1, %1 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
-        "s_nop 1\n\t"
-        "v_add_f32_dpp %0, %1, %1 row_bcast:31 row_mask:0x8 bank_mask:0x8\n\t"
-        "s_nop 1"
-        : "+v"(dst), "+v"(v));
-    return dst;
 }
 
 __device__ __forceinline__ int wave_max_i(int v) {
@@ -243,7 +186,5 @@ __device__ __forceinline__ int xcd_order(int b, int n) {
     const int x = b & 7, q = n >> 3, rem = n & 7;
     return x * q + min(x, rem) + (b >> 3);
 }
-
-__device__ __forceinline__ unsigned lane_id() { return __lane_id(); }
 
 }  // namespace msp
