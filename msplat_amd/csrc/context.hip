@@ -736,9 +736,8 @@ int msplat_hip_train_step(const MsplatTrainArgs* a, int32_t* radii_out, float* l
     if (r != MSPLAT_OK) return r;
     const CamParams p = cam_params(&a->r);
     const size_t Px = (size_t)p.W * p.H;
-    const dim3 sgrid((p.W + 15) / 16, (p.H + 15) / 16);
     ENSURE(c->v_rendered, Px * 12);
-    ENSURE(c->loss_part, (size_t)sgrid.x * sgrid.y * 12);
+    ENSURE(c->loss_part, (size_t)ssim_part_bound(p.H, p.W) * 12);
     ENSURE(c->loss_d, 16);
     stage_mark(c, S_LOSS);
     // the loss sum goes straight to pinned host memory (loss_h[1])

@@ -313,9 +313,11 @@ void launch_raster_work(hipStream_t s, const CamParams& p, int64_t max_items, co
                         Items it, Entries pk, const int* final_idx,
                         ChunkBufs cb, const int* live_end, unsigned long long* out);
 
-// The loss: SSIM + L1 forward and backward per 32x32 tile; writes the loss
-// gradient image and one partial (sum SSIM, sum L1, pixels) per tile, and
-// returns the number of partials.
+// The loss: SSIM + L1 forward and backward in tiles whose shape goes by the
+// image's size; writes the loss gradient image and one partial (sum SSIM, sum
+// L1, pixels) per tile, and returns the number of partials, at most
+// ssim_part_bound(H, W).
+int ssim_part_bound(int H, int W);
 int launch_ssim(hipStream_t s, int H, int W, const float* img, const float* gt, float w,
                 float inv_n, float* v_rendered, float* loss_part);
 

@@ -27,6 +27,8 @@
 // folded in a fixed order by one workgroup of the next kernel (loss_fold in
 // kernels.hpp); it equals the sum over pixels of
 // w*(1 - mean_c SSIM) + (1-w)*mean_c |gt - r|.
+#include <algorithm>
+
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -352,6 +354,10 @@ int run(hipStream_t s, int H, int W, const float* img, const float* gt, float w,
 }
 
 }  // namespace
+
+int ssim_part_bound(int H, int W) {
+    return std::max({tiles<TileS>(W, H), tiles<TileM>(W, H), tiles<TileL>(W, H)});
+}
 
 int launch_ssim(hipStream_t s, int H, int W, const float* img, const float* gt, float w,
                 float inv_n, float* v_rendered, float* loss_part) {
