@@ -1,7 +1,7 @@
 // radix.hip — device-wide scans and a stable LSD radix sort of (u32 key, u32
 // value) pairs, used by the binning to order the gaussians by depth and
 // their super-tile references by super-tile, and by the nearest-neighbour
-// search to order points by cell.
+// search to order points along a Morton curve.
 //
 // Sort (more than FUSE_BLOCKS blocks): digits of up to 9 bits,
 // reduce-then-scan per pass over 2048-key blocks (512 threads x 4 keys):

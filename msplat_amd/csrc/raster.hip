@@ -712,8 +712,8 @@ __device__ __forceinline__ void for_each_to(F f) {
 
 // Window of a backward wave: up to WIN entries that reach its quadrant, and
 // the dummy behind them; their gradient sums; the rows' lists of window slots.
-// 8.1 KB; the 107 vector registers allow four waves a SIMD (five, at 96
-// registers with spills, measured 2% slower; 128 entries the same).
+// 8.1 KB; the 117 vector registers allow four waves a SIMD (five, at 96
+// registers with spills, measured 2% slower; windows of 128 entries the same).
 constexpr int WIN = 96;
 struct BwdLds {
     float4 geo[WIN + 1];      // x, y, conic a, b
@@ -1042,7 +1042,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
 
 // Algorithmic work of the most recent forward (+ backward): one thread per
 // pixel walks its item's entries in the order of the per-pixel loops of the
-// reference kernels, without quadrant culling or lockstep, and counts
+// reference kernels, without block culling or lockstep, and counts
 // (pixel, entry) pairs: forward tested / sigma in range / composited,
 // backward tested / sigma in range / carrying a gradient.  The counts
 // define the algorithmic flops of the roofline; they change no state.
