@@ -712,7 +712,7 @@ __device__ __forceinline__ void for_each_to(F f) {
 
 // Window of a backward wave: up to WIN entries that reach its quadrant, and
 // the dummy behind them; their gradient sums; the rows' lists of window slots.
-// 8.1 KB; the 117 vector registers allow four waves a SIMD (five, at 96
+// 8.2 KB; the 119 vector registers allow four waves a SIMD (five, at 96
 // registers with spills, measured 2% slower; windows of 128 entries the same).
 constexpr int WIN = 96;
 struct BwdLds {
@@ -722,6 +722,7 @@ struct BwdLds {
     int gid[WIN];             // gaussian
     float4 sa[WIN], sb[WIN];  // the sums 0..3 and 4..7 of gacc's nine
     float sc[WIN];            // and the last
+    uint8_t rows[WIN];        // rows an entry is wanted by
     uint8_t list[4][WIN];
 };
 
@@ -826,9 +827,13 @@ __device__ __forceinline__ void bwd_column(float4 g, float4 c, float blue, int n
 // row's lanes (four DPP steps each), and an entry's gradient sums over the
 // pixels stay in its lane's registers: no reduction over lanes.
 // One wave is a workgroup of its own, for one quadrant of a record: no
-// barriers, and a heavy quadrant holds up nothing but itself.  It gathers a
-// window of up to WIN entries that reach its quadrant, walks them, and adds
-// the window's sums to gacc with consecutive lanes on consecutive floats.
+// barriers, and a heavy quadrant holds up nothing but itself.  It puts together
+// a window of up to WIN entries that reach its quadrant, gathers them and lists
+// them by row, walks them, and adds the window's sums to gacc with consecutive
+// lanes on consecutive floats.  (Gathered and listed 64 entries of the tile at a
+// time, most of them unwanted, 100k needles of sd 110 pixels at 1297x840, whose
+// rectangles cover tiles that they miss, took 734 us, now 584, where lane =
+// pixel took 519; the whole step 1941, 1796 and 1797.)
 // The window's sums are kept in LDS; an LDS float atomic takes 193 cycles of
 // the CU for a wave whatever its addresses (a plain store 7.5), so each row
 // adds its sums in turn with ordinary loads and stores (entries of one row are
@@ -887,13 +892,20 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     const float fx0 = (float)(px.j - (i & 3)), fy0 = (float)(px.i - (i >> 2));
     unsigned ngrad = 0;     // pairs of this wave that carry a gradient (wave-uniform)
     unsigned nwit = 0;      // entries this wave evaluated (wave-uniform)
+    float Tfin = 1.f, vo0 = 0.f, vo1 = 0.f, vo2 = 0.f;
+    if (px.inside) {
+        Tfin = final_T[pix];
+        vo0 = v_out[3 * pix + 0];
+        vo1 = v_out[3 * pix + 1];
+        vo2 = v_out[3 * pix + 2];
+    }
 
     // the record's chunks one after the other (a tile in one piece is one);
     // each starts from its own state
     int item = rec.x;
     for (int cs = rec.z, ce; cs < rec.w && item < item_end; cs = ce, ++item) {
     ce = multi ? min(cs + CHUNK, rec.w) : rec.w;
-    float T = 1.f, Tfin = 1.f, B0 = 0.f, B1 = 0.f, B2 = 0.f, vo0 = 0.f, vo1 = 0.f, vo2 = 0.f;
+    float T = Tfin, B0 = 0.f, B1 = 0.f, B2 = 0.f;
     // bf = cs - 1 for pixels outside the image: no entry passes e_idx <= bf
     int bf = cs - 1;
     const size_t chunk_pix = (size_t)item * TILE_PIX + px.lp;
@@ -904,19 +916,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
                            __builtin_amdgcn_readlane(rbf, 32), __builtin_amdgcn_readlane(rbf, 48)};
     int top = min(ce - 1, max(max(row_bf[0], row_bf[1]), max(row_bf[2], row_bf[3])));
     if (top < cs) continue;
-    if (px.inside) {
-        Tfin = final_T[pix];
-        vo0 = v_out[3 * pix + 0];
-        vo1 = v_out[3 * pix + 1];
-        vo2 = v_out[3 * pix + 2];
-        if (!multi) {
-            T = Tfin;
-        } else {
-            T = cb.pT[chunk_pix] * cb.cT[chunk_pix];
-            B0 = cb.aC[3 * chunk_pix + 0];
-            B1 = cb.aC[3 * chunk_pix + 1];
-            B2 = cb.aC[3 * chunk_pix + 2];
-        }
+    // the next 64 entries' block masks and ids, loaded ahead of their use
+    int idx = top - lane;
+    unsigned mask = idx >= cs ? pk.bmask[idx] : 0u;
+    int gid = idx >= cs ? (int)pk.ids[idx] : 0;
+    if (px.inside && multi) {
+        T = cb.pT[chunk_pix] * cb.cT[chunk_pix];
+        B0 = cb.aC[3 * chunk_pix + 0];
+        B1 = cb.aC[3 * chunk_pix + 1];
+        B2 = cb.aC[3 * chunk_pix + 2];
     }
     // The colour terms of v_alpha enter only as sum_k v_out_k (...)_k:
     // D = sum_k v_out_k B_k (accumulated colour behind) and TB = sum_k
@@ -931,34 +939,49 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
         st.E[p] = row_bcast<p>(E);
     };
     for_each_to<16>(spread);
-
-    // the next 64 entries' block masks and ids, loaded ahead of their use
-    int idx = top - lane;
-    unsigned mask = idx >= cs ? pk.bmask[idx] : 0u;
-    int gid = idx >= cs ? (int)pk.ids[idx] : 0;
+    const int bf_low = min(min(row_bf[0], row_bf[1]), min(row_bf[2], row_bf[3]));
     while (top >= cs) {
-        // fill the window, 64 entries at a time while they fit
-        int nw = 0, n[4] = {0, 0, 0, 0};
+        // the window's entries, from 64 of the list at a time while they fit
+        int nw = 0;
         while (top >= cs) {
             // rows this entry is wanted by: its block is reached, and it is
             // not behind the last contributor of the row's pixels
             unsigned m = (mask >> (4 * w)) & 15u;
+            if (top > bf_low) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (idx > row_bf[r]) m &= ~(1u << r);
+                for (int r = 0; r < 4; ++r)
+                    if (idx > row_bf[r]) m &= ~(1u << r);
+            }
             const uint64_t in = wave_ballot(m != 0u);
             const int cnt = __popcll(in);
             if (nw + cnt > WIN) break;
-            const int slot = nw + lanes_below(in);
             if (m) {
-                const float4* r = pk.rec + 4 * (size_t)gid;
+                const int slot = nw + lanes_below(in);
+                s.rows[slot] = (uint8_t)m;
+                s.gid[slot] = gid;
+                s.aux[slot].y = __int_as_float(-idx);
+            }
+            nw += cnt;
+            top -= 64;
+            idx = top - lane;
+            mask = idx >= cs ? pk.bmask[idx] : 0u;
+            gid = idx >= cs ? (int)pk.ids[idx] : 0;
+        }
+        __builtin_amdgcn_wave_barrier();
+        // their records and the rows' lists, 64 of the window at a time
+        int n[4] = {0, 0, 0, 0};
+        for (int k0 = 0; k0 < nw; k0 += 64) {
+            const int slot = k0 + lane;
+            unsigned m = 0;
+            if (slot < nw) {
+                m = s.rows[slot];
+                const float4* r = pk.rec + 4 * (size_t)s.gid[slot];
                 const float4 g = r[0];
                 const float4 c = r[1];
                 const float braw = r[2].x;
                 s.geo[slot] = g;
                 s.col[slot] = make_float4(c.x, c.y, fmaxf(c.z + 0.5f, 0.f), fmaxf(c.w + 0.5f, 0.f));
-                s.aux[slot] = make_float2(fmaxf(braw + 0.5f, 0.f), __int_as_float(-idx));
-                s.gid[slot] = gid;
+                s.aux[slot].x = fmaxf(braw + 0.5f, 0.f);
             }
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -967,11 +990,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
                 if (lane_of(b)) s.list[r][at] = (uint8_t)slot;
                 n[r] += __popcll(b);
             }
-            nw += cnt;
-            top -= 64;
-            idx = top - lane;
-            mask = idx >= cs ? pk.bmask[idx] : 0u;
-            gid = idx >= cs ? (int)pk.ids[idx] : 0;
         }
         __builtin_amdgcn_wave_barrier();
         const int longest = max(max(n[0], n[1]), max(n[2], n[3]));

@@ -618,14 +618,16 @@ def _needle_scene(width, height, angles, seed, n=400):
     return sc
 
 
-# near an axis, along a wide and a tall image, and at any angle
-@pytest.mark.parametrize("width,height,angles", [(2000, 64, (-0.3, 0.3)), (64, 2000, (1.3, 1.9)),
-                                                 (420, 410, (-1.5, 1.5))])
-def test_raster_long_needles(dev, width, height, angles):
+# near an axis, along a wide and a tall image, and at any angle; long lists of
+# which a block wants few entries, in one piece and in chunks
+@pytest.mark.parametrize("width,height,angles,n", [(2000, 64, (-0.3, 0.3), 400), (64, 2000, (1.3, 1.9), 400),
+                                                   (420, 410, (-1.5, 1.5), 400), (340, 330, (-1.5, 1.5), 3000),
+                                                   (160, 120, (-1.5, 1.5), 3000)])
+def test_raster_long_needles(dev, width, height, angles, n):
     """Needles hundreds of pixels long, whose terms of sigma cancel: a pixel's
     computed sigma is off by more than rounding of its value, and the block
     masks have to let through every entry that a pixel takes all the same."""
-    _train_compare(dev, _needle_scene(width, height, angles, width))
+    _train_compare(dev, _needle_scene(width, height, angles, width, n))
 
 
 def test_raster_backward_equal_terms(dev):
