@@ -864,14 +864,15 @@ __device__ __forceinline__ void bwd_column(float4 g, float4 c, float blue, int n
 // the CU for a wave whatever its addresses (a plain store 7.5), so each row
 // adds its sums in turn with ordinary loads and stores (entries of one row are
 // distinct, those of different rows are not).
-// Bound: the vector units (153M instructions in 1.5M gaussians' step at
-// 1297x840, four cycles each, are its 286 us).  Per (entry, pixel) pair of
-// lanes: about 57 vector instructions, no scalar ones and no LDS access, where
-// lane = pixel took 65, 11 and 11; a block of 4 x 4 pixels leaves fewer pairs
+// Bound: the vector units (294M instructions in a step of 1.5M trained gaussians
+// at 1297x840: four cycles each are 0.48 of its 0.53 ms).  Per (entry, pixel)
+// pair of lanes: about 57 vector instructions, no scalar ones and no LDS access
+// (75, 6 and 3 with the windows, lists and sums around them), where lane = pixel
+// took 65, 11 and 11; a block of 4 x 4 pixels leaves fewer pairs
 // without a gradient than an 8 x 8 quadrant (2.10M wave steps against 2.75M).
 // Measured against lane = pixel with 8 x 8 quadrants: 10k gaussians at 256x256
-// 33 -> 17 us, 120k at 324x210 59 -> 38 us, 1M in a blob at 2594x1680 581 ->
-// 552 us, 1.5M at 1297x840 283 -> 286 us.  The colour terms on the matrix cores
+// 32 -> 16 us, 120k at 324x210 60 -> 37 us, 1M in a blob at 2594x1680 592 ->
+// 558 us, 1.5M at 1297x840 281 -> 284 us.  The colour terms on the matrix cores
 // (v_mfma_f32_4x4x1) instead of by DPP: the same time, from register spills.
 // COUNT: count the wave's evaluated entries and gradient pairs into work
 // (a launch without counters runs the variant that does not count).
