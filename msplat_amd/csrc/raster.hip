@@ -684,9 +684,10 @@ __device__ __forceinline__ float row_bcast(float v) {
 }
 // The colour terms of a column's four pixels, lane X + 4 y of each row holding
 // pixel y's (v0, v1, v2): rv[y] = v0 r + v1 g + v2 b, and (c0, c1, c2) = sum over
-// y of (v0, v1, v2) fac[y], by multiply-adds in order.  The compiler does not fold a broadcast into a multiply-add by itself.
-// One block with the DPP wait states in front: the compiler's hazard logic
-// does not look inside, and may place a copy of v0, v1 or v2 right before it.
+// y of (v0, v1, v2) fac[y], by multiply-adds in order.  The compiler does not
+// fold a broadcast into a multiply-add by itself.  One block with the DPP wait
+// states in front: the compiler's hazard logic does not look inside, and may
+// place a copy of v0, v1 or v2 right before it.
 #define MSP_COLOUR(op, d0, d1, d2, d3, v, s0, s1, s2, s3)                               \
     op " " d0 ", " v ", " s0 " row_newbcast:%[n0] row_mask:0xf bank_mask:0xf\n\t"       \
     op " " d1 ", " v ", " s1 " row_newbcast:%[n1] row_mask:0xf bank_mask:0xf\n\t"       \
@@ -765,8 +766,8 @@ struct EntrySums {
 };
 
 // Column X of the row's block (pixels X, X + 4, X + 8, X + 12; column 3 comes
-// first), all 16 entries of the group at once: lane l of a row holds the row's l-th entry, deepest
-// first.  vo0..2 and bf are per pixel, in the pixel's lane: the pixel takes the
+// first), all 16 entries of the group at once: lane l of a row holds the row's
+// l-th entry, deepest first.  vo0..2 and bf are per pixel, in the pixel's lane: the pixel takes the
 // entries up to index bf (tested as the sign of bf - index, formed by an add:
 // a subtraction that takes its subtrahend through DPP, v_subrev, was measured
 // to broadcast the other operand).
